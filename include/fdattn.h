@@ -168,8 +168,35 @@ int fd_paged_decode_partial_hint(
     void* workspace, size_t workspace_bytes,
     void* stream, int64_t total_tokens);
 
-/* Measurement helper: fd_paged_decode_partial (same arguments, same results)
- * that also records when each workgroup of the decode launch reaches a few
+/* Entries of the arrival-counter array below. */
+#define FD_DECODE_COUNTERS 4096
+
+/* fd_paged_decode_partial_hint for a caller that keeps arrival counters
+ * beside its workspace: a device array of FD_DECODE_COUNTERS uint32, all zero
+ * before its first call (every call leaves it zero). Launches that may
+ * overlap need one each, like the workspace. Launches whose rows are cut by
+ * their lengths count each row's finished tasks there, so that the last one
+ * merges the row; without the array (the other entry points, or NULL) such a
+ * launch takes the counters from its workspace and clears them with a small
+ * launch of its own first. Same results either way. No counterpart in the
+ * reference. */
+int fd_paged_decode_counted(
+    const void* q, int64_t q_stride_seq, int64_t q_stride_head,
+    const void* k_cache, const void* v_cache,
+    int64_t kv_stride_block, int64_t kv_stride_head, int64_t kv_stride_token,
+    int64_t num_blocks,
+    const int32_t* block_table, int64_t bt_stride, int32_t bt_width,
+    const int32_t* lens, const int32_t* row_order,
+    int32_t n, int32_t num_heads, int32_t num_kv_heads, int32_t head_size,
+    int32_t block_size, float scale, int32_t kv_dtype,
+    void* out, int64_t out_stride_seq, int64_t out_stride_head,
+    int32_t out_dtype,
+    float* lse, int64_t lse_stride_head,
+    void* workspace, size_t workspace_bytes,
+    void* stream, int64_t total_tokens, uint32_t* counters);
+
+/* Measurement helper: fd_paged_decode_partial (same arguments; the same bits
+ * where fd_decode_balanced_parts gives 0, within rounding otherwise) that also records when each workgroup of the decode launch reaches a few
  * points, for launches that take the 16-bit VALU kernel (otherwise
  * FD_ERR_UNSUPPORTED, nothing launched). timeline: a device buffer of
  * timeline_workgroups * 8 uint64 (16-byte aligned, zeroed by the caller);
@@ -241,6 +268,19 @@ typedef struct {
 int fd_decode_plan_info(int32_t n, int32_t num_heads, int32_t num_kv_heads, int32_t head_size,
                         int32_t block_size, int32_t bt_width, int32_t kv_dtype, int32_t aligned,
                         int32_t host_tier, int64_t total_tokens, FdDecodePlan* plan);
+
+/* Whether a decode launch of these sizes (aligned, with the workspace the size
+ * query asks for) is cut by the rows' lengths on the device instead of by the
+ * table width: *parts is the number of tasks aimed at per kv head and
+ * head-group pass, 0 if the cut by table width that fd_decode_plan_info
+ * describes is launched (kernel, heads_per_task and passes hold either way).
+ * Cut by length are launches of fewer (sequence, kv head, pass) pairs than
+ * the GPU has CUs whose rows may be long enough to gain; the last task of a
+ * row merges its parts, so there is no combine pass. fd_paged_decode_timeline
+ * always cuts by table width. No counterpart in the reference. */
+int fd_decode_balanced_parts(int32_t n, int32_t num_heads, int32_t num_kv_heads,
+                             int32_t head_size, int32_t block_size, int32_t bt_width,
+                             int32_t kv_dtype, int32_t host_tier, int32_t* parts);
 
 /* Size of the device scratch behind fd_paged_decode_partial_noalloc. */
 #define FD_NOALLOC_SCRATCH_BYTES (32u << 20)
@@ -318,6 +358,20 @@ int fd_split_decode(
     float* lse, int64_t lse_stride_head,
     void* workspace, size_t workspace_bytes,
     void* stream);
+
+/* fd_split_decode with the caller's arrival counters
+ * (fd_paged_decode_counted). */
+int fd_split_decode_counted(
+    const void* q, int64_t q_stride_seq, int64_t q_stride_head,
+    const fd_kv_tier* hbm, const fd_kv_tier* host,
+    const int32_t* row_order,
+    int32_t n, int32_t num_heads, int32_t num_kv_heads, int32_t head_size,
+    int32_t block_size, float scale, int32_t kv_dtype,
+    void* out, int64_t out_stride_seq, int64_t out_stride_head,
+    int32_t out_dtype,
+    float* lse, int64_t lse_stride_head,
+    void* workspace, size_t workspace_bytes,
+    void* stream, uint32_t* counters);
 
 /* ------------------------------------------------------------------------
  * Device-side tier split of a decode step.

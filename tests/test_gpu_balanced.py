@@ -1,0 +1,189 @@
+"""Decode launches whose rows are cut by their lengths on the device
+(balanced_task in decode_tiled.h) against the float64 oracle, where that cut
+can go wrong: one row and rows on both sides of a 64-lane group, empty and
+one-token rows among long ones, rows longer than the 256 blocks a task holds,
+parts forced down to the smallest size, every kernel family, one tier and two,
+an order that leaves rows out, range errors, and the entry points with and
+without arrival counters. Bars of test_gpu_decode: fp32 out 2e-3 (fp32 KV
+5e-5), lse 1e-4 relative."""
+
+from __future__ import annotations
+
+import ctypes
+import math
+
+import pytest
+import torch
+
+import oracle
+from tests.test_gpu_decode import assert_lse_close, assert_out_close
+from tests.test_gpu_split_fused import run_fused, two_tier_case
+from vllm_fastdecoder_amd import _lib, ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(lens, H, KVH, D, dtype, seed, spare=8):
+    """Rows of the given lengths over a shuffled pool, host layout."""
+    BS = 16
+    g = torch.Generator().manual_seed(seed)
+    nb = [-(-x // BS) for x in lens]
+    pool = sum(nb) + 1
+    perm = torch.randperm(pool, generator=g).to(torch.int32)
+    bt = torch.zeros(len(lens), max(nb) + spare, dtype=torch.int32)
+    pos = 0
+    for i, k in enumerate(nb):
+        bt[i, :k] = perm[pos:pos + k]
+        pos += k
+    q = torch.randn(len(lens), H, D, generator=g).to(dtype)
+    kc = torch.randn(pool, KVH, BS, D, generator=g).to(dtype)
+    vc = torch.randn(pool, KVH, BS, D, generator=g).to(dtype)
+    return q, kc, vc, bt, torch.tensor(lens, dtype=torch.int32)
+
+
+def _run(case, dev, out=None, lse=None, row_order=None):
+    q, kc, vc, bt, lens = case
+    n, H, D = q.shape
+    out = torch.empty(n, H, D, device=dev) if out is None else out
+    lse = torch.empty(H, n, device=dev) if lse is None else lse
+    ops.decode_attn(q.to(dev), kc.to(dev), vc.to(dev), bt.to(dev), lens.to(dev),
+                    1 / math.sqrt(D), out, lse, row_order=row_order)
+    torch.cuda.synchronize()
+    return out, lse
+
+
+def _check(case, out, lse, rows=slice(None)):
+    q, kc, vc, bt, lens = case
+    ref_out, ref_lse = oracle.decode_attn_host_layout_f64(q, kc, vc, bt, lens,
+                                                          1 / math.sqrt(q.shape[2]))
+    tol = 5e-5 if q.dtype == torch.float32 else 2e-3
+    nz = lens[rows] > 0
+    out, lse = out[rows].cpu(), lse[:, rows].cpu()
+    assert_out_close(out, ref_out[rows], tol, mask=nz)
+    assert_lse_close(lse, ref_lse[:, rows], mask=nz)
+    assert torch.all(out[~nz] == 0) and torch.all(torch.isneginf(lse[:, ~nz]))
+
+
+def _lens(n, seed, hi=900):
+    """Rows of 0 to hi tokens: empty, one-token and block-edge rows first."""
+    g = torch.Generator().manual_seed(seed)
+    lens = torch.randint(0, hi, (n,), generator=g).tolist()
+    for k, x in enumerate((hi, 0, 1, 15, 16, 17)):
+        if k < n:
+            lens[k] = x
+    return lens
+
+
+@pytest.mark.parametrize("H,KVH,D,dtype", [
+    (2, 2, 128, torch.float16), (4, 2, 128, torch.bfloat16), (2, 2, 64, torch.bfloat16),
+    (2, 2, 80, torch.float16), (4, 2, 256, torch.bfloat16),       # VALU
+    (8, 2, 128, torch.bfloat16), (14, 2, 64, torch.float16), (16, 1, 96, torch.bfloat16),  # mm
+    (8, 2, 256, torch.bfloat16),                                  # mfma
+    (2, 2, 128, torch.float32), (8, 2, 72, torch.float32), (20, 2, 256, torch.float32),  # f32
+])
+@pytest.mark.parametrize("n", [1, 7, 65])
+def test_forced_cuts_match_oracle(gpu, H, KVH, D, dtype, n, monkeypatch):
+    """Cuts wherever they can be made: about three parts per row and kv head."""
+    monkeypatch.setenv("FD_BALANCE", str(3 * n * KVH))
+    case = _case(_lens(n, n + D), H, KVH, D, dtype, seed=n)
+    assert ops.balanced_parts(n, H, KVH, D, 16, case[3].shape[1], dtype) > 0
+    out, lse = _run(case, gpu)
+    _check(case, out, lse)
+
+
+@pytest.mark.parametrize("n,want", [(1, 1), (2, 512), (63, 70), (64, 256), (65, 66), (130, 512),
+                                    (512, 700)])
+def test_row_counts_and_part_counts(gpu, n, want, monkeypatch):
+    """From fewer parts than cut rows need (they stay whole) to parts of the
+    smallest size; row counts around the 64-lane groups, up to the most the
+    cut takes."""
+    monkeypatch.setenv("FD_BALANCE", str(want))
+    case = _case(_lens(n, n, hi=400 if n > 64 else 1500), 8, 1, 128, torch.bfloat16, seed=n)
+    _check(case, *_run(case, gpu))
+
+
+def test_rows_past_one_tasks_blocks(gpu, monkeypatch):
+    """One part per row wanted, rows of more than 256 blocks: the parts stop at
+    the 256 blocks a task can hold."""
+    monkeypatch.setenv("FD_BALANCE", "2")
+    case = _case([9000, 33, 4097, 0], 4, 1, 128, torch.float16, seed=5)
+    _check(case, *_run(case, gpu))
+
+
+def test_chosen_by_the_plan(gpu):
+    """A small grouped-query batch takes the cut by itself, and gives the same
+    bits on every call (the counters are back at zero) and in any order; a
+    batch of one row per CU does not take it."""
+    case = _case([900, 2500, 64, 700, 3000], 32, 8, 128, torch.bfloat16, seed=9)
+    assert ops.balanced_parts(5, 32, 8, 128, 16, case[3].shape[1], torch.bfloat16) > 0
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert ops.balanced_parts(cus // 8, 32, 8, 128, 16, 256, torch.bfloat16) == 0
+    first = _run(case, gpu)
+    _check(case, *first)
+    for order in (None, torch.tensor([4, 1, 0, 3, 2], dtype=torch.int32)):
+        again = _run(case, gpu, row_order=order)
+        assert torch.equal(again[0], first[0]) and torch.equal(again[1], first[1])
+
+
+def test_order_entries_outside_the_rows_are_skipped(gpu, monkeypatch):
+    monkeypatch.setenv("FD_BALANCE", "64")
+    case = _case([900, 500, 64, 700], 8, 2, 128, torch.bfloat16, seed=10)
+    out = torch.full((4, 8, 128), 7.0, device=gpu)
+    lse = torch.full((8, 4), 7.0, device=gpu)
+    _run(case, gpu, out, lse, row_order=torch.tensor([3, -1, 0, 9], dtype=torch.int32))
+    _check(case, out, lse, rows=[0, 3])
+    assert torch.all(out[[1, 2]] == 7.0) and torch.all(lse[:, [1, 2]] == 7.0)
+
+
+def test_range_errors_stay_in_their_rows(gpu, monkeypatch):
+    """A bad block id and a length past the table: NaN in those rows only."""
+    monkeypatch.setenv("FD_BALANCE", "96")
+    case = _case([900, 800, 700, 600], 8, 2, 128, torch.bfloat16, seed=11, spare=0)
+    q, kc, vc, bt, lens = case
+    bad_bt, bad_lens = bt.clone(), lens.clone()
+    bad_bt[1, 40] = kc.shape[0]
+    bad_lens[2] = bt.shape[1] * 16 + 1
+    out, lse = _run((q, kc, vc, bad_bt, bad_lens), gpu)
+    assert torch.isnan(out[[1, 2]]).all() and torch.isnan(lse[:, [1, 2]]).all()
+    _check(case, out, lse, rows=[0, 3])
+
+
+@pytest.mark.parametrize("H,KVH,dtype", [(4, 4, torch.float16), (8, 2, torch.bfloat16),
+                                         (8, 2, torch.float32)])
+def test_two_tiers(gpu, H, KVH, dtype, monkeypatch):
+    """Cuts anywhere in a row's two block lists, both tiers ending in a partial
+    block, against the launch that is not cut this way."""
+    c = two_tier_case(9, H, KVH, 128, dtype, seed=3, dev=gpu, gpu_first=False)
+    monkeypatch.setenv("FD_BALANCE", "0")
+    ref_out, ref_lse = run_fused(c, gpu)
+    monkeypatch.setenv("FD_BALANCE", str(30 * KVH))
+    out, lse = run_fused(c, gpu)
+    assert not torch.equal(out, ref_out)  # another cut: summed in another order
+    torch.testing.assert_close(out, ref_out, atol=2e-5, rtol=0)
+    torch.testing.assert_close(lse, ref_lse, atol=1e-5, rtol=1e-5)
+
+
+def test_entry_points_without_counters(gpu):
+    """The C entry points that bring no counters: a workspace of the query's
+    size, full of ones, gives the counted call's bits; one that only covers
+    the cut by table width (here none) is still taken."""
+    case = _case([900, 500, 64], 32, 8, 128, torch.bfloat16, seed=12, spare=0)
+    q, kc, vc, bt, lens = (x.to(gpu) for x in case)
+    ref = _run(case, gpu)
+    lib = _lib.load_lib()
+    need = ops.workspace_bytes(3, 32, 8, 128, 16, bt.shape[1])
+    assert need > 0
+    for size in (need, 0):
+        ws = torch.full((max(size, 1),), 0xFF, dtype=torch.uint8, device=gpu)
+        out, lse = torch.empty(3, 32, 128, device=gpu), torch.empty(32, 3, device=gpu)
+        _lib.check(lib.fd_paged_decode_partial(
+            q.data_ptr(), q.stride(0), q.stride(1), kc.data_ptr(), vc.data_ptr(), kc.stride(0),
+            kc.stride(1), kc.stride(2), kc.shape[0], bt.data_ptr(), bt.stride(0), bt.shape[1],
+            lens.data_ptr(), None, 3, 32, 8, 128, 16, 1 / math.sqrt(128), _lib.FD_BF16,
+            out.data_ptr(), out.stride(0), out.stride(1), _lib.FD_F32, lse.data_ptr(),
+            lse.stride(0), ws.data_ptr() if size else None, ctypes.c_size_t(size),
+            torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        if size:
+            assert torch.equal(out, ref[0]) and torch.equal(lse, ref[1])
+        _check(case, out, lse)

@@ -144,7 +144,16 @@ int run_decode(DecodeArgs& a, const char* who, const void* q, int64_t q_stride_s
   if (host)
     sp = plan_decode(n, num_heads, num_kv_heads, head_size, block_size, (int32_t)width, kv_dtype,
                      aligned, false, fill);
-  const size_t need = decode_workspace_bytes(sp, n, num_heads, head_size);
+  // Balanced cuts need a workspace for whatever the rows' lengths make of
+  // them. A caller that brings less (it planned without them) gets the cuts
+  // by table width.
+  const size_t bal = balanced_partial_bytes(sp, num_heads, head_size) +
+                     (a.counters == nullptr ? balanced_counter_bytes(sp, n, num_kv_heads) : 0);
+  if (bal > 0 && (workspace == nullptr || workspace_bytes < bal || !aligned16(workspace)))
+    sp.bal_parts = 0;
+  // a timeline is of whole tasks by table width, as its buffer is sized for
+  if (a.timeline != nullptr) sp.bal_parts = 0;
+  const size_t need = sp.bal_parts > 0 ? 0 : decode_workspace_bytes(sp, n, num_heads, head_size);
   if (need > 0 && (workspace == nullptr || workspace_bytes < need || !aligned16(workspace)))
     return set_error(FD_ERR_WORKSPACE,
                      "%s: workspace of %zu bytes (16-byte aligned) required, got %zu", who, need,
@@ -181,7 +190,7 @@ extern "C" {
 
 const char* fd_last_error(void) { return g_err; }
 
-int fd_abi_version(void) { return 12; }
+int fd_abi_version(void) { return 13; }
 
 int fd_paged_decode_workspace_size(int32_t n, int32_t num_heads, int32_t num_kv_heads,
                                    int32_t head_size, int32_t block_size, int32_t bt_width,
@@ -203,6 +212,9 @@ int fd_paged_decode_workspace_size(int32_t n, int32_t num_heads, int32_t num_kv_
     // what a token total may make of it (fd_paged_decode_partial_hint)
     most = std::max(most, fill_workspace_bound(sp, n, num_heads, num_kv_heads, head_size,
                                                block_size, bt_width, dts[c]));
+    // balanced cuts, with room for the arrival counters
+    most = std::max(most, balanced_partial_bytes(sp, num_heads, head_size) +
+                              balanced_counter_bytes(sp, n, num_kv_heads));
   }
   *bytes = most;
   return FD_OK;
@@ -236,6 +248,19 @@ int fd_decode_plan_info(int32_t n, int32_t num_heads, int32_t num_kv_heads, int3
   plan->max_splits = sp.max_splits;
   plan->wg_cap = sp.fast ? sp.wg_cap : 0;
   plan->wave_blocks = sp.fast ? sp.wave_blocks : 0;
+  return FD_OK;
+}
+
+int fd_decode_balanced_parts(int32_t n, int32_t num_heads, int32_t num_kv_heads,
+                             int32_t head_size, int32_t block_size, int32_t bt_width,
+                             int32_t kv_dtype, int32_t host_tier, int32_t* parts) {
+  if (parts == nullptr) return set_error(FD_ERR_INVALID, "balanced_parts: parts is NULL");
+  if (n < 0 || num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads != 0 ||
+      head_size <= 0 || block_size <= 0 || bt_width < 0 || !valid_dtype(kv_dtype))
+    return set_error(FD_ERR_INVALID, "balanced_parts: bad sizes");
+  *parts = plan_decode(n, num_heads, num_kv_heads, head_size, block_size, bt_width, kv_dtype, true,
+                       host_tier == 0)
+               .bal_parts;
   return FD_OK;
 }
 
@@ -279,6 +304,26 @@ int fd_paged_decode_partial_hint(
                     workspace_bytes, stream, total_tokens);
 }
 
+int fd_paged_decode_counted(
+    const void* q, int64_t q_stride_seq, int64_t q_stride_head, const void* k_cache,
+    const void* v_cache, int64_t kv_stride_block, int64_t kv_stride_head,
+    int64_t kv_stride_token, int64_t num_blocks, const int32_t* block_table, int64_t bt_stride,
+    int32_t bt_width, const int32_t* lens, const int32_t* row_order, int32_t n,
+    int32_t num_heads, int32_t num_kv_heads, int32_t head_size, int32_t block_size, float scale,
+    int32_t kv_dtype, void* out, int64_t out_stride_seq, int64_t out_stride_head,
+    int32_t out_dtype, float* lse, int64_t lse_stride_head, void* workspace,
+    size_t workspace_bytes, void* stream, int64_t total_tokens, uint32_t* counters) {
+  DecodeArgs a{};
+  a.tier[0] = KvTier{k_cache, v_cache, kv_stride_block, kv_stride_head, kv_stride_token,
+                     num_blocks, block_table, bt_stride, bt_width, lens};
+  a.ntiers = 1;
+  a.counters = counters;
+  return run_decode(a, "decode", q, q_stride_seq, q_stride_head, row_order, n, num_heads,
+                    num_kv_heads, head_size, block_size, scale, kv_dtype, out, out_stride_seq,
+                    out_stride_head, out_dtype, lse, lse_stride_head, workspace,
+                    workspace_bytes, stream, total_tokens);
+}
+
 int fd_paged_decode_timeline(
     const void* q, int64_t q_stride_seq, int64_t q_stride_head, const void* k_cache,
     const void* v_cache, int64_t kv_stride_block, int64_t kv_stride_head,
@@ -304,13 +349,13 @@ int fd_paged_decode_timeline(
                     workspace_bytes, stream);
 }
 
-int fd_split_decode(const void* q, int64_t q_stride_seq, int64_t q_stride_head,
+int fd_split_decode_counted(const void* q, int64_t q_stride_seq, int64_t q_stride_head,
                     const fd_kv_tier* hbm, const fd_kv_tier* host, const int32_t* row_order,
                     int32_t n, int32_t num_heads, int32_t num_kv_heads, int32_t head_size,
                     int32_t block_size, float scale, int32_t kv_dtype, void* out,
                     int64_t out_stride_seq, int64_t out_stride_head, int32_t out_dtype,
                     float* lse, int64_t lse_stride_head, void* workspace,
-                    size_t workspace_bytes, void* stream) {
+                    size_t workspace_bytes, void* stream, uint32_t* counters) {
   if (hbm == nullptr || host == nullptr)
     return set_error(FD_ERR_INVALID, "split_decode: NULL tier descriptor");
   DecodeArgs a{};
@@ -321,10 +366,24 @@ int fd_split_decode(const void* q, int64_t q_stride_seq, int64_t q_stride_head,
                        d.num_blocks, d.block_table, d.bt_stride, d.bt_width, d.lens};
   }
   a.ntiers = 2;
+  a.counters = counters;
   return run_decode(a, "split_decode", q, q_stride_seq, q_stride_head, row_order, n, num_heads,
                     num_kv_heads, head_size, block_size, scale, kv_dtype, out, out_stride_seq,
                     out_stride_head, out_dtype, lse, lse_stride_head, workspace,
                     workspace_bytes, stream);
+}
+
+int fd_split_decode(const void* q, int64_t q_stride_seq, int64_t q_stride_head,
+                    const fd_kv_tier* hbm, const fd_kv_tier* host, const int32_t* row_order,
+                    int32_t n, int32_t num_heads, int32_t num_kv_heads, int32_t head_size,
+                    int32_t block_size, float scale, int32_t kv_dtype, void* out,
+                    int64_t out_stride_seq, int64_t out_stride_head, int32_t out_dtype,
+                    float* lse, int64_t lse_stride_head, void* workspace,
+                    size_t workspace_bytes, void* stream) {
+  return fd_split_decode_counted(q, q_stride_seq, q_stride_head, hbm, host, row_order, n,
+                                 num_heads, num_kv_heads, head_size, block_size, scale, kv_dtype,
+                                 out, out_stride_seq, out_stride_head, out_dtype, lse,
+                                 lse_stride_head, workspace, workspace_bytes, stream, nullptr);
 }
 
 int fd_plan_tiers(const int32_t* block_table, int64_t bt_stride, int32_t bt_width,

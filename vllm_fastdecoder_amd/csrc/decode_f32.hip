@@ -186,9 +186,7 @@ __global__ __launch_bounds__(kWave * kWavesPerTask) void decode_f32_kernel(Tiled
   }
 
   publish_wave_state<D, G>(ws, wave, lane, m, l, acc, wb.bad);
-  __syncthreads();
-  if (wave != 0) return;
-  finish_task<F32, D, G>(p, t, ws, lane);
+  end_task<F32, D, G>(p, t, ws, wave, lane);
 }
 
 template <int D, int G>

@@ -277,9 +277,7 @@ __global__ __launch_bounds__(kWave * kWavesPerTask) void decode_mfma_kernel(Tile
     ws.l[wave][lane] = lt;
   }
   if (lane == 0) ws.bad[wave] = wb.bad ? 1 : 0;
-  __syncthreads();
-  if (wave != 0) return;
-  finish_task<T, D, G>(p, t, ws, lane);
+  end_task<T, D, G>(p, t, ws, wave, lane);
 }
 
 template <typename T, int D, int G>

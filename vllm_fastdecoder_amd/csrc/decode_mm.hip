@@ -98,6 +98,7 @@ struct __align__(16) MmLds {  // 16-byte V rows, float4 merge reads
     float m[kWavesPerTask][kCols];
     float l[kWavesPerTask][kCols];
     int bad[kWavesPerTask];
+    int last;  // balanced cuts: this task is its row's last to arrive
   };
   union {
     uint16_t stage[kStage];
@@ -345,11 +346,13 @@ __global__ __launch_bounds__(kWave * kWavesPerTask) void decode_mm_kernel(TiledP
   for (int g = 0; g < CG; ++g) {
     const float lt = xor_sum<16>(l[g]);
     __syncthreads();  // the V staging (g = 0) or the previous group's merge is done
+    if (kCols * g + 4 * R < t.gcount) {  // rows of real columns
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
+      for (int c = 0; c < NC; ++c) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        mg.acc[wave][4 * R + e][16 * c + col] = acc[g][c][e] * (1.f / kPScale);
+        for (int e = 0; e < 4; ++e)
+          mg.acc[wave][4 * R + e][16 * c + col] = acc[g][c][e] * (1.f / kPScale);
+      }
     }
     if (lane < kCols) {
       mg.m[wave][lane] = m[g];
@@ -392,9 +395,9 @@ __global__ __launch_bounds__(kWave * kWavesPerTask) void decode_mm_kernel(TiledP
       const float inv = 1.f / ltot;
 #pragma unroll
       for (int e = 0; e < 8; ++e) o[e] *= inv;
-      float lse_nat = (M + fast_log2(ltot)) * kLn2;
+      float lse2 = M + fast_log2(ltot);
       if (bad) {
-        lse_nat = qnan();
+        lse2 = qnan();
 #pragma unroll
         for (int e = 0; e < 8; ++e) o[e] = qnan();
       }
@@ -403,14 +406,17 @@ __global__ __launch_bounds__(kWave * kWavesPerTask) void decode_mm_kernel(TiledP
         const int h = t.h0 + hc;
         if (write_final) {
           store8<T>(p.out, (int64_t)t.i * p.out_ss + (int64_t)h * p.out_sh + d0, p.out_f32, o);
-          if (d0 == 0) p.lse[(int64_t)h * p.lse_sh + t.i] = lse_nat;
+          if (d0 == 0) p.lse[(int64_t)h * p.lse_sh + t.i] = lse2 * kLn2;
         } else {
-          const int64_t pidx = ((int64_t)t.i * p.H + h) * p.S + t.split;
-          store8<T>(p.part_o, pidx * p.D + d0, true, o);
-          if (d0 == 0) p.part_lse[pidx] = lse_nat;
+          store_partial(p, t, h, d0, o, lse2);
         }
       }
     }
+  }
+  // a balanced launch (one column group): the row's last task merges its parts
+  if constexpr (CG == 1) {
+    if (p.bal_parts == 0 || t.nsplit == 1) return;
+    if (last_to_arrive(p, t, &mg.last)) merge_parts<T, D>(p, t);
   }
 }
 

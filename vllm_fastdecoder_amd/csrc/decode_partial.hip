@@ -191,7 +191,9 @@ __global__ __launch_bounds__(kWave) void decode_generic_kernel(GenericParams p) 
 //                        matrix cores (4+ query heads per kv head), the one
 //                        with P.V there too (D <= 128);
 //   FD_WAVE_BLOCKS=<b>   blocks per working wave (0: every wave works);
-//   FD_WG_CAP=<k>        at most k workgroups per CU (0: no cap).
+//   FD_WG_CAP=<k>        at most k workgroups per CU (0: no cap);
+//   FD_BALANCE=<w>       balanced cuts aiming at w workgroups wherever they can be made
+//                        (0: none).
 // Like getenv, the first definition of a name counts.
 struct Tuning {
   const char* split_blocks = nullptr;
@@ -199,6 +201,7 @@ struct Tuning {
   const char* kernel = nullptr;
   const char* wave_blocks = nullptr;
   const char* wg_cap = nullptr;
+  const char* balance = nullptr;
 
   bool kernel_forced(const char* name) const {
     return kernel != nullptr && strcmp(kernel, name) == 0;
@@ -222,6 +225,7 @@ Tuning read_tuning() {
     else if (!t.kernel && (v = value(s, "DECODE_KERNEL"))) t.kernel = v;
     else if (!t.wave_blocks && (v = value(s, "WAVE_BLOCKS"))) t.wave_blocks = v;
     else if (!t.wg_cap && (v = value(s, "WG_CAP"))) t.wg_cap = v;
+    else if (!t.balance && (v = value(s, "BALANCE"))) t.balance = v;
   }
   return t;
 }
@@ -437,6 +441,78 @@ int32_t quarter_row_blocks(int32_t n, int32_t kv_tasks, int32_t D, bool f32, boo
   return 0;
 }
 
+// ---------------------------------------------------------- balanced cuts
+// Launches of fewer (sequence, kv-head pass) pairs than CUs: the rows are cut
+// on the device by their lengths (decode_tiled.h, balanced_task) so that one
+// round of workgroups, one or two per CU, streams equal shares, and a row's
+// last task merges its parts in the kernel. The plan by table width above
+// gave such launches one task per row or fixed-size tasks: the CUs holding
+// the longest rows finished last, and split rows paid a combine launch
+// (4-5 us). Measured on MI355X against that plan (HIP graph replay, us, the
+// same inputs in turn; 6.8 TB/s floor in brackets):
+//   1 x 900 tokens, 32/8 heads, bf16 [0.5]                14.0 -> 7.8
+//   64 x U[1024, 4096], 8/1, bf16 [12.1]                  22.7 -> 19.0
+//   40 x U[50, 3100], 28/4, bf16 [21.4]                   33.8 -> 29.7
+//   24 x U[200, 4000], 16/8, D = 256, bf16 [56.0]         95.2 -> 66.8
+//   12 x U[64, 1500], 32/8, fp32 [10.7]                   25.9 -> 19.8
+//   3 x U[12k, 50k], 32/8, bf16 [55.4]                    77.3 -> 62.1
+//   4 x U[3000, 9000], 32/32, fp16 [42.5]                 59.5 -> 48.8
+//   1 x 100,000, 8/1, bf16 [7.5]                          77.5 -> 32.8
+// The lines of the rule:
+//   * pairs < CUs: from one pair per CU on, whole rows already fill the GPU
+//     and balance by themselves (256 pairs of U[1024, 4096], 32/8: 65 us
+//     either way; 512 pairs 115 -> 122, the merges cost what the cut gains).
+//   * one workgroup per CU up to 0.4 pairs per CU, two above: few pairs are
+//     cut finely enough at one (12 x 8 pairs fp32: 19.8 at one, 20.9 at two;
+//     64 x 1: 19.1 / 20.4), many need the finer parts of two (160 pairs: 36.6
+//     at one, 29.7 at two; 192 pairs: 71.9 / 66.8). Three are worse (uneven
+//     rounds, more merges: 30.7, 69.6).
+//   * a cut has to save kBalMerge blocks of 8 KiB on the longest row, about
+//     what a merge adds (partial written 0.7 us, arrival 1 us, merge 1.5 us, and
+//     ~0.8 us for the cut itself): checked here against the table width,
+//     which bounds the row, and in the kernel against the row. 8 x 32 rows of
+//     U[128, 1024] (whole rows 15.7 us) lose cut (16.5).
+// FD_SPLIT_BLOCKS (forced tasks) turns the cuts off.
+constexpr double kBalTileBytes = 8192.0;  // the unit of the figures below
+constexpr double kBalMerge = 20.0;        // blocks one task streams in the time a merge adds
+constexpr double kBalRates = 1.65;        // a task's own rate (45 GB/s) over a 256th of HBM's
+constexpr double kBalMinBlocks = 8.0;     // smallest part (4: 9.2 us instead of 9.1 above, 16: 10.5)
+
+void plan_balanced(SplitPlan& sp, const Tuning& tune, int32_t n, int32_t H, int32_t D,
+                   int32_t kv_tasks, int32_t G, int32_t wt, int32_t elt, int cus) {
+  if (cus <= 0 || n <= 0 || n > kMaxBalRows || G > 16 || wt <= 0 || wt > kMaxBalBlocks) return;
+  if (tune.split_blocks != nullptr && atoi(tune.split_blocks) > 0) return;
+  const int64_t pairs = (int64_t)n * kv_tasks;
+  const double units = 2.0 * kTileTokens * D * elt / kBalTileBytes;  // of one block
+  const int32_t least = std::max(2, (int32_t)(kBalMinBlocks / units));
+  const int32_t whole = (int32_t)(kBalMerge / units);
+  int64_t want = 0;  // workgroups
+  if (tune.balance != nullptr) {
+    want = atoi(tune.balance);
+  } else if (pairs < cus && wt > least + whole &&
+             (double)(cus - pairs) * wt * units > kBalMerge * cus) {
+    want = 5 * pairs <= 2LL * cus ? cus : 2LL * cus;
+  }
+  if (want <= 0 || pairs > kMaxBalPairs) return;
+  const int64_t parts = std::max<int64_t>(n, want / kv_tasks);
+  // parts the lengths can make at most: see balanced_task (a part holds at
+  // most kMaxSplitBlocks blocks), and a row of the table's width alone
+  const int64_t over = ((int64_t)n * wt + kMaxSplitBlocks - 1) / kMaxSplitBlocks;
+  const int64_t grid = std::min(std::max(parts, over) + n, (int64_t)n * ((wt + least - 1) / least));
+  if (grid <= n) return;  // no row can be cut
+  // a row's partials have 32-bit byte offsets, the grid divides as small_div does
+  if (grid * H * D >= (1 << 28) || grid * kv_tasks >= (1 << 22)) return;
+  sp.bal_parts = (int32_t)parts;
+  sp.bal_min = least;
+  sp.bal_grid = (int32_t)grid;
+  // (forced cuts, for comparison runs and tests, cut what they can)
+  sp.bal_whole = tune.balance != nullptr ? -kMaxBalBlocks : whole;
+  sp.bal_share = (float)(kBalRates * kv_tasks / cus);
+  const int64_t cap = (parts * kv_tasks + cus - 1) / cus;
+  sp.bal_cap = cap <= 4 ? (int32_t)cap : 0;
+  if (tune.wg_cap != nullptr && *tune.wg_cap != 0) sp.bal_cap = std::max(0, atoi(tune.wg_cap));
+}
+
 }  // namespace
 
 // Blocks per task (16 .. 256) from a launch-time model. Only the shapes are
@@ -598,6 +674,7 @@ SplitPlan plan_decode(int32_t n, int32_t H, int32_t KVH, int32_t D, int32_t BS,
     const int32_t longest = std::min(sb, wt > 0 ? wt : 1);
     sp.wave_blocks = (longest + kWavesPerTask - 1) / kWavesPerTask;
   }
+  plan_balanced(sp, tune, n, H, D, kv_tasks, G, wt, elt, cus);
   if (tune.wave_blocks != nullptr) sp.wave_blocks = std::max(0, atoi(tune.wave_blocks));
   if (tune.wg_cap != nullptr && *tune.wg_cap != 0) sp.wg_cap = std::max(0, atoi(tune.wg_cap));
   return sp;
@@ -627,6 +704,23 @@ size_t decode_workspace_bytes(const SplitPlan& sp, int32_t n, int32_t H, int32_t
   if (sp.max_splits <= 1) return 0;
   const size_t parts = (size_t)n * H * sp.max_splits;
   return parts * D * sizeof(float) + parts * sizeof(float) + 256;
+}
+
+size_t balanced_partial_bytes(const SplitPlan& sp, int32_t H, int32_t D) {
+  if (sp.bal_parts <= 0) return 0;
+  const size_t parts = (size_t)sp.bal_grid * H;
+  return (parts * (D + 1) * sizeof(float) + 255) / 256 * 256;
+}
+
+size_t balanced_counter_bytes(const SplitPlan& sp, int32_t n, int32_t KVH) {
+  return sp.bal_parts > 0 ? (size_t)n * KVH * sp.passes * sizeof(uint32_t) : 0;
+}
+
+// Clears a balanced launch's arrival counters where the caller keeps none.
+// (A kernel, not a memset: the call may be captured in a graph.)
+__global__ __launch_bounds__(256) void clear_counters_kernel(uint32_t* c, int32_t count) {
+  const int32_t k = blockIdx.x * 256 + threadIdx.x;
+  if (k < count) c[k] = 0;
 }
 
 int launch_decode(const DecodeArgs& a, const SplitPlan& sp, hipStream_t s) {
@@ -715,20 +809,44 @@ int launch_decode(const DecodeArgs& a, const SplitPlan& sp, hipStream_t s) {
   tp.wave_blocks = sp.wave_blocks;
   tp.xcd_group = a.D % 64 != 0;
   tp.timeline = a.timeline;
+  const bool balanced = sp.bal_parts > 0;
   const size_t parts = (size_t)a.n * a.H * sp.max_splits;
-  if (sp.max_splits > 1) {
+  if (balanced) {
+    const size_t bparts = (size_t)sp.bal_grid * a.H;
+    tp.part_o = static_cast<float*>(a.workspace);
+    tp.part_lse = tp.part_o + bparts * a.D;
+    tp.bal_parts = sp.bal_parts;
+    tp.bal_min = sp.bal_min;
+    tp.bal_whole = sp.bal_whole;
+    tp.bal_share = sp.bal_share;
+    tp.order = a.order;
+    tp.wave_blocks = 0;
+    tp.counters = a.counters;
+    if (tp.counters == nullptr) {
+      const int32_t count = a.n * a.KVH * sp.passes;
+      tp.counters = reinterpret_cast<uint32_t*>(static_cast<char*>(a.workspace) +
+                                                balanced_partial_bytes(sp, a.H, a.D));
+      hipLaunchKernelGGL(clear_counters_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256),
+                         0, s, tp.counters, count);
+      const hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return hip_error(e, "clear_counters_kernel launch");
+    }
+  } else if (sp.max_splits > 1) {
     char* ws = static_cast<char*>(a.workspace);
     tp.part_o = reinterpret_cast<float*>(ws);
     tp.part_lse = reinterpret_cast<float*>(ws + parts * a.D * sizeof(float));
   }
-  const int64_t tasks = (int64_t)a.n * a.KVH * sp.passes * sp.max_splits;
+  const int64_t tasks = balanced ? (int64_t)sp.bal_grid * a.KVH * sp.passes
+                                 : (int64_t)a.n * a.KVH * sp.passes * sp.max_splits;
   if (tasks > INT32_MAX) return set_error(FD_ERR_UNSUPPORTED, "decode: too many tasks");
   if (a.timeline != nullptr && tasks > a.timeline_tasks)
     return set_error(FD_ERR_INVALID, "decode_timeline: %lld workgroups, room for %lld",
                      (long long)tasks, (long long)a.timeline_tasks);
-  hipError_t e = dispatch_tiled(tp, (unsigned)tasks, sp, a.kv_dtype, a.D, two, s);
+  SplitPlan lp = sp;
+  if (balanced) lp.wg_cap = sp.bal_cap;
+  hipError_t e = dispatch_tiled(tp, (unsigned)tasks, lp, a.kv_dtype, a.D, two, s);
   if (e != hipSuccess) return hip_error(e, "decode kernel launch");
-  if (sp.max_splits > 1) {
+  if (!balanced && sp.max_splits > 1) {
     const int64_t threads = (int64_t)a.n * a.H * (a.D / 4);
     hipLaunchKernelGGL(combine_splits_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256),
                        0, s, tp.part_o, tp.part_lse, a.tier[0].lens,

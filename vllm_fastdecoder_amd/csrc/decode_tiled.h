@@ -81,6 +81,12 @@ struct TiledParams {
   int32_t S;        // max splits per (sequence, kv head)
   int32_t split_blocks;
   int32_t wave_blocks;  // blocks per working wave (0: every wave works; wave_blocks())
+  int32_t bal_parts;  // > 0: balanced cuts (balanced_task()): parts per kv-head pass aimed at
+  int32_t bal_min;    // balanced cuts: blocks per part at least
+  int32_t bal_whole;  // balanced cuts: blocks a cut has to save (whole rows otherwise)
+  float bal_share;    // balanced cuts: blocks of one task's own rate in the time in which HBM
+                      // delivers one block of every row of all kv-head passes together
+  uint32_t* counters; // balanced cuts: arrivals per (sequence, kv-head pass), zero between launches
   bool xcd_group;   // adjacent kv heads of a row on one XCD (xcd_task)
   uint64_t* timeline;  // measurement only: kTimelineSlots stamps per workgroup (NULL: none)
 };
@@ -238,6 +244,20 @@ __device__ __forceinline__ void store8(void* out, int64_t off, bool f32, const f
   }
 }
 
+// The same for 4 outputs.
+template <typename T>
+__device__ __forceinline__ void store4(void* out, int64_t off, bool f32, const float* o) {
+  if (std::is_same<T, F32>::value || f32) {
+    *reinterpret_cast<float4*>(static_cast<float*>(out) + off) =
+        make_float4(o[0], o[1], o[2], o[3]);
+  } else if constexpr (!std::is_same<T, F32>::value) {
+    uint2 u;
+    u.x = to_out(T{}, o[0]) | (uint32_t(to_out(T{}, o[1])) << 16);
+    u.y = to_out(T{}, o[2]) | (uint32_t(to_out(T{}, o[3])) << 16);
+    *reinterpret_cast<uint2*>(static_cast<uint16_t*>(out) + off) = u;
+  }
+}
+
 // ---------------------------------------------------------------- tasks
 
 // One task of a tiled launch: (sequence i, kv head kh, split) and the range
@@ -252,6 +272,7 @@ struct Task {
   int nba, nb;
   int b_begin, b_end, nsplit;
   bool range_bad;  // a length needs more blocks than its table has
+  int kp, slot0;   // balanced cuts: kv-head pass of the task, first part of its row
 };
 
 // blockIdx.x -> task: kv head fastest, then head group (one unless a kv head
@@ -284,8 +305,177 @@ __device__ __forceinline__ int xcd_task(int b, int tasks) {
   return (g + 1) * kGroup <= tasks ? g * kGroup + kXcdHeads * (r % kXcds) + r / kXcds : b;
 }
 
+// Balanced cuts: how the launch's tasks are drawn from the rows' lengths
+// themselves, on the device. The launch wants at most S = bal_parts parts per
+// kv-head pass (as many workgroups as the CUs take at once, one round): a
+// part holds at most c blocks, a row of nb blocks is cut into ceil(nb / c)
+// parts of equal size (+-1), a row without blocks is one part, and c is the
+// first size tried at which all rows make at most S parts. Then all tasks
+// start together and stream about the same share, however uneven the rows
+// and however wide the table is. The host cannot do this: it sees neither
+// the lengths nor (without a token total) their sum. Whatever c the search
+// ends at, there are at most S + n parts (c >= N / S for the N blocks of all
+// rows), or N / 256 + n when parts reach the 256 blocks a task can hold: the
+// grid's bound. Workgroups past the last part return.
+//
+// Every wave works the cut out by itself from the n lengths (one load per 64
+// rows, all in flight together, then DPP scans): the same chain of dependent
+// loads as a task with a dispatch order, lengths -> block ids -> K.
+constexpr int kBalChunks = 8;                  // lengths a lane holds
+constexpr int kMaxBalRows = kBalChunks * kWave;  // rows of a balanced launch
+constexpr int kMaxBalPairs = 4096;             // (sequence, kv-head pass) counters
+
+// Inclusive prefix sum over the wave: row shifts within each 16 lanes, then
+// the rows' last lanes broadcast to the rows after them.
+__device__ __forceinline__ int wave_scan(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false);  // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false);  // row_shr:2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false);  // row_shr:4
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false);  // row_shr:8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1, 3
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2, 3
+  return x;
+}
+
+__device__ __forceinline__ int wave_max_int(int x) {  // of values >= 0
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false));
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false));
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false));
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false));
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false));
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false));
+  return __builtin_amdgcn_readlane(x, kWave - 1);
+}
+
+// Blocks of a row of la / lb tokens (0 when a length is past its table: such
+// a row is one part, which writes its NaN).
+template <bool TWO>
+__device__ __forceinline__ int row_blocks(const TiledParams& p, int la, int lb) {
+  if (la > p.tier[0].bt_width * p.BS || (TWO && lb > p.tier[1].bt_width * p.BS)) return 0;
+  return (max(la, 0) + kTileTokens - 1) / kTileTokens +
+         (TWO ? (max(lb, 0) + kTileTokens - 1) / kTileTokens : 0);
+}
+
+// a / d for 0 <= a < 2^22 and d > 0, rcp = 1 / d within a few ulp: the
+// product is within one of the quotient (the compiler's general division is
+// ~20 dependent instructions, and a task's start waits for several).
+__device__ __forceinline__ int small_div(int a, int d, float rcp) {
+  int q = (int)((float)a * rcp);
+  const int r = a - q * d;
+  q += r >= d ? 1 : 0;
+  q -= r < 0 ? 1 : 0;
+  return q;
+}
+__device__ __forceinline__ float fast_rcp(int d) { return __builtin_amdgcn_rcpf((float)d); }
+
+constexpr int kMaxBalBlocks = 1 << 20;  // table width of a balanced launch, in 16-token tiles
+constexpr int kBalTries = 6;            // part sizes tried
+
+template <int G, bool TWO, int kBalChunks>
+__device__ __forceinline__ bool balanced_task(const TiledParams& p, Task& t) {
+  const int lane = threadIdx.x & (kWave - 1);
+  int row[kBalChunks], la[kBalChunks], lb[kBalChunks], nb[kBalChunks], parts[kBalChunks];
+  bool skips = false;  // the caller's order lists an entry outside [0, n)
+#pragma unroll
+  for (int c = 0; c < kBalChunks; ++c) {
+    row[c] = c * kWave + lane;
+    la[c] = lb[c] = 0;
+    if (c == 0 || c * kWave < p.n) {
+      const int r = min(c * kWave + lane, p.n - 1);
+      la[c] = p.tier[0].lens[r];
+      if constexpr (TWO) lb[c] = p.tier[1].lens[r];
+      if (p.order != nullptr) skips |= (unsigned)p.order[r] >= (unsigned)p.n;
+    }
+  }
+  const int P = p.KVH * p.passes;
+  const int j = small_div(blockIdx.x, P, fast_rcp(P));  // part; kv-head passes run fastest
+  t.kp = blockIdx.x - j * P;
+  const int pass = small_div(t.kp, p.KVH, fast_rcp(p.KVH));
+  t.kh = t.kp - pass * p.KVH;
+  t.h0 = t.kh * p.hpk + pass * G;
+  t.gcount = min(G, p.hpk - pass * G);
+  // A permutation of the rows changes nothing here; an order with entries
+  // outside [0, n) leaves the rows it does not list to the caller.
+  if (__ballot(skips) != 0) {
+#pragma unroll
+    for (int c = 0; c < kBalChunks; ++c) {
+      row[c] = c * kWave + lane < p.n ? p.order[c * kWave + lane] : p.n;
+      const bool on = (unsigned)row[c] < (unsigned)p.n;
+      la[c] = on ? p.tier[0].lens[row[c]] : 0;
+      if constexpr (TWO) lb[c] = on ? p.tier[1].lens[row[c]] : 0;
+    }
+  }
+  auto listed = [&](int c) -> bool { return (unsigned)row[c] < (unsigned)p.n; };
+  int sum = 0, longest = 0;
+#pragma unroll
+  for (int c = 0; c < kBalChunks; ++c) {
+    nb[c] = parts[c] = 0;
+    if (c == 0 || c * kWave < p.n) {
+      nb[c] = listed(c) ? row_blocks<TWO>(p, la[c], lb[c]) : 0;
+      sum += nb[c];
+      longest = max(longest, nb[c]);
+    }
+  }
+  const int total = __builtin_amdgcn_readlane(wave_scan(sum), kWave - 1);
+  // First size: as many parts as wanted if rows end half a part short of a
+  // whole one on average; then larger by the share of parts too many.
+  const int want = p.bal_parts;
+  int size = (int)((float)total * __builtin_amdgcn_rcpf((float)want - 0.5f * (float)min(want, p.n)));
+  size = max(max(size, p.bal_min), (total + want - 1) / want);
+  // Whole rows where cutting saves less than the parts' merge costs: the
+  // longest row at a task's own rate against the parts, or HBM's time for all
+  // rows if that is longer.
+  if (wave_max_int(longest) <= max(size, (int)(p.bal_share * (float)total)) + p.bal_whole)
+    size = kMaxSplitBlocks;
+  size = __builtin_amdgcn_readfirstlane(min(size, kMaxSplitBlocks));
+  for (int tries = 0;; ++tries) {
+    const float rcp = fast_rcp(size);
+    int count = 0;
+#pragma unroll
+    for (int c = 0; c < kBalChunks; ++c) {
+      if (c == 0 || c * kWave < p.n) {
+        parts[c] = listed(c) ? max(1, small_div(nb[c] + size - 1, size, rcp)) : 0;
+        count += parts[c];
+      }
+    }
+    const int all = __builtin_amdgcn_readlane(wave_scan(count), kWave - 1);
+    if (all <= want || size >= kMaxSplitBlocks || tries >= kBalTries) break;
+    const float grow = (float)size * (float)(all - want) * __builtin_amdgcn_rcpf((float)want);
+    size = __builtin_amdgcn_readfirstlane(min(size + 1 + (int)(0.5f * grow), kMaxSplitBlocks));
+  }
+  int base = 0;  // parts of the rows before chunk c
+#pragma unroll
+  for (int c = 0; c < kBalChunks; ++c) {
+    if (c > 0 && c * kWave >= p.n) break;
+    const int upto = base + wave_scan(parts[c]);  // parts up to and with this lane's row
+    const int end = __builtin_amdgcn_readlane(upto, kWave - 1);
+    if (j < end) {
+      const int at = __popcll(__ballot(upto <= j));  // the lane of part j's row
+      t.i = __builtin_amdgcn_readlane(row[c], at);
+      t.la = __builtin_amdgcn_readlane(la[c], at);
+      t.lb = __builtin_amdgcn_readlane(lb[c], at);
+      t.nb = __builtin_amdgcn_readlane(nb[c], at);
+      t.nsplit = __builtin_amdgcn_readlane(parts[c], at);
+      t.slot0 = __builtin_amdgcn_readlane(upto, at) - t.nsplit;
+      t.split = j - t.slot0;
+      t.nba = t.la > 0 ? (t.la + kTileTokens - 1) / kTileTokens : 0;
+      // the row's first `more` parts hold one block more than the others
+      const int each = small_div(t.nb, t.nsplit, fast_rcp(t.nsplit));
+      const int more = t.nb - each * t.nsplit;
+      t.b_begin = t.split * each + min(t.split, more);
+      t.b_end = t.b_begin + each + (t.split < more ? 1 : 0);
+      t.range_bad = t.la > p.tier[0].bt_width * p.BS || (TWO && t.lb > p.tier[1].bt_width * p.BS);
+      return true;
+    }
+    base = end;
+  }
+  return false;
+}
+
 template <int G, bool TWO>
 __device__ __forceinline__ bool decode_task(const TiledParams& p, Task& t) {
+  if (p.bal_parts > 0)
+    return p.n <= kWave ? balanced_task<G, TWO, 1>(p, t) : balanced_task<G, TWO, kBalChunks>(p, t);
   const int task = p.xcd_group ? xcd_task(blockIdx.x, gridDim.x) : (int)blockIdx.x;
   t.kh = task % p.KVH;
   int rest = task / p.KVH;
@@ -407,6 +597,7 @@ struct WaveStates {
   float m[kWavesPerTask][G];
   float l[kWavesPerTask][G];
   int bad[kWavesPerTask];
+  int last;  // balanced cuts: this task is its row's last to arrive
 };
 
 // Folds the TPW = 64 / LPT lane-rows of a wave (each with its own softmax
@@ -446,9 +637,41 @@ __device__ __forceinline__ void publish_wave_state(WaveStates<D, G>& ws, int wav
   if (lane == 0) ws.bad[wave] = bad ? 1 : 0;
 }
 
+// Split partials of balanced cuts are written and read at agent scope (sc1:
+// past the XCD's own L2), as a row's tasks run on several XCDs.
+constexpr int kAgentScope = 16;
+typedef unsigned int part_u32x4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t part_rsrc(const float* base, int64_t elems) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), (short)0, (int)(elems * 4),
+                                           0x00020000);
+}
+
+// Writes a split task's partial of 8 dims of query head h: the normalised
+// output and, with d0 == 0, the LSE (lse2: log2 domain).
+__device__ __forceinline__ void store_partial(const TiledParams& p, const Task& t, int h, int d0,
+                                              const float* o, float lse2) {
+  if (p.bal_parts > 0) {
+    const int64_t pidx = (int64_t)(t.slot0 + t.split) * p.H + h;
+    const __amdgpu_buffer_rsrc_t ro = part_rsrc(p.part_o + pidx * p.D, p.D);
+#pragma unroll
+    for (int e = 0; e < 8; e += 4) {
+      const part_u32x4 u = {__float_as_uint(o[e]), __float_as_uint(o[e + 1]),
+                            __float_as_uint(o[e + 2]), __float_as_uint(o[e + 3])};
+      __builtin_amdgcn_raw_buffer_store_b128(u, ro, (d0 + e) * 4, 0, kAgentScope);
+    }
+    if (d0 == 0)
+      __hip_atomic_store(p.part_lse + pidx, lse2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  } else {
+    const int64_t pidx = ((int64_t)t.i * p.H + h) * p.S + t.split;
+    store8<F32>(p.part_o, pidx * p.D + d0, true, o);
+    if (d0 == 0) p.part_lse[pidx] = lse2 * kLn2;
+  }
+}
+
 // Wave 0, after the workgroup barrier: merges the waves' states with the
-// log-sum-exp rule and writes the final result (one split) or this split's
-// partial for the combine pass.
+// log-sum-exp rule and writes the final result, or this split's partial for
+// the combine pass.
 template <typename T, int D, int G>
 __device__ __forceinline__ void finish_task(const TiledParams& p, const Task& t,
                                             const WaveStates<D, G>& ws, int lane) {
@@ -494,9 +717,9 @@ __device__ __forceinline__ void finish_task(const TiledParams& p, const Task& t,
     const float inv = 1.f / lt;
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] *= inv;
-    float lse_nat = (M + fast_log2(lt)) * kLn2;
+    float lse2 = M + fast_log2(lt);
     if (bad) {
-      lse_nat = qnan();
+      lse2 = qnan();
 #pragma unroll
       for (int e = 0; e < 8; ++e) o[e] = qnan();
     }
@@ -505,14 +728,110 @@ __device__ __forceinline__ void finish_task(const TiledParams& p, const Task& t,
       if (write_final) {
         store8<T>(p.out, (int64_t)t.i * p.out_ss + (int64_t)h * p.out_sh + chunk * 8,
                   p.out_f32, o);
-        if (lane == 0) p.lse[(int64_t)h * p.lse_sh + t.i] = lse_nat;
+        if (lane == 0) p.lse[(int64_t)h * p.lse_sh + t.i] = lse2 * kLn2;
       } else {
-        const int64_t pidx = ((int64_t)t.i * p.H + h) * p.S + t.split;
-        store8<T>(p.part_o, pidx * p.D + chunk * 8, true, o);
-        if (lane == 0) p.part_lse[pidx] = lse_nat;
+        store_partial(p, t, h, chunk * 8, o, lse2);
       }
     }
   }
+}
+
+
+// Whether the tasks of this row still to come leave the merge to this one: a
+// balanced launch has no combine pass; the last of a row's parts to arrive
+// merges them. Called by the whole workgroup once its partial is written;
+// true on every thread of the last one, which also leaves the counter at zero
+// for the next launch. The partial's stores go through to memory (sc1) and
+// are waited for before the arrival is counted, and the last task reads the
+// parts with sc1 loads, so no cache is written back or invalidated (an
+// agent-scope release / acquire pair does both, and held launches up to 2x).
+__device__ __forceinline__ bool last_to_arrive(const TiledParams& p, const Task& t, int* last) {
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's partial stores are done
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    uint32_t* c = p.counters + (int64_t)t.i * p.KVH * p.passes + t.kp;
+    const uint32_t before =
+        __hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const bool done = before == (uint32_t)t.nsplit - 1;
+    if (done) __hip_atomic_store(c, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    *last = done ? 1 : 0;
+  }
+  __syncthreads();
+  return __builtin_amdgcn_readfirstlane(*last) != 0;
+}
+
+// Merges the row's parts and writes its result (the whole workgroup of the
+// row's last task): a thread takes 4 dims of a head and folds the parts in
+// order, kPartsInFlight of them read together, as each round of reads is a
+// trip past the L2. The order is fixed, whichever task arrives last.
+constexpr int kPartsInFlight = 8;
+
+template <typename T, int D>
+__device__ __forceinline__ void merge_parts(const TiledParams& p, const Task& t) {
+  constexpr int LPT = D / 4;  // threads per head
+  const int64_t first = (int64_t)t.slot0 * p.H + t.h0;
+  const __amdgpu_buffer_rsrc_t ro =
+      part_rsrc(p.part_o + first * p.D, ((int64_t)(t.nsplit - 1) * p.H + t.gcount) * p.D);
+  const __amdgpu_buffer_rsrc_t rl =
+      part_rsrc(p.part_lse + first, (int64_t)(t.nsplit - 1) * p.H + t.gcount);
+  for (int it = threadIdx.x; it < t.gcount * LPT; it += kWave * kWavesPerTask) {
+    const int g = it / LPT;
+    const int d0 = (it % LPT) * 4;
+    if (d0 >= p.D) continue;
+    float M = neg_inf(), l = 0.f, acc[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int k0 = 0; k0 < t.nsplit; k0 += kPartsInFlight) {
+      float lv[kPartsInFlight];
+      part_u32x4 x[kPartsInFlight];
+#pragma unroll
+      for (int u = 0; u < kPartsInFlight; ++u) {
+        // a part past the last reads the last one again, weightless
+        const uint32_t pi = (uint32_t)(min(k0 + u, t.nsplit - 1) * p.H + g);
+        lv[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rl, pi * 4, 0, kAgentScope));
+        x[u] = __builtin_amdgcn_raw_buffer_load_b128(
+            ro, (pi * (uint32_t)p.D + (uint32_t)d0) * 4, 0, kAgentScope);
+      }
+      float mn = M;
+#pragma unroll
+      for (int u = 0; u < kPartsInFlight; ++u) {
+        lv[u] = k0 + u < t.nsplit ? lv[u] : neg_inf();
+        mn = fmaxf(mn, lv[u]);
+      }
+      const float ms = mn == neg_inf() ? 0.f : mn;
+      const float alpha = fast_exp2(M - ms);
+      l *= alpha;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[e] *= alpha;
+#pragma unroll
+      for (int u = 0; u < kPartsInFlight; ++u) {
+        const float w = fast_exp2(lv[u] - ms);
+        l += w;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          // a part of weight 0 (read again, or all its scores -inf) may hold NaN
+          const float o = w == 0.f ? 0.f : __uint_as_float(x[u][e]);
+          acc[e] = __builtin_fmaf(w, o, acc[e]);
+        }
+      }
+      M = mn;
+    }
+    const float inv = 1.f / l;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] *= inv;
+    const int h = t.h0 + g;
+    store4<T>(p.out, (int64_t)t.i * p.out_ss + (int64_t)h * p.out_sh + d0, p.out_f32, acc);
+    if (d0 == 0) p.lse[(int64_t)h * p.lse_sh + t.i] = (M + fast_log2(l)) * kLn2;
+  }
+}
+
+// The end of a task of the kernels whose waves publish WaveStates: the waves
+// merge, and in a balanced launch a row's last task merges its parts.
+template <typename T, int D, int G>
+__device__ __forceinline__ void end_task(const TiledParams& p, const Task& t, WaveStates<D, G>& ws,
+                                         int wave, int lane) {
+  __syncthreads();
+  if (wave == 0) finish_task<T, D, G>(p, t, ws, lane);
+  if (p.bal_parts == 0 || t.nsplit == 1) return;
+  if (last_to_arrive(p, t, &ws.last)) merge_parts<T, D>(p, t);
 }
 
 // Query head of the task's head slot g: slots past the task's heads repeat

@@ -212,12 +212,10 @@ __global__ __launch_bounds__(kWave * kWavesPerTask) void decode_tiled_kernel(Til
 
   // ---- merge the TPW lane-rows of each head into this wave's state, publish it
   publish_wave_state<D, G>(ws, wave, lane, m, l, acc, wb.bad);
-  __syncthreads();
-  if (wave != 0) return;
-  finish_task<T, D, G>(p, t, ws, lane);
-  stamp(kTlEnd);
+  end_task<T, D, G>(p, t, ws, wave, lane);
+  if (wave == 0) stamp(kTlEnd);
   if constexpr (TL) {
-    if (lane == 0)
+    if (wave == 0 && lane == 0)
       p.timeline[(int64_t)blockIdx.x * kTimelineSlots + kTlInfo] =
           (uint64_t)(t.b_end - t.b_begin) | ((uint64_t)wb.stride << 16) |
           ((uint64_t)(uint32_t)t.i << 32);

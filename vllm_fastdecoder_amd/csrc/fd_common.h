@@ -248,6 +248,8 @@ struct DecodeArgs {
   int64_t lse_sh;
   void* workspace;
   size_t workspace_bytes;
+  uint32_t* counters;  // balanced launches' arrival counters, all zero (NULL: taken from the
+                       // workspace and cleared by a launch of their own)
   // measurement only (fd_paged_decode_timeline): per-workgroup time stamps
   // of a VALU-kernel launch, kTimelineSlots words per workgroup; NULL in
   // every other call
@@ -270,6 +272,12 @@ struct SplitPlan {
                          // kernel_g), each over the same blocks
   int32_t wave_blocks;   // blocks per working wave of a task (0: every wave works)
   bool no_kv_adj;        // separate K and V loads even where V follows K (FD_KV_ADJ=0)
+  int32_t bal_parts;     // > 0: balanced cuts (decode_tiled.h): parts per kv-head pass aimed at,
+  int32_t bal_min;       // 16-token tiles per part at least,
+  int32_t bal_grid;      // the parts the grid holds per kv-head pass,
+  int32_t bal_cap;       // its wg_cap,
+  int32_t bal_whole;     // and balanced_task's figures for leaving rows whole
+  float bal_share;
   int* occupancy_query;  // planner only: when set, the tiled launchers store the selected
                          // kernel's workgroups per CU there instead of launching it
 };
@@ -283,6 +291,10 @@ SplitPlan plan_decode(int32_t n, int32_t H, int32_t KVH, int32_t D, int32_t BS,
                       double fill = 0.0);
 size_t decode_workspace_bytes(const SplitPlan& sp, int32_t n, int32_t H,
                               int32_t D);
+// Workspace of a plan's balanced launch (0 when it has none): the partials,
+// and the arrival counters behind them when the caller brings none.
+size_t balanced_partial_bytes(const SplitPlan& sp, int32_t H, int32_t D);
+size_t balanced_counter_bytes(const SplitPlan& sp, int32_t n, int32_t KVH);
 // Workspace a plan of these sizes may need whatever the rows' token total
 // (the slot fill, half rows), 0 when neither can apply to it.
 size_t fill_workspace_bound(const SplitPlan& sp, int32_t n, int32_t H, int32_t KVH, int32_t D,

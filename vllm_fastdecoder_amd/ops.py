@@ -121,7 +121,7 @@ class _Workspace:
             buf = self._bufs.pop(key, None)  # re-inserted below: most recent last
             if buf is None or buf.numel() < nbytes:
                 cap = max(nbytes, 2 * (buf.numel() if buf is not None else 0), 16)
-                buf = torch.empty(cap, dtype=torch.uint8, device=torch.device("cuda", key[0]))
+                buf = self._allocate(key, cap)
                 if key in self._pinned:
                     self._pinned[key].append(buf)
             if pin and key not in self._pinned:
@@ -134,11 +134,39 @@ class _Workspace:
                 del self._bufs[victim]
             return buf
 
+    @staticmethod
+    def _allocate(key: tuple[int, int], nbytes: int) -> torch.Tensor:
+        """nbytes of scratch followed, on the next 256-byte boundary, by the
+        stream's arrival counters (fd_paged_decode_counted), cleared on the
+        stream that will use them."""
+        device, stream = key
+        head = _counters_offset(nbytes)
+        size = head + 4 * _lib.DECODE_COUNTERS
+
+        def make():
+            t = torch.empty(size, dtype=torch.uint8, device=torch.device("cuda", device))
+            t[head:].zero_()
+            return t[:nbytes]
+
+        if _current_stream(device) == stream:
+            return make()
+        with torch.cuda.stream(torch.cuda.ExternalStream(stream, device=device)):
+            return make()
+
     def release(self, device: torch.device, stream: int) -> None:
         """Ends a pin: the stream's replaced buffers go, its current one stays
         (and may be evicted again)."""
         with self._lock:
             self._pinned.pop(self._key(device, stream), None)
+
+
+def _counters_offset(nbytes: int) -> int:
+    return (nbytes + 255) // 256 * 256
+
+
+def _counters_ptr(buf: torch.Tensor | None) -> int | None:
+    """The arrival counters behind a buffer of WORKSPACE."""
+    return None if buf is None else buf.data_ptr() + _counters_offset(buf.numel())
 
 
 WORKSPACE = _Workspace()
@@ -189,6 +217,18 @@ def decode_plan_info(n: int, H: int, KVH: int, D: int, BS: int, width: int, dtyp
             "wave_blocks": plan.wave_blocks}
 
 
+def balanced_parts(n: int, H: int, KVH: int, D: int, BS: int, width: int, dtype: torch.dtype,
+                   host_tier: bool = False) -> int:
+    """Tasks per kv head and head-group pass that a decode launch of these
+    sizes aims at when it cuts the rows by their lengths on the device
+    (fd_decode_balanced_parts); 0: the cut by table width that
+    decode_plan_info describes."""
+    parts = ctypes.c_int32()
+    _lib.check(_lib.load_lib().fd_decode_balanced_parts(n, H, KVH, D, BS, width, _DT[dtype],
+                                                        int(host_tier), ctypes.byref(parts)))
+    return parts.value
+
+
 _GET_DEVICE = getattr(torch._C, "_cuda_getDevice", None)
 
 
@@ -200,14 +240,30 @@ def _current_device() -> int:
     return torch.cuda.current_device() if torch.cuda.is_available() else -1
 
 
+_ENV_NAMES = ("FD_SPLIT_BLOCKS", "FD_DECODE_KERNEL", "FD_BALANCE")
+# os.environ encodes the name on every lookup (~0.6 us each, on every decode
+# call); on POSIX its own dict is keyed by the encoded names
+_ENV_DATA = getattr(os.environ, "_data", None)
+if not isinstance(_ENV_DATA, dict) or not all(isinstance(k, bytes) for k in _ENV_DATA):
+    _ENV_DATA = None
+_ENV_KEYS = tuple(name.encode() for name in _ENV_NAMES)
+
+
+def _planner_env() -> tuple:
+    """The planner overrides a workspace's size depends on."""
+    if _ENV_DATA is None:
+        return tuple(os.environ.get(k) for k in _ENV_NAMES)
+    get = _ENV_DATA.get
+    a, b, c = _ENV_KEYS
+    return get(a), get(b), get(c)
+
+
 def workspace_bytes(n: int, H: int, KVH: int, D: int, BS: int, width: int) -> int:
     """Workspace a decode call of this shape needs on the current device
     (remembered per shape, device and the planner overrides it depends on:
-    FD_SPLIT_BLOCKS, and FD_DECODE_KERNEL, which can allow more splits; the
-    device's CU count sets the split bounds)."""
-    env = os.environ
-    key = (n, H, KVH, D, BS, width, env.get("FD_SPLIT_BLOCKS"), env.get("FD_DECODE_KERNEL"),
-           _current_device())
+    FD_SPLIT_BLOCKS, FD_BALANCE, and FD_DECODE_KERNEL, which can allow more
+    splits; the device's CU count sets the split bounds)."""
+    key = (n, H, KVH, D, BS, width, _planner_env(), _current_device())
     size = _WS_SIZES.get(key)
     if size is None:
         c = ctypes.c_size_t()
@@ -272,8 +328,10 @@ def paged_decode_partial(
     _require(W == 0 or bt.stride(1) == 1, "block_table rows must be contiguous")
     ln = ln.contiguous()
     need = workspace_bytes(n, H, num_kv_heads, D, block_size, W)
+    counters = None  # a caller's own workspace has none
     if workspace is None:
         workspace = WORKSPACE.get(dev, need)
+        counters = _counters_ptr(workspace)
     ws_ptr = workspace.data_ptr() if workspace is not None else None
     ws_len = workspace.numel() * workspace.element_size() if workspace is not None else 0
     order_ptr = None
@@ -303,10 +361,8 @@ def paged_decode_partial(
                  and timeline.shape[1] == 8 and timeline.is_contiguous(),
                  "timeline must be a contiguous int64 [workgroups, 8] GPU tensor")
         _lib.check(lib.fd_paged_decode_timeline(*args, timeline.data_ptr(), timeline.shape[0]))
-    elif total_tokens is None:
-        _lib.check(lib.fd_paged_decode_partial(*args))
     else:
-        _lib.check(lib.fd_paged_decode_partial_hint(*args, int(total_tokens)))
+        _lib.check(lib.fd_paged_decode_counted(*args, int(total_tokens or 0), counters))
 
 
 def _tier(k_cache, v_cache, strides, num_blocks, block_table, lens, n, dev, what):
@@ -397,14 +453,14 @@ def split_decode(
         order_ptr = row_order.data_ptr()
     lib = _lib.load_lib()
     _lib.check(
-        lib.fd_split_decode(
+        lib.fd_split_decode_counted(
             q.data_ptr(), q.stride(0), q.stride(1),
             ctypes.byref(hbm), ctypes.byref(host), order_ptr,
             n, H, KVH, D, BS, float(softmax_scale), kv_dt,
             out.data_ptr(), out.stride(0), out.stride(1), _DT[out.dtype],
             lse.data_ptr(), lse.stride(0),
             ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0,
-            _stream_for(q),
+            _stream_for(q), _counters_ptr(ws),
         )
     )
     del keep_a, keep_b  # the launch is enqueued; later reuse is stream-ordered
