@@ -94,7 +94,7 @@ __global__ __launch_bounds__(kWave * kWavesPerTask) void decode_f32_kernel(Tiled
   constexpr int POL = KEEP ? kKvLoadKeep : kKvLoadPolicy;
   Vec8 kb[2][STEPS][2], vb[2][STEPS][2];
   auto load_half = [&](int slot, int u) {
-    const BlockSrc src = block_src<TWO>(p, wb, t.kh, u >> 1);
+    const BlockSrc src = block_src<TWO>(p, wb, t, u >> 1);
     const uint32_t off = src.t1 ? off1 : off0;
     const uint32_t step = src.t1 ? step1 : step0;
     const uint32_t base = (u & 1) ? (src.t1 ? half1 : half0) : 0u;

@@ -142,7 +142,7 @@ __global__ __launch_bounds__(kWave * kWavesPerTask) void decode_mfma_kernel(Tile
   // right after block k's scores and land while block k's softmax and P.V run.
   Vec8 kb[KS], vb[2][TPL][CPL];
   auto load_block = [&](int slot, int k) {
-    const BlockSrc src = block_src<TWO>(p, wb, t.kh, k);
+    const BlockSrc src = block_src<TWO>(p, wb, t, k);
     const uint32_t koff = src.t1 ? koff1 : koff0;
     const uint32_t voff = src.t1 ? voff1 : voff0;
     const uint32_t vtok = src.t1 ? vtok1 : vtok0;

@@ -208,7 +208,7 @@ __global__ __launch_bounds__(kWave * kWavesPerTask) void decode_mm_kernel(TiledP
   // shapes: HBM is already busy and the extra requests only queue.)
   Vec8 kb[2][KS], vb[2][NLD];
   auto load_block = [&](int slot, int k) {
-    const BlockSrc src = block_src<TWO>(p, wb, t.kh, k);
+    const BlockSrc src = block_src<TWO>(p, wb, t, k);
     const uint32_t koff = src.t1 ? koff1 : koff0;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) kb[slot][ks] = buffer_ld16<POL>(src.k, koff, 64 * ks);

@@ -565,11 +565,34 @@ __device__ __forceinline__ WaveBlocks wave_blocks(const TiledParams& p, const Ta
   w.first = t.b_begin + wave;
   w.nw = wave < ws && w.first < t.b_end ? (t.b_end - w.first + ws - 1) / ws : 0;
   w.k1 = TWO ? (t.nba > w.first ? (t.nba - w.first + ws - 1) / ws : 0) : w.nw;
+  if constexpr (TWO) {
+    // A range with blocks of both tiers: the last `h` waves take tier 1's
+    // (one to three waves, by its share of the blocks), the others tier 0's:
+    // a wave that waits for the link holds up no HBM blocks, and the link is
+    // busy from the start. Measured with the shorter host reads of block_src
+    // (HIP graph replay, us; HBM and link time of the bytes in brackets):
+    // 33 rows of U[40, 1800], 32/8, one host block each [15 + 21] 53 -> 45;
+    // 24 x 32 heads of U[256, 1024], 7.5 % host [35 + 303] 362 -> 316; 8 x 32,
+    // 10 % [10 + 119] 146 -> 132; 60 % host [15 + 2787] 2783 -> 2761.
+    const int na = min(t.nba, t.b_end) - t.b_begin;
+    const int nh = t.b_end - t.b_begin - na;
+    const int h = min(kWavesPerTask - 1, max(1, (4 * nh + (na + nh) / 2) / max(na + nh, 1)));
+    const int wa = kWavesPerTask - h;
+    if (na > 0 && nh > 0 && ws == kWavesPerTask && na <= wa * kMaxWaveBlocks &&
+        nh <= h * kMaxWaveBlocks) {
+      const bool host = wave >= wa;
+      w.stride = host ? h : wa;
+      w.first = host ? t.b_begin + na + wave - wa : t.b_begin + wave;
+      const int end = host ? t.b_end : t.b_begin + na;
+      w.nw = w.first < end ? (end - w.first + w.stride - 1) / w.stride : 0;
+      w.k1 = host ? 0 : w.nw;
+    }
+  }
   int bid = 0, sub = 0;
   bool my_bad = false;
   if (lane < w.nw) {
     // tile u of the row: tile u % tpb of the row's cache block u / tpb
-    const int u = w.first + ws * lane;
+    const int u = w.first + w.stride * lane;
     if (TWO && u >= t.nba) {
       const TierParams& tp = p.tier[1];
       const int ut = u - t.nba;
@@ -849,20 +872,29 @@ struct BlockSrc {
   bool t1;
 };
 
+// A tier-1 block's resources end with its last valid token (a tier's last
+// block may be partial): rows past it read as zero and cost no traffic, which
+// counts over the link, where a row's newest block is often all it has (33
+// rows with one host block each, 2.2 -> 1.2 MB over the link). In HBM the
+// extra scalar work per block costs more than the bytes (full batch of 256
+// grouped-query rows: 387 -> 401 us), so tier 0 keeps whole blocks.
 template <bool TWO>
-__device__ __forceinline__ BlockSrc block_src(const TiledParams& p, const WaveBlocks& wb, int kh,
-                                              int k) {
+__device__ __forceinline__ BlockSrc block_src(const TiledParams& p, const WaveBlocks& wb,
+                                              const Task& t, int k) {
   const bool t1 = TWO && k >= wb.k1;
   const int bid = __builtin_amdgcn_readlane(wb.my_bid, k);
   const int sub = __builtin_amdgcn_readlane(wb.my_sub, k);
   const TierParams& a = p.tier[0];
   const TierParams& b = p.tier[TWO ? 1 : 0];
-  const int64_t base = (int64_t)bid * (t1 ? b.sb : a.sb) + (int64_t)kh * (t1 ? b.sh : a.sh) +
+  const int64_t base = (int64_t)bid * (t1 ? b.sb : a.sb) + (int64_t)t.kh * (t1 ? b.sh : a.sh) +
                        (int64_t)sub * kTileTokens * (t1 ? b.st : a.st);
-  const uint32_t rb = t1 ? b.run_bytes : a.run_bytes;
+  uint32_t cut = 0;  // bytes of the block's rows past its tokens
+  if (t1)
+    cut = (uint32_t)(kTileTokens - block_tokens<TWO>(t, wb.first + wb.stride * k)) *
+          (uint32_t)b.st * 2;
   BlockSrc s;
-  s.k = make_rsrc((t1 ? b.k : a.k) + base, t1 ? b.k_run_bytes : a.k_run_bytes);
-  s.v = make_rsrc((t1 ? b.v : a.v) + base, rb);
+  s.k = make_rsrc((t1 ? b.k : a.k) + base, (t1 ? b.k_run_bytes : a.k_run_bytes) - cut);
+  s.v = make_rsrc((t1 ? b.v : a.v) + base, (t1 ? b.run_bytes : a.run_bytes) - cut);
   s.kp = reinterpret_cast<const char*>((t1 ? b.k : a.k) + base);
   s.t1 = t1;
   return s;

@@ -112,7 +112,7 @@ __global__ __launch_bounds__(kWave * kWavesPerTask) void decode_tiled_kernel(Til
 
   Vec8 kb[2][STEPS], vb[2][STEPS];
   auto load_block = [&](int slot, int k) {
-    const BlockSrc src = block_src<TWO>(p, wb, t.kh, k);
+    const BlockSrc src = block_src<TWO>(p, wb, t, k);
     if (adj_block(k)) {
       // global rather than buffer loads here: ~1 % faster for K + V runs
       // (and ~0.3 % slower for separate K and V rows), measured on MI355X;
