@@ -233,6 +233,16 @@ int fd_paged_decode_workspace_size(
     int32_t n, int32_t num_heads, int32_t num_kv_heads, int32_t head_size,
     int32_t block_size, int32_t bt_width, size_t* bytes);
 
+/* Bytes of workspace one fd_paged_decode_counted / fd_split_decode_counted
+ * call with these sizes needs: the exact figure for one kv dtype and token
+ * total, where fd_paged_decode_workspace_size covers them all. host_tier: 1 if
+ * a tier lies in pinned host memory (a two-tier call asks for both and takes
+ * the larger). No counterpart in the reference. */
+int fd_decode_workspace_need(int32_t n, int32_t num_heads, int32_t num_kv_heads,
+                             int32_t head_size, int32_t block_size, int32_t bt_width,
+                             int32_t kv_dtype, int32_t host_tier, int64_t total_tokens,
+                             size_t* bytes);
+
 /* Which kernel a decode launch of these sizes takes, and how it is cut into
  * tasks (the planner of fd_paged_decode_partial / fd_split_decode, on the
  * current device). No counterpart in the reference; for tests and for

@@ -136,6 +136,12 @@ SIGNATURES: dict[str, tuple] = {
         c_int,
         [c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, POINTER(c_size_t)],
     ),
+    "fd_decode_workspace_need": (
+        c_int,
+        [c_int32, c_int32, c_int32, c_int32, c_int32, c_int32,  # n, H, KVH, D, BS, bt_width
+         c_int32, c_int32, c_int64,                             # kv_dtype, host_tier, total_tokens
+         POINTER(c_size_t)],
+    ),
     "fd_decode_plan_info": (
         c_int,
         [c_int32, c_int32, c_int32, c_int32, c_int32, c_int32,  # n, H, KVH, D, BS, bt_width

@@ -45,6 +45,25 @@ SOURCE_FLAGS = {
 CXX_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-pthread", "-Wall", "-Wno-unused-function"]
 
 
+# The torch-facing call path (csrc/torch/torch_call.cpp), a Python module of
+# its own beside the library it links to: the library itself knows no torch.
+TORCH_CALL_SRC = CSRC / "torch" / "torch_call.cpp"
+TORCH_CALL_PATH = PKG_DIR / "_torch_call.so"
+
+
+def torch_call_command(out: Path, lib: Path) -> list[str]:
+    import sysconfig
+
+    from torch.utils import cpp_extension
+
+    libs = cpp_extension.library_paths()[0]
+    return [cxx(), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D_GLIBCXX_USE_CXX11_ABI=1",
+            *(f"-isystem{p}" for p in cpp_extension.include_paths()),
+            f"-isystem{sysconfig.get_paths()['include']}", str(TORCH_CALL_SRC), "-o", str(out),
+            str(lib), f"-L{libs}", "-Wl,-rpath,$ORIGIN", f"-Wl,-rpath,{libs}",
+            "-lc10", "-ltorch", "-ltorch_cpu", "-ltorch_python"]
+
+
 def sources() -> list[Path]:
     return sorted(CSRC.glob("*.hip"))
 
@@ -96,8 +115,12 @@ def build(verbose: bool = False, out: Path | None = None) -> Path:
             for f in [pool.submit(_run, c, verbose) for c in cmds]:
                 f.result()
         _run([hipcc(), f"--offload-arch={ARCH}", "-fPIC", "-shared", "-pthread",
-              *map(str, objs + hobjs), "-o", str(tmp)], verbose)
+              f"-Wl,-soname,{LIB_NAME}", *map(str, objs + hobjs), "-o", str(tmp)], verbose)
     os.replace(tmp, out)
+    if out == LIB_PATH:
+        tmp = TORCH_CALL_PATH.with_suffix(".so.tmp")
+        _run(torch_call_command(tmp, out), verbose)
+        os.replace(tmp, TORCH_CALL_PATH)
     return out
 
 

@@ -220,6 +220,23 @@ int fd_paged_decode_workspace_size(int32_t n, int32_t num_heads, int32_t num_kv_
   return FD_OK;
 }
 
+int fd_decode_workspace_need(int32_t n, int32_t num_heads, int32_t num_kv_heads,
+                             int32_t head_size, int32_t block_size, int32_t bt_width,
+                             int32_t kv_dtype, int32_t host_tier, int64_t total_tokens,
+                             size_t* bytes) {
+  if (bytes == nullptr) return set_error(FD_ERR_INVALID, "workspace_need: bytes is NULL");
+  if (n < 0 || num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads != 0 ||
+      head_size <= 0 || block_size <= 0 || bt_width < 0 || total_tokens < 0 ||
+      !valid_dtype(kv_dtype))
+    return set_error(FD_ERR_INVALID, "workspace_need: bad sizes");
+  const SplitPlan sp = plan_decode(n, num_heads, num_kv_heads, head_size, block_size, bt_width,
+                                   kv_dtype, true, host_tier == 0,
+                                   row_fill(total_tokens, n, bt_width, block_size));
+  *bytes = sp.bal_parts > 0 ? balanced_partial_bytes(sp, num_heads, head_size)
+                            : decode_workspace_bytes(sp, n, num_heads, head_size);
+  return FD_OK;
+}
+
 int fd_decode_plan_info(int32_t n, int32_t num_heads, int32_t num_kv_heads, int32_t head_size,
                         int32_t block_size, int32_t bt_width, int32_t kv_dtype, int32_t aligned,
                         int32_t host_tier, int64_t total_tokens, FdDecodePlan* plan) {

@@ -16,6 +16,7 @@ caches must be pinned (see pinned.py); the kernels read them in place.
 from __future__ import annotations
 
 import ctypes
+import logging
 import os
 import threading
 
@@ -170,6 +171,36 @@ def _counters_ptr(buf: torch.Tensor | None) -> int | None:
 
 
 WORKSPACE = _Workspace()
+
+
+_NATIVE = None  # the native call module; False once it could not be loaded
+
+
+def _native():
+    """The native call path (csrc/torch/torch_call.cpp): ordinary calls go
+    from the tensors straight to the C ABI. False where the module cannot be
+    loaded (built for another torch): every call then takes the checks below
+    and ctypes, with the same kernels and results."""
+    global _NATIVE
+    if _NATIVE is None:
+        _lib.load_lib()  # a missing or stale library fails here
+        try:
+            from . import _torch_call
+
+            _torch_call.init(WORKSPACE.get, device_ptr, torch._C._cuda_getCurrentRawStream)
+            _NATIVE = _torch_call
+        except (ImportError, AttributeError) as e:
+            logging.getLogger("fastdecode").warning(
+                "FastDecode: native call path unavailable (%s); calls go through ctypes", e)
+            _NATIVE = False
+    return _NATIVE
+
+
+def _native_result(got):
+    """(out, lse) of a native call; its FdError where the library refused."""
+    if len(got) == 1:
+        _lib.check(got[0])
+    return got
 
 
 def reserve_workspace(stream: torch.cuda.Stream, nbytes: int) -> torch.Tensor:
@@ -1037,6 +1068,15 @@ def paged_decode(
 
     timeline: measurement only (see paged_decode_partial).
     """
+    # One native call where nothing is unusual. Host time per call, measured on
+    # one box: 13-15 -> 5-8 us; a decode of one row of 900 tokens, eager calls
+    # back to back: 14.7 -> 7.7 us (its GPU time is 7.6).
+    native = _NATIVE or _native()
+    if native and timeline is None:
+        got = native.paged_decode(q, key_cache, value_cache, block_table, seqused_k,
+                                  softmax_scale, out, lse, row_order, max_seqlen_k, total_tokens)
+        if got is not None:
+            return _native_result(got)
     _require(key_cache.dim() == 4 and value_cache.shape == key_cache.shape,
              "key_cache/value_cache must be [B, BS, KVH, D]")
     B, BS, KVH, D = key_cache.shape
@@ -1146,6 +1186,12 @@ def reshape_and_cache(key, value, key_cache, value_cache, slot_mapping,
     (e.g. plan_tiers' error count); nothing is written when it is non-zero."""
     _require(kv_cache_dtype in ("auto", "float16", "bfloat16", "fp16", "bf16"),
              f"quantized KV cache ({kv_cache_dtype}) is not supported")
+    native = _NATIVE or _native()
+    if native:
+        status = native.cache_write(key, value, key_cache, value_cache, slot_mapping, error_count,
+                                    write_gate)
+        if status is not None:
+            return _lib.check(status)
     _require(key_cache.dim() == 4 and value_cache.shape == key_cache.shape
              and key_cache.stride() == value_cache.stride(), "caches must be [B, BS, KVH, D]")
     B, BS, KVH, D = key_cache.shape
