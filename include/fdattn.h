@@ -486,6 +486,26 @@ int fd_reshape_and_cache(
     int32_t dtype, int32_t* error_count, const int32_t* write_gate,
     void* stream);
 
+/* The same rows written into both tiers' caches in one launch, each by its
+ * own slot mapping (fd_plan_tiers' gpu_slot_mapping / host_slot_mapping: a
+ * token has a slot >= 0 in one of them). Slots past a cache are not written.
+ * No counterpart in the reference, which writes each tier by its own call. */
+typedef struct fd_cache_target {
+  void* k_cache;
+  void* v_cache;
+  int64_t stride_block, stride_token, stride_head; /* elements */
+  int64_t num_blocks;
+  const int64_t* slot_mapping; /* int64 [num_tokens], device-readable */
+} fd_cache_target;
+
+int fd_reshape_and_cache_tiers(
+    const void* key, int64_t key_stride_tok, int64_t key_stride_head,
+    const void* value, int64_t value_stride_tok, int64_t value_stride_head,
+    const fd_cache_target* hbm, const fd_cache_target* host,
+    int32_t num_tokens, int32_t num_kv_heads, int32_t head_size,
+    int32_t block_size, int32_t dtype, const int32_t* write_gate,
+    void* stream);
+
 /* Host-side range check of host-resident slots before a write, the rule of
  * cpu_attn.cpp:506-510: every slot must lie in [0, capacity). Returns FD_OK,
  * or FD_ERR_RANGE with *first_bad (if not NULL) set to the first offending

@@ -57,6 +57,21 @@ class FdKvTier(ctypes.Structure):
     ]
 
 
+class FdCacheTarget(ctypes.Structure):
+    """struct fd_cache_target of include/fdattn.h: one cache of
+    fd_reshape_and_cache_tiers."""
+
+    _fields_ = [
+        ("k_cache", c_void_p),
+        ("v_cache", c_void_p),
+        ("stride_block", c_int64),
+        ("stride_token", c_int64),
+        ("stride_head", c_int64),
+        ("num_blocks", c_int64),
+        ("slot_mapping", c_void_p),
+    ]
+
+
 # name -> (restype, argtypes); the order follows include/fdattn.h
 SIGNATURES: dict[str, tuple] = {
     "fd_last_error": (c_char_p, []),
@@ -224,6 +239,13 @@ SIGNATURES: dict[str, tuple] = {
             c_int32, c_int32, c_int32,             # n, H, D
             c_void_p,                              # stream
         ],
+    ),
+    "fd_reshape_and_cache_tiers": (
+        c_int,
+        [c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64,  # key, value, strides
+         POINTER(FdCacheTarget), POINTER(FdCacheTarget),          # hbm, host
+         c_int32, c_int32, c_int32, c_int32,                      # T, KVH, D, block_size
+         c_int32, c_void_p, c_void_p],                            # dtype, write_gate, stream
     ),
     "fd_reshape_and_cache": (
         c_int,

@@ -132,6 +132,29 @@ def _write_hbm_tier(key, value, key_cache, value_cache, slots, kv_cache_dtype, l
                               getattr(layer, "_k_scale", None), getattr(layer, "_v_scale", None))
 
 
+def _write_tiers(key, value, key_cache, value_cache, ds, kv_cache_dtype, layer, k_host, v_host):
+    """A step's KV rows into both tiers, nothing when the planner counted an
+    error: one launch with this library's op and an unquantised cache, else
+    the seam's HBM write and this library's host write."""
+    if (OPS.reshape_and_cache is HipOps.reshape_and_cache
+            and kv_cache_dtype in ("auto", "float16", "bfloat16", "fp16", "bf16")):
+        ops.reshape_and_cache_tiers(key, value, key_cache, value_cache, ds.gpu_slots, k_host,
+                                    v_host, ds.host_slots, write_gate=ds.errors)
+        return
+    _write_hbm_tier(key, value, key_cache, value_cache, ds.gpu_slots, kv_cache_dtype, layer,
+                    write_gate=ds.errors)
+    ops.reshape_and_cache(key, value, k_host.transpose(1, 2), v_host.transpose(1, 2),
+                          ds.host_slots, write_gate=ds.errors)
+
+
+def _rows_in_place(t: torch.Tensor, n: int) -> bool:
+    """Whether the fast kernels take the first n rows of t [T, H, D] as they
+    lie (contiguous in D, 16-byte aligned rows)."""
+    st, sh, sd = t.stride()
+    return (t.shape[0] >= n and sd == 1 and st % 8 == 0 and sh % 8 == 0
+            and t.data_ptr() % 16 == 0)
+
+
 # The planner's capacity error (plan.py:133-137), raised by the host planner
 # (plan.build_host_plan) and, for steps planned on the GPU, by
 # raise_step_errors one step later.
@@ -253,6 +276,29 @@ class DeviceStep:
     # the decode rows' host-tier view, fetched once per step for the hybrid
     # split (host_tables)
     _host: tuple | None = field(default=None, repr=False)
+    # (gpu_bt, gpu_lens, cpu_bt, cpu_lens) of the decode rows where they are
+    # not the step's rows as they lie: gathered with the plan, on its stream
+    dec: tuple | None = field(default=None, repr=False)
+
+    @property
+    def all_decode(self) -> bool:
+        """Every row is a decode row: token t is row t's, and the decode rows'
+        tables are the step's."""
+        return self.n_dec == self.gpu_bt.shape[0] == self.gpu_slots.shape[0]
+
+    def dec_tables(self) -> tuple[torch.Tensor, ...]:
+        """(gpu_bt, gpu_lens, cpu_bt, cpu_lens) of the decode rows, the same
+        for every layer of the step (four gathers a layer took 12 us of GPU
+        time and 20 us of host time)."""
+        if self.all_decode:
+            return self.gpu_bt, self.gpu_lens, self.cpu_bt, self.cpu_lens
+        if self.dec is not None:
+            return self.dec
+        return self._gather()
+
+    def _gather(self) -> tuple[torch.Tensor, ...]:
+        return tuple(t.index_select(0, self.dec_rows) for t in
+                     (self.gpu_bt, self.gpu_lens, self.cpu_bt, self.cpu_lens))
 
     def check_errors(self, wait: bool = True) -> None:
         """Raises the planner's RuntimeError if this step's tier planner found
@@ -326,7 +372,7 @@ def build_device_step(query_start_loc_cpu: torch.Tensor, seq_lens_cpu: torch.Ten
         if fre.numel() else torch.zeros(0, dtype=torch.int64)
     f_cu = torch.zeros(fre.numel() + 1, dtype=torch.int32)
     f_cu[1:] = torch.cumsum(f_q, 0).to(torch.int32)
-    return DeviceStep(
+    step = DeviceStep(
         gpu_bt=gpu_bt, cpu_bt=cpu_bt, gpu_lens=gpu_lens, cpu_lens=cpu_lens,
         gpu_slots=gpu_slots, host_slots=host_slots,
         dec_rows=d(dec), dec_tok=d(qsl[dec]), dec_order=d(longest_first(seq[dec])),
@@ -334,6 +380,9 @@ def build_device_step(query_start_loc_cpu: torch.Tensor, seq_lens_cpu: torch.Ten
         f_max=int(f_q.max()) if f_q.numel() else 0, n_f_tok=int(f_tok.numel()), errors=errors,
         errors_host=errors_host, errors_ready=errors_ready,
     )
+    if step.n_dec and not step.all_decode:
+        step.dec = step._gather()
+    return step
 
 
 @dataclass
@@ -512,20 +561,19 @@ class SplitDecodeImpl:
         #    nothing is written when the planner counted an error (every slot
         #    is checked before any write, cpu_attn.cpp:506-510)
         if self.kv_sharing_target_layer_name is None:
-            _write_hbm_tier(key, value, key_cache, value_cache, ds.gpu_slots,
-                            self.kv_cache_dtype, layer, write_gate=ds.errors)
-            ops.reshape_and_cache(key, value, k_host.transpose(1, 2), v_host.transpose(1, 2),
-                                  ds.host_slots, write_gate=ds.errors)
+            _write_tiers(key, value, key_cache, value_cache, ds, self.kv_cache_dtype, layer,
+                         k_host, v_host)
 
         # 2) decode rows: both tiers in one launch (a row without host tokens
         #    is plain paged attention over its HBM blocks), or, with
         #    device_step_hybrid, the hybrid split of that launch
         hybrid = None
         if ds.n_dec:
-            q = query.index_select(0, ds.dec_tok)
-            gbt = ds.gpu_bt.index_select(0, ds.dec_rows)
-            gl = ds.gpu_lens.index_select(0, ds.dec_rows)
-            cbt = ds.cpu_bt.index_select(0, ds.dec_rows)
+            # rows that lie in token order are read, and written, in place
+            in_order = ds.all_decode
+            q = (query[:ds.n_dec] if in_order and _rows_in_place(query, ds.n_dec)
+                 else query.index_select(0, ds.dec_tok))
+            gbt, gl, cbt, cl = ds.dec_tables()
             share = self._host_share() if self.device_step_hybrid else 0.0
             # the rows' whole context bounds their host-tier bytes: below the
             # threshold the tables are not even fetched (no host wait)
@@ -539,10 +587,18 @@ class SplitDecodeImpl:
                                                     v_host, cbt_h, cl_h, float(self.scale), share,
                                                     hbm_lens_dev=gl, host_block_table_dev=cbt)
             if hybrid is None:
-                out, _ = OPS.split_decode(q, key_cache, value_cache, gbt, gl, k_host, v_host, cbt,
-                                          ds.cpu_lens.index_select(0, ds.dec_rows),
-                                          float(self.scale), row_order=ds.dec_order)
-                output.index_copy_(0, ds.dec_tok, out)
+                if (in_order and OPS.split_decode is HipOps.split_decode
+                        and output.dtype == q.dtype and output.shape[1:] == q.shape[1:]
+                        and output.is_cuda and _rows_in_place(output, ds.n_dec)
+                        and output.untyped_storage().data_ptr()
+                        != query.untyped_storage().data_ptr()):
+                    ops.split_decode(q, key_cache, value_cache, gbt, gl, k_host, v_host, cbt, cl,
+                                     float(self.scale), out=output[:ds.n_dec],
+                                     row_order=ds.dec_order)
+                else:
+                    out, _ = OPS.split_decode(q, key_cache, value_cache, gbt, gl, k_host, v_host,
+                                              cbt, cl, float(self.scale), row_order=ds.dec_order)
+                    output.index_copy_(0, ds.dec_tok, out)
 
         # 3) fresh prefills attend only this step's q/k/v (backend.py:331-340)
         try:

@@ -529,6 +529,50 @@ int fd_reshape_and_cache(const void* key, int64_t key_stride_tok, int64_t key_st
   return launch_cache_write(a, static_cast<hipStream_t>(stream));
 }
 
+int fd_reshape_and_cache_tiers(const void* key, int64_t key_stride_tok, int64_t key_stride_head,
+                               const void* value, int64_t value_stride_tok,
+                               int64_t value_stride_head, const fd_cache_target* hbm,
+                               const fd_cache_target* host, int32_t num_tokens,
+                               int32_t num_kv_heads, int32_t head_size, int32_t block_size,
+                               int32_t dtype, const int32_t* write_gate, void* stream) {
+  if (hbm == nullptr || host == nullptr)
+    return set_error(FD_ERR_INVALID, "reshape_and_cache_tiers: NULL target");
+  if (num_tokens < 0 || num_kv_heads <= 0 || head_size <= 0 || block_size <= 0)
+    return set_error(FD_ERR_INVALID, "reshape_and_cache_tiers: bad sizes");
+  if (!valid_dtype(dtype)) return set_error(FD_ERR_INVALID, "reshape_and_cache_tiers: bad dtype");
+  if (num_tokens == 0) return FD_OK;
+  if (!key || !value)
+    return set_error(FD_ERR_INVALID, "reshape_and_cache_tiers: NULL tensor pointer");
+  CacheWriteArgs w[2] = {};
+  const fd_cache_target* targets[2] = {hbm, host};
+  for (int t = 0; t < 2; ++t) {
+    const fd_cache_target& c = *targets[t];
+    if (c.num_blocks < 0 || !c.k_cache || !c.v_cache || !c.slot_mapping)
+      return set_error(FD_ERR_INVALID, "reshape_and_cache_tiers: bad target %d", t);
+    CacheWriteArgs& a = w[t];
+    a.key = key;
+    a.key_st = key_stride_tok;
+    a.key_sh = key_stride_head;
+    a.value = value;
+    a.value_st = value_stride_tok;
+    a.value_sh = value_stride_head;
+    a.kc = c.k_cache;
+    a.vc = c.v_cache;
+    a.c_sb = c.stride_block;
+    a.c_st = c.stride_token;
+    a.c_sh = c.stride_head;
+    a.num_blocks = c.num_blocks;
+    a.slots = c.slot_mapping;
+    a.T = num_tokens;
+    a.KVH = num_kv_heads;
+    a.D = head_size;
+    a.BS = block_size;
+    a.elt = dtype_size(dtype);
+    a.gate = write_gate;
+  }
+  return launch_cache_write(w[0], static_cast<hipStream_t>(stream), &w[1]);
+}
+
 int fd_check_slots(const int64_t* slots, int64_t m, int64_t capacity, int64_t* first_bad) {
   if (m < 0) return set_error(FD_ERR_INVALID, "check_slots: negative count");
   if (m > 0 && slots == nullptr) return set_error(FD_ERR_INVALID, "check_slots: NULL slots");

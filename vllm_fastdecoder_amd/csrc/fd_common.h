@@ -336,7 +336,8 @@ struct CacheWriteArgs {
   int32_t* err;
   const int32_t* gate;  // nothing is written when *gate != 0 (may be NULL)
 };
-int launch_cache_write(const CacheWriteArgs& a, hipStream_t s);
+// b: a second cache for the same rows (T, KVH, D, dtype), or NULL.
+int launch_cache_write(const CacheWriteArgs& a, hipStream_t s, const CacheWriteArgs* b = nullptr);
 
 int launch_stream_copy(void* dst, const void* src, size_t bytes, hipStream_t s);
 

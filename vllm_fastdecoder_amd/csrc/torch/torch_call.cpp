@@ -358,6 +358,55 @@ PyObject* split_decode(PyObject*, PyObject* const* a, Py_ssize_t na) {
   });
 }
 
+// key and value rows [T, KVH, D] of one shape, T given by the slots.
+bool kv_rows(const at::Tensor* key, const at::Tensor* value) {
+  return key != nullptr && value != nullptr && key->is_cuda() && value->device() == key->device() &&
+         key->dim() == 3 && value->sizes().equals(key->sizes()) &&
+         value->scalar_type() == key->scalar_type() && dtype_code(key->scalar_type()) >= 0 &&
+         key->stride(2) == 1 && value->stride(2) == 1;
+}
+
+// A cache the rows go to: [B, BS, KVH, D] views with token and head dims 1
+// and 2, or the host tier's [C, KVH, BS, D] with 2 and 1. 1: filled in; 0: not
+// for this path; -1: a Python error is set.
+int cache_target(const at::Tensor& key, PyObject* k_o, PyObject* v_o, PyObject* slots_o, int token,
+                 int head, fd_cache_target* c, int64_t* T, int64_t* BS) {
+  const at::Tensor* k = plain(k_o);
+  const at::Tensor* v = plain(v_o);
+  const at::Tensor* slots = plain_gpu(slots_o, at::kLong);
+  if (k == nullptr || v == nullptr || slots == nullptr || k->dim() != 4 || !same_layout(*k, *v) ||
+      slots->dim() != 1 || !slots->is_contiguous() || slots->device() != key.device())
+    return 0;
+  *T = slots->size(0);
+  *BS = k->size(token);
+  if (*T <= 0 || !fits32(*T) || key.size(0) < *T || k->size(head) != key.size(1) ||
+      k->size(3) != key.size(2) || !fits32(*BS))
+    return 0;
+  for (const at::Tensor* t : {k, v})
+    if (t->scalar_type() != key.scalar_type() ||
+        !(t->is_cuda() ? t->device() == key.device() : t->is_cpu()))
+      return 0;
+  const void *kp, *vp;
+  if (!cache_ptr(k_o, *k, &kp) || !cache_ptr(v_o, *v, &vp)) return -1;
+  c->k_cache = const_cast<void*>(kp);
+  c->v_cache = const_cast<void*>(vp);
+  c->stride_block = k->stride(0);
+  c->stride_token = k->stride(token);
+  c->stride_head = k->stride(head);
+  c->num_blocks = k->size(0);
+  c->slot_mapping = slots->data_ptr<int64_t>();
+  return 1;
+}
+
+// None, or an int32 device counter's address.
+bool device_counter(PyObject* o, int32_t** c) {
+  *c = nullptr;
+  if (o == Py_None) return true;
+  const at::Tensor* t = plain_gpu(o, at::kInt);
+  if (t != nullptr) *c = t->data_ptr<int32_t>();
+  return t != nullptr;
+}
+
 // cache_write(key, value, key_cache, value_cache, slots, error_count,
 //             write_gate): the caches as [B, BS, KVH, D] views -> status
 PyObject* cache_write(PyObject*, PyObject* const* a, Py_ssize_t na) {
@@ -365,45 +414,49 @@ PyObject* cache_write(PyObject*, PyObject* const* a, Py_ssize_t na) {
     if (na != 7 || modes_active()) return not_here();
     const at::Tensor* key = plain(a[0]);
     const at::Tensor* value = plain(a[1]);
-    const at::Tensor* k = plain(a[2]);
-    const at::Tensor* v = plain(a[3]);
-    const at::Tensor* slots = plain_gpu(a[4], at::kLong);
-    if (key == nullptr || value == nullptr || k == nullptr || v == nullptr || slots == nullptr ||
-        !key->is_cuda() || value->device() != key->device() || slots->device() != key->device() ||
-        key->dim() != 3 || value->dim() != 3 || k->dim() != 4 || !same_layout(*k, *v) ||
-        slots->dim() != 1 || !slots->is_contiguous())
+    int32_t *err, *gate;
+    if (!kv_rows(key, value) || !device_counter(a[5], &err) || !device_counter(a[6], &gate) ||
+        (err != nullptr && err == gate))
       return not_here();
-    const int64_t T = slots->size(0), KVH = k->size(2), D = k->size(3);
-    if (T <= 0 || !fits32(T) || !fits32(KVH) || !fits32(D) || !fits32(k->size(1)))
-      return not_here();
-    for (const at::Tensor* t : {key, value})
-      if (t->size(0) < T || t->size(1) != KVH || t->size(2) != D || t->stride(2) != 1 ||
-          t->scalar_type() != k->scalar_type())
-        return not_here();
-    // (value is cut to key's shape by the caller's contract: the same rows of both)
-    if (v->scalar_type() != k->scalar_type() || dtype_code(k->scalar_type()) < 0 ||
-        !value->sizes().equals(key->sizes()))
-      return not_here();
-    for (const at::Tensor* t : {k, v})
-      if (!(t->is_cuda() ? t->device() == key->device() : t->is_cpu())) return not_here();
-    int32_t* counter[2] = {nullptr, nullptr};
-    for (int i = 0; i < 2; ++i) {
-      if (a[5 + i] == Py_None) continue;
-      const at::Tensor* c = plain_gpu(a[5 + i], at::kInt);
-      if (c == nullptr) return not_here();
-      counter[i] = c->data_ptr<int32_t>();
-    }
-    if (counter[0] != nullptr && counter[0] == counter[1]) return not_here();
-    const void *kp, *vp;
+    fd_cache_target c{};
+    int64_t T, BS;
+    const int got = cache_target(*key, a[2], a[3], a[4], 1, 2, &c, &T, &BS);
+    if (got <= 0) return got == 0 ? not_here() : nullptr;
     void* stream;
-    if (!cache_ptr(a[2], *k, &kp) || !cache_ptr(a[3], *v, &vp) ||
-        !current_stream(key->get_device(), &stream))
-      return nullptr;
+    if (!current_stream(key->get_device(), &stream)) return nullptr;
     const int status = without_gil([&] { return fd_reshape_and_cache(
         key->data_ptr(), key->stride(0), key->stride(1), value->data_ptr(), value->stride(0),
-        value->stride(1), const_cast<void*>(kp), const_cast<void*>(vp), k->stride(0), k->stride(1),
-        k->stride(2), k->size(0), slots->data_ptr<int64_t>(), (int32_t)T, (int32_t)KVH, (int32_t)D,
-        (int32_t)k->size(1), dtype_code(k->scalar_type()), counter[0], counter[1], stream); });
+        value->stride(1), c.k_cache, c.v_cache, c.stride_block, c.stride_token, c.stride_head,
+        c.num_blocks, c.slot_mapping, (int32_t)T, (int32_t)key->size(1), (int32_t)key->size(2),
+        (int32_t)BS, dtype_code(key->scalar_type()), err, gate, stream); });
+    return PyLong_FromLong(status);
+  });
+}
+
+// cache_write_tiers(key, value, key_cache, value_cache, slots, host_k, host_v,
+//                   host_slots, write_gate): the host caches as [C, KVH, BS, D]
+PyObject* cache_write_tiers(PyObject*, PyObject* const* a, Py_ssize_t na) {
+  return guarded([&]() -> PyObject* {
+    if (na != 9 || modes_active()) return not_here();
+    const at::Tensor* key = plain(a[0]);
+    const at::Tensor* value = plain(a[1]);
+    int32_t* gate;
+    if (!kv_rows(key, value) || !device_counter(a[8], &gate)) return not_here();
+    fd_cache_target c[2] = {};
+    int64_t T[2], BS[2];
+    for (int t = 0; t < 2; ++t) {
+      PyObject* const* x = a + 2 + 3 * t;
+      const int got = cache_target(*key, x[0], x[1], x[2], t == 0 ? 1 : 2, t == 0 ? 2 : 1, &c[t],
+                                   &T[t], &BS[t]);
+      if (got <= 0) return got == 0 ? not_here() : nullptr;
+    }
+    if (T[0] != T[1] || BS[0] != BS[1]) return not_here();
+    void* stream;
+    if (!current_stream(key->get_device(), &stream)) return nullptr;
+    const int status = without_gil([&] { return fd_reshape_and_cache_tiers(
+        key->data_ptr(), key->stride(0), key->stride(1), value->data_ptr(), value->stride(0),
+        value->stride(1), &c[0], &c[1], (int32_t)T[0], (int32_t)key->size(1),
+        (int32_t)key->size(2), (int32_t)BS[0], dtype_code(key->scalar_type()), gate, stream); });
     return PyLong_FromLong(status);
   });
 }
@@ -429,6 +482,9 @@ PyMethodDef methods[] = {
      METH_FASTCALL, nullptr},
     {"cache_write", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(cache_write)),
      METH_FASTCALL, nullptr},
+    {"cache_write_tiers",
+     reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(cache_write_tiers)), METH_FASTCALL,
+     nullptr},
     {nullptr, nullptr, 0, nullptr},
 };
 

@@ -1204,6 +1204,26 @@ def reshape_and_cache(key, value, key_cache, value_cache, slot_mapping,
                  B, BS, slot_mapping, error_count, write_gate)
 
 
+def reshape_and_cache_tiers(key, value, key_cache, value_cache, slot_mapping, host_k_cache,
+                            host_v_cache, host_slot_mapping,
+                            write_gate: torch.Tensor | None = None) -> None:
+    """reshape_and_cache into both tiers (plan_tiers' slot mappings), in one
+    launch where the arguments allow it: key_cache / value_cache
+    [B, BS, KVH, D] views, host_k_cache / host_v_cache [C, KVH, BS, D] pinned
+    host memory. write_gate as in reshape_and_cache. No counterpart in the
+    reference, which writes each tier by its own call."""
+    native = _NATIVE or _native()
+    if native:
+        status = native.cache_write_tiers(key, value, key_cache, value_cache, slot_mapping,
+                                          host_k_cache, host_v_cache, host_slot_mapping,
+                                          write_gate)
+        if status is not None:
+            return _lib.check(status)
+    reshape_and_cache(key, value, key_cache, value_cache, slot_mapping, write_gate=write_gate)
+    reshape_and_cache(key, value, host_k_cache.transpose(1, 2), host_v_cache.transpose(1, 2),
+                      host_slot_mapping, write_gate=write_gate)
+
+
 def store_kv(k, v, slots, k_cache, v_cache) -> None:
     """Host-tier KV write, signature of cpu_attn.cpp:492-517.
 
