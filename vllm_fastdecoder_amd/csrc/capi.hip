@@ -137,10 +137,15 @@ int run_decode(DecodeArgs& a, const char* who, const void* q, int64_t q_stride_s
                              (int32_t)width, kv_dtype, aligned, true, fill);
   // Over the link the matrix-core kernels' K tiles (16 token rows of 16 bytes
   // per lane group) read slower than the VALU kernel's whole rows (measured
-  // on a GQA-4 host tier: 47.9 against 55.9 GB/s; in HBM the two are within
-  // 3 %), so launches that read pinned host memory take the VALU kernel.
+  // on a GQA-4 host tier: 47.9 against 55.9 GB/s), so partials over pinned
+  // host memory take the VALU kernel. A two-tier launch on decode_mm_kernel
+  // reads its host blocks in whole rows and stays there for its HBM blocks,
+  // most of which the VALU kernel's per-head work holds up (33 rows of
+  // U[40, 1800], 32/8, one host block each: 45 -> 35 us; 64 of U[500, 1500]: 97 -> 80).
   bool host = false;
-  for (int t = 0; (sp.mfma || sp.mm) && t < a.ntiers; ++t) host = host || in_host_memory(a.tier[t].k);
+  const int read_in_rows = a.ntiers > 1 && sp.mm ? 1 : 0;  // of the tiers, the last
+  for (int t = 0; (sp.mfma || sp.mm) && t < a.ntiers - read_in_rows; ++t)
+    host = host || in_host_memory(a.tier[t].k);
   if (host)
     sp = plan_decode(n, num_heads, num_kv_heads, head_size, block_size, (int32_t)width, kv_dtype,
                      aligned, false, fill);
@@ -182,19 +187,9 @@ int run_decode(DecodeArgs& a, const char* who, const void* q, int64_t q_stride_s
 }
 
 }  // namespace
-}  // namespace fd
 
-using namespace fd;
-
-extern "C" {
-
-const char* fd_last_error(void) { return g_err; }
-
-int fd_abi_version(void) { return 13; }
-
-int fd_paged_decode_workspace_size(int32_t n, int32_t num_heads, int32_t num_kv_heads,
-                                   int32_t head_size, int32_t block_size, int32_t bt_width,
-                                   size_t* bytes) {
+int workspace_size(int32_t n, int32_t num_heads, int32_t num_kv_heads, int32_t head_size,
+                   int32_t block_size, int32_t bt_width, WorkspaceScope scope, size_t* bytes) {
   if (bytes == nullptr) return set_error(FD_ERR_INVALID, "workspace_size: bytes is NULL");
   if (n < 0 || num_heads <= 0 || num_kv_heads <= 0 || head_size <= 0 || block_size <= 0 ||
       bt_width < 0)
@@ -212,12 +207,30 @@ int fd_paged_decode_workspace_size(int32_t n, int32_t num_heads, int32_t num_kv_
     // what a token total may make of it (fd_paged_decode_partial_hint)
     most = std::max(most, fill_workspace_bound(sp, n, num_heads, num_kv_heads, head_size,
                                                block_size, bt_width, dts[c]));
+    if (scope == WorkspaceScope::kCutsByWidth) continue;
     // balanced cuts, with room for the arrival counters
     most = std::max(most, balanced_partial_bytes(sp, num_heads, head_size) +
                               balanced_counter_bytes(sp, n, num_kv_heads));
   }
   *bytes = most;
   return FD_OK;
+}
+
+}  // namespace fd
+
+using namespace fd;
+
+extern "C" {
+
+const char* fd_last_error(void) { return g_err; }
+
+int fd_abi_version(void) { return 13; }
+
+int fd_paged_decode_workspace_size(int32_t n, int32_t num_heads, int32_t num_kv_heads,
+                                   int32_t head_size, int32_t block_size, int32_t bt_width,
+                                   size_t* bytes) {
+  return workspace_size(n, num_heads, num_kv_heads, head_size, block_size, bt_width,
+                        WorkspaceScope::kAll, bytes);
 }
 
 int fd_decode_workspace_need(int32_t n, int32_t num_heads, int32_t num_kv_heads,

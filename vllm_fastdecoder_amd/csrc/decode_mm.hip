@@ -118,6 +118,7 @@ __global__ __launch_bounds__(kWave * kWavesPerTask) void decode_mm_kernel(TiledP
   constexpr int TC = kTileTokens * CPT;  // V: 16-byte chunks per block
   constexpr int NLD = (TC + kWave - 1) / kWave;  // V: loads per block (lane l of load j
                                                  // takes chunk 64 j + l, if < TC)
+  static_assert(NLD == KS, "a block's K and V are as many loads in either order");
   constexpr float kPScale = std::is_same<T, F16>::value ? 128.f : 1.f;
   // K is read in 64-byte column slices, so most lines are read by two loads
   // of the wave; below 128 dims (64 aside) non-temporal lines were often
@@ -132,7 +133,7 @@ __global__ __launch_bounds__(kWave * kWavesPerTask) void decode_mm_kernel(TiledP
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   Task t;
-  if (!decode_task<COLS, TWO>(p, t)) return;
+  if (!decode_task<COLS, TWO, CG == 1>(p, t)) return;
   if (t.nb == 0 || t.range_bad) {
     if (t.split == 0 && wave == 0) write_empty<T, D, COLS>(p, t, lane);
     return;
@@ -160,7 +161,7 @@ __global__ __launch_bounds__(kWave * kWavesPerTask) void decode_mm_kernel(TiledP
   int vtok[NLD];
   const TierParams& t0 = p.tier[0];
   const uint32_t koff0 = (uint32_t)(((int64_t)col * t0.st + R * 8) * 2);
-  uint32_t voff0[NLD], voff1[NLD], koff1 = 0;
+  uint32_t voff0[NLD], voff1[NLD];
 #pragma unroll
   for (int j = 0; j < NLD; ++j) {
     const int c = kWave * j + lane < TC ? kWave * j + lane : 0;  // spare lanes read chunk 0
@@ -170,7 +171,6 @@ __global__ __launch_bounds__(kWave * kWavesPerTask) void decode_mm_kernel(TiledP
   }
   if constexpr (TWO) {
     const TierParams& t1 = p.tier[1];
-    koff1 = (uint32_t)(((int64_t)col * t1.st + R * 8) * 2);
 #pragma unroll
     for (int j = 0; j < NLD; ++j) {
       const int c = kWave * j + lane < TC ? kWave * j + lane : 0;
@@ -209,9 +209,16 @@ __global__ __launch_bounds__(kWave * kWavesPerTask) void decode_mm_kernel(TiledP
   Vec8 kb[2][KS], vb[2][NLD];
   auto load_block = [&](int slot, int k) {
     const BlockSrc src = block_src<TWO>(p, wb, t, k);
-    const uint32_t koff = src.t1 ? koff1 : koff0;
+    if (TWO && src.t1) {
+      // tier 1's K in whole rows, as V: over the link a wave's 1 KiB in one
+      // run reads 15 % faster than 64 bytes of every row; block_scores turns
+      // it into the A operand through LDS
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) kb[slot][ks] = buffer_ld16<POL>(src.k, koff, 64 * ks);
+      for (int j = 0; j < KS; ++j) kb[slot][j] = buffer_ld16<POL>(src.k, voff1[j]);
+    } else {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) kb[slot][ks] = buffer_ld16<POL>(src.k, koff0, 64 * ks);
+    }
 #pragma unroll
     for (int j = 0; j < NLD; ++j)
       vb[slot][j] = buffer_ld16<POL>(src.v, src.t1 ? voff1[j] : voff0[j]);
@@ -220,7 +227,23 @@ __global__ __launch_bounds__(kWave * kWavesPerTask) void decode_mm_kernel(TiledP
 
   // Scores of the K block in `slot` for every group (log2 domain, masked
   // past ntok).
-  auto block_scores = [&](int slot, int ntok, float (*s)[4]) {
+  auto block_scores = [&](int slot, int k, int ntok, float (*s)[4]) {
+    if (TWO && k >= wb.k1) {
+      // rows to A operand, through the LDS slot that takes the block's V next
+      // (DS operations of a wave run in order)
+      uint16_t* st = stage + (k & 1) * kTileTokens * D;
+#pragma unroll
+      for (int j = 0; j < KS; ++j) {
+        if (TC % kWave == 0 || vtok[j] < kTileTokens)
+          *reinterpret_cast<uint4*>(st + 8 * (kWave * j + lane)) = make_uint4(
+              kb[slot][j].w[0], kb[slot][j].w[1], kb[slot][j].w[2], kb[slot][j].w[3]);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+        if (32 * (ks + 1) <= D || k_dims_on(ks)) kb[slot][ks] = ld16(st + col * D + R * 8 + 32 * ks);
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    }
     f32x4 sv[CG];
 #pragma unroll
     for (int g = 0; g < CG; ++g) sv[g] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -316,18 +339,18 @@ __global__ __launch_bounds__(kWave * kWavesPerTask) void decode_mm_kernel(TiledP
     int k = 0;
     load_block(0, 0);
     for (; k + 2 < nw; k += 2) {
-      block_scores(0, ntok_of(k), s);
+      block_scores(0, k, ntok_of(k), s);
       load_block(1, k + 1);
       block_update(0, k, ntok_of(k), s);
-      block_scores(1, ntok_of(k + 1), s);
+      block_scores(1, k + 1, ntok_of(k + 1), s);
       load_block(0, k + 2);
       block_update(1, k + 1, ntok_of(k + 1), s);
     }
-    block_scores(0, ntok_of(k), s);
+    block_scores(0, k, ntok_of(k), s);
     if (k + 1 < nw) {
       load_block(1, k + 1);
       block_update(0, k, ntok_of(k), s);
-      block_scores(1, ntok_of(k + 1), s);
+      block_scores(1, k + 1, ntok_of(k + 1), s);
       block_update(1, k + 1, ntok_of(k + 1), s);
     } else {
       block_update(0, k, ntok_of(k), s);
@@ -346,7 +369,7 @@ __global__ __launch_bounds__(kWave * kWavesPerTask) void decode_mm_kernel(TiledP
   for (int g = 0; g < CG; ++g) {
     const float lt = xor_sum<16>(l[g]);
     __syncthreads();  // the V staging (g = 0) or the previous group's merge is done
-    if (kCols * g + 4 * R < t.gcount) {  // rows of real columns
+    if (CG > 1 || 4 * R < t.gcount) {  // rows of real columns
 #pragma unroll
       for (int c = 0; c < NC; ++c) {
 #pragma unroll
@@ -408,7 +431,7 @@ __global__ __launch_bounds__(kWave * kWavesPerTask) void decode_mm_kernel(TiledP
           store8<T>(p.out, (int64_t)t.i * p.out_ss + (int64_t)h * p.out_sh + d0, p.out_f32, o);
           if (d0 == 0) p.lse[(int64_t)h * p.lse_sh + t.i] = lse2 * kLn2;
         } else {
-          store_partial(p, t, h, d0, o, lse2);
+          store_partial<CG == 1>(p, t, h, d0, o, lse2);
         }
       }
     }

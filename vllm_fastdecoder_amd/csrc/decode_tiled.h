@@ -472,9 +472,10 @@ __device__ __forceinline__ bool balanced_task(const TiledParams& p, Task& t) {
   return false;
 }
 
-template <int G, bool TWO>
+// BAL: the kernel takes balanced cuts (tasks of at most 16 heads do).
+template <int G, bool TWO, bool BAL = true>
 __device__ __forceinline__ bool decode_task(const TiledParams& p, Task& t) {
-  if (p.bal_parts > 0)
+  if (BAL && p.bal_parts > 0)
     return p.n <= kWave ? balanced_task<G, TWO, 1>(p, t) : balanced_task<G, TWO, kBalChunks>(p, t);
   const int task = p.xcd_group ? xcd_task(blockIdx.x, gridDim.x) : (int)blockIdx.x;
   t.kh = task % p.KVH;
@@ -672,9 +673,10 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t part_rsrc(const float* base, i
 
 // Writes a split task's partial of 8 dims of query head h: the normalised
 // output and, with d0 == 0, the LSE (lse2: log2 domain).
+template <bool BAL = true>
 __device__ __forceinline__ void store_partial(const TiledParams& p, const Task& t, int h, int d0,
                                               const float* o, float lse2) {
-  if (p.bal_parts > 0) {
+  if (BAL && p.bal_parts > 0) {
     const int64_t pidx = (int64_t)(t.slot0 + t.split) * p.H + h;
     const __amdgpu_buffer_rsrc_t ro = part_rsrc(p.part_o + pidx * p.D, p.D);
 #pragma unroll

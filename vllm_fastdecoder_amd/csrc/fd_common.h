@@ -300,6 +300,12 @@ size_t balanced_counter_bytes(const SplitPlan& sp, int32_t n, int32_t KVH);
 size_t fill_workspace_bound(const SplitPlan& sp, int32_t n, int32_t H, int32_t KVH, int32_t D,
                             int32_t BS, int32_t bt_width, int32_t kv_dtype);
 int launch_decode(const DecodeArgs& a, const SplitPlan& sp, hipStream_t s);
+// Workspace a decode call of these sizes may need: for every launch it may
+// become, or for the cuts by table width alone (which a call falls back to
+// when its workspace covers no more).
+enum class WorkspaceScope { kCutsByWidth, kAll };
+int workspace_size(int32_t n, int32_t num_heads, int32_t num_kv_heads, int32_t head_size,
+                   int32_t block_size, int32_t bt_width, WorkspaceScope scope, size_t* bytes);
 
 struct MergeArgs {
   void* out;

@@ -66,12 +66,15 @@ extern "C" int fd_paged_decode_partial_noalloc(
     int64_t lse_stride_head, void* stream) {
   // The size query plans for the fast kernels, the only ones with split
   // partials, so it bounds what the call below can need; it is pure host code.
+  // (Cuts by the rows' lengths are used where the scratch holds their parts.)
   size_t need = 0;
+  bool sized = false;
   if (n > 0 && num_heads > 0 && num_kv_heads > 0 && head_size > 0 && block_size > 0 &&
       bt_width >= 0) {
-    const int rc = fd_paged_decode_workspace_size(n, num_heads, num_kv_heads, head_size,
-                                                  block_size, bt_width, &need);
+    const int rc = fd::workspace_size(n, num_heads, num_kv_heads, head_size, block_size, bt_width,
+                                      fd::WorkspaceScope::kCutsByWidth, &need);
     if (rc != FD_OK) return rc;
+    sized = true;
   }
   if (need > kScratchBytes)
     return fd::set_error(FD_ERR_WORKSPACE,
@@ -80,7 +83,7 @@ extern "C" int fd_paged_decode_partial_noalloc(
                          "fd_paged_decode_partial with a workspace instead",
                          need, kScratchBytes);
   void* ws = nullptr;
-  if (need > 0) {
+  if (sized) {
     const int rc = scratch_address(&ws);
     if (rc != FD_OK) return rc;
   }
@@ -89,5 +92,5 @@ extern "C" int fd_paged_decode_partial_noalloc(
                                  block_table, bt_stride, bt_width, lens, row_order, n, num_heads,
                                  num_kv_heads, head_size, block_size, scale, kv_dtype, out,
                                  out_stride_seq, out_stride_head, out_dtype, lse, lse_stride_head,
-                                 ws, need > 0 ? kScratchBytes : 0, stream);
+                                 ws, ws != nullptr ? kScratchBytes : 0, stream);
 }
