@@ -251,8 +251,9 @@ int fd_decode_workspace_need(int32_t n, int32_t num_heads, int32_t num_kv_heads,
  *   aligned     1 if the launch meets the tiled kernels' alignment rules
  *               (16-byte aligned q, out and caches; strides multiples of 8
  *               elements), else 0 (the generic kernel)
- *   host_tier   1 if a tier lies in pinned host memory (16-bit launches then
- *               take the VALU kernel)
+ *   host_tier   1 if the cache lies in pinned host memory (16-bit partials
+ *               then take the VALU kernel; a two-tier launch with only its
+ *               host tier there takes the matrix-core kernel where 0 gives it)
  *   total_tokens the rows' token total, as given to
  *               fd_paged_decode_partial_hint (0: unknown)
  * FD_DECODE_KERNEL and FD_SPLIT_BLOCKS are honoured as in a launch. */
@@ -334,8 +335,10 @@ int fd_paged_decode_partial_noalloc(
  *   out[i, h, :] = softmax(scale * q . [K_hbm ; K_host]^T) @ [V_hbm ; V_host]
  *   lse[h, i]    = logsumexp over both tiers (natural log),
  * which equals merge(partial_hbm, partial_host) of the separate calls. The
- * kernel walks each row's HBM-tier blocks, then its host-tier blocks, as one
- * list and merges in-kernel: no partial round trip and no merge launch.
+ * kernel takes each row's HBM-tier and host-tier blocks as one list and merges
+ * in-kernel: no partial round trip and no merge launch. Up to 64 rows over a
+ * host tier in pinned memory, some workgroups take the host tier's blocks and
+ * the others the HBM tier's, so that the link and HBM are read at once.
  *
  * Each tier is described by an fd_kv_tier: the same cache/stride/table/length
  * conventions as fd_paged_decode_partial, per tier (tier-relative block ids,

@@ -1,8 +1,10 @@
-"""Two-tier launches whose tasks divide their waves between the tiers
-(wave_blocks in decode_tiled.h) and read only the valid tokens of a host block
-(block_src): host shares from one block to all but one, rows up to the 256
-blocks a task holds (past 64 blocks per wave the division does not apply),
-stale host rows full of NaN. Bars of test_gpu_split_fused."""
+"""Two-tier launches: tasks that divide their waves between the tiers
+(wave_blocks in decode_tiled.h), host blocks read only as far as they hold
+tokens (block_src), and host workers that take the host tier alone
+(balanced_task, decode_mm_tiers_kernel): host shares from one block to all but
+one, rows up to the 256 blocks a task holds (past 64 blocks per wave the
+division does not apply), stale host rows full of NaN, one worker taking every
+part in turn. Bars of test_gpu_split_fused."""
 
 from __future__ import annotations
 
@@ -23,21 +25,17 @@ ROWS = [(1, 1, 1), (1, 40, 16), (40, 1, 3), (3, 3, 15), (20, 11, 7), (11, 20, 9)
         (193, 63, 16), (63, 192, 1), (128, 128, 8), (0, 5, 2), (5, 0, 16), (0, 0, 16)]
 
 
-@pytest.mark.parametrize("split", ["256", "32"])
-@pytest.mark.parametrize("H,KVH,D,dtype", [(2, 2, 128, torch.float16), (4, 1, 128, torch.bfloat16),
-                                           (2, 1, 256, torch.float16), (2, 2, 64, torch.float32)])
-def test_tier_shares(gpu, H, KVH, D, dtype, split, monkeypatch):
-    monkeypatch.setenv("FD_SPLIT_BLOCKS", split)
-    BS, n = 16, len(ROWS)
+def _run(gpu, H, KVH, D, dtype, rows, row_order=None, bad_row=None):
+    BS, n = 16, len(rows)
     g = torch.Generator().manual_seed(D + H)
-    G, C = sum(r[0] for r in ROWS), sum(r[1] for r in ROWS)
-    W = max(a + b for a, b, _ in ROWS)
+    G, C = sum(r[0] for r in rows), sum(r[1] for r in rows)
+    W = max(a + b for a, b, _ in rows)
     pool_k = torch.randn(G + C, KVH, BS, D, generator=g).to(dtype)
     pool_v = torch.randn(G + C, KVH, BS, D, generator=g).to(dtype)
-    bt_g, bt_c, full = (torch.zeros(n, W, dtype=torch.int32) for _ in range(3))
+    bt_g, bt_c, full = (torch.zeros(n, max(W, 1), dtype=torch.int32) for _ in range(3))
     lens_g, lens_c = [], []
     pg, pc = torch.randperm(G, generator=g).int(), torch.randperm(C, generator=g).int()
-    for i, (a, b, last) in enumerate(ROWS):
+    for i, (a, b, last) in enumerate(rows):
         bt_g[i, :a], pg = pg[:a], pg[a:]
         bt_c[i, :b], pc = pc[:b], pc[b:]
         full[i, :a], full[i, a:a + b] = bt_g[i, :a], bt_c[i, :b] + G
@@ -52,15 +50,62 @@ def test_tier_shares(gpu, H, KVH, D, dtype, split, monkeypatch):
     hk, hv = pinned_empty((C, KVH, BS, D), dtype), pinned_empty((C, KVH, BS, D), dtype)
     hk.copy_(pool_k[G:])
     hv.copy_(pool_v[G:])
-    out = torch.empty(n, H, D, device=gpu)
-    out, lse = ops.split_decode(
+    if bad_row is not None:  # a host block id past the host cache
+        bt_c[bad_row, 0] = C + 1
+    out = torch.full((n, H, D), 7.0, device=gpu)
+    lse = torch.full((H, n), 7.0, device=gpu)
+    ops.split_decode(
         q.to(gpu), kv[..., :D], kv[..., D:], bt_g.to(gpu),
         torch.tensor(lens_g, dtype=torch.int32, device=gpu), hk, hv, bt_c.to(gpu),
-        torch.tensor(lens_c, dtype=torch.int32, device=gpu), 1 / math.sqrt(D), out=out)
+        torch.tensor(lens_c, dtype=torch.int32, device=gpu), 1 / math.sqrt(D), out=out, lse=lse,
+        row_order=row_order)
     torch.cuda.synchronize()
     ref_out, ref_lse = oracle.decode_attn_host_layout_f64(q, pool_k, pool_v, full, lens,
                                                           1 / math.sqrt(D))
-    nz = lens > 0
-    assert_out_close(out, ref_out, 5e-5 if dtype == torch.float32 else 2e-3, mask=nz)
-    assert_lse_close(lse, ref_lse, mask=nz)
-    assert torch.all(out[~nz.to(gpu)] == 0) and torch.all(torch.isneginf(lse[:, ~nz.to(gpu)]))
+    return out, lse, ref_out, ref_lse, lens
+
+
+def _check(got, dtype, rows=None):
+    out, lse, ref_out, ref_lse, lens = got
+    rows = list(range(len(lens))) if rows is None else rows
+    nz = lens[rows] > 0
+    out, lse = out.cpu()[rows], lse.cpu()[:, rows]
+    assert_out_close(out, ref_out[rows], 5e-5 if dtype == torch.float32 else 2e-3, mask=nz)
+    assert_lse_close(lse, ref_lse[:, rows], mask=nz)
+    assert torch.all(out[~nz] == 0) and torch.all(torch.isneginf(lse[:, ~nz]))
+
+
+@pytest.mark.parametrize("split", ["256", "32"])
+@pytest.mark.parametrize("H,KVH,D,dtype", [(2, 2, 128, torch.float16), (4, 1, 128, torch.bfloat16),
+                                           (2, 1, 256, torch.float16), (2, 2, 64, torch.float32)])
+def test_tier_shares(gpu, H, KVH, D, dtype, split, monkeypatch):
+    monkeypatch.setenv("FD_SPLIT_BLOCKS", split)
+    _check(_run(gpu, H, KVH, D, dtype, ROWS), dtype)
+
+
+@pytest.mark.parametrize("workers", ["1", "32"])
+@pytest.mark.parametrize("H,KVH,D,dtype", [
+    (2, 2, 128, torch.float16), (6, 2, 128, torch.bfloat16), (4, 1, 128, torch.bfloat16),
+    (7, 1, 48, torch.float16), (16, 1, 64, torch.bfloat16), (10, 2, 80, torch.float16)])
+def test_host_workers(gpu, H, KVH, D, dtype, workers, monkeypatch):
+    """Rows of every tier share, one row, and 64 (the most the workers take);
+    the same bits on a second call and in any order."""
+    monkeypatch.setenv("FD_HOST_WGS", workers)
+    first = _run(gpu, H, KVH, D, dtype, ROWS)
+    _check(first, dtype)
+    order = torch.randperm(len(ROWS), generator=torch.Generator().manual_seed(2)).int()
+    again = _run(gpu, H, KVH, D, dtype, ROWS, row_order=order)
+    assert torch.equal(again[0], first[0]) and torch.equal(again[1], first[1])
+    _check(_run(gpu, H, KVH, D, dtype, [(30, 9, 4)]), dtype)
+    _check(_run(gpu, H, KVH, D, dtype, [(i % 5, (3 * i) % 7, 1 + i % 16) for i in range(64)]), dtype)
+
+
+def test_host_workers_leave_out_and_range_errors(gpu):
+    rows = list(range(len(ROWS)))
+    order = torch.tensor([r if r not in (2, 5) else -1 for r in rows], dtype=torch.int32)
+    got = _run(gpu, 4, 1, 128, torch.bfloat16, ROWS, row_order=order)
+    _check(got, torch.bfloat16, [r for r in rows if r not in (2, 5)])
+    assert torch.all(got[0][[2, 5]] == 7.0) and torch.all(got[1][:, [2, 5]] == 7.0)
+    got = _run(gpu, 4, 1, 128, torch.bfloat16, ROWS, bad_row=4)
+    _check(got, torch.bfloat16, [r for r in rows if r != 4])
+    assert torch.isnan(got[0][4]).all() and torch.isnan(got[1][:, 4]).all()

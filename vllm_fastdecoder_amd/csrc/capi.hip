@@ -152,10 +152,19 @@ int run_decode(DecodeArgs& a, const char* who, const void* q, int64_t q_stride_s
   // Balanced cuts need a workspace for whatever the rows' lengths make of
   // them. A caller that brings less (it planned without them) gets the cuts
   // by table width.
-  const size_t bal = balanced_partial_bytes(sp, num_heads, head_size) +
-                     (a.counters == nullptr ? balanced_counter_bytes(sp, n, num_kv_heads) : 0);
-  if (bal > 0 && (workspace == nullptr || workspace_bytes < bal || !aligned16(workspace)))
-    sp.bal_parts = 0;
+  auto fits_workspace = [&](const SplitPlan& c) -> bool {
+    const size_t bal = balanced_partial_bytes(c, num_heads, head_size) +
+                       (a.counters == nullptr ? balanced_counter_bytes(c, n, num_kv_heads) : 0);
+    return bal == 0 || (workspace != nullptr && workspace_bytes >= bal && aligned16(workspace));
+  };
+  if (a.ntiers > 1 && in_host_memory(a.tier[1].k) && !in_host_memory(a.tier[0].k)) {
+    SplitPlan hw = sp;
+    if (plan_host_workers(hw, n, num_heads, num_kv_heads, head_size, block_size, (int32_t)width,
+                          kv_dtype) &&
+        fits_workspace(hw))
+      sp = hw;
+  }
+  if (!fits_workspace(sp)) sp.bal_parts = 0;
   // a timeline is of whole tasks by table width, as its buffer is sized for
   if (a.timeline != nullptr) sp.bal_parts = 0;
   const size_t need = sp.bal_parts > 0 ? 0 : decode_workspace_bytes(sp, n, num_heads, head_size);
@@ -211,6 +220,12 @@ int workspace_size(int32_t n, int32_t num_heads, int32_t num_kv_heads, int32_t h
     // balanced cuts, with room for the arrival counters
     most = std::max(most, balanced_partial_bytes(sp, num_heads, head_size) +
                               balanced_counter_bytes(sp, n, num_kv_heads));
+    // a two-tier launch with its host tier in pinned memory
+    SplitPlan hw = sp;
+    if (plan_host_workers(hw, n, num_heads, num_kv_heads, head_size, block_size, bt_width,
+                          dts[c]))
+      most = std::max(most, balanced_partial_bytes(hw, num_heads, head_size) +
+                                balanced_counter_bytes(hw, n, num_kv_heads));
   }
   *bytes = most;
   return FD_OK;
@@ -247,6 +262,10 @@ int fd_decode_workspace_need(int32_t n, int32_t num_heads, int32_t num_kv_heads,
                                    row_fill(total_tokens, n, bt_width, block_size));
   *bytes = sp.bal_parts > 0 ? balanced_partial_bytes(sp, num_heads, head_size)
                             : decode_workspace_bytes(sp, n, num_heads, head_size);
+  SplitPlan hw = sp;
+  if (host_tier != 0 && plan_host_workers(hw, n, num_heads, num_kv_heads, head_size, block_size,
+                                          bt_width, kv_dtype))
+    *bytes = std::max(*bytes, balanced_partial_bytes(hw, num_heads, head_size));
   return FD_OK;
 }
 

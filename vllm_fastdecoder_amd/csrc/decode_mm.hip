@@ -106,11 +106,15 @@ struct __align__(16) MmLds {  // 16-byte V rows, float4 merge reads
   };
 };
 
-template <typename T, int D, int CG, bool TWO>
-__global__ __launch_bounds__(kWave * kWavesPerTask) void decode_mm_kernel(TiledParams p) {
+// One task of the kernel, over tier 0's blocks, both tiers' or (one wave, a
+// host worker's) tier 1's.
+template <typename T, int D, int CG, int TS>
+__device__ __forceinline__ void mm_task(const TiledParams& p, const Task& t, MmLds<D>& lds,
+                                        int wave, int lane) {
+  constexpr bool TWO = TS == kBothTiers;
+  constexpr bool SOLO = TS == kSecondTier;
   static_assert(D % 16 == 0 && D >= 32 && D <= 128, "decode_mm_kernel: D = 16 m, 32..128");
   static_assert(CG == 1 || CG == 2 || (CG == 4 && D <= 64), "decode_mm_kernel: CG 1, 2, 4");
-  constexpr int COLS = kCols * CG;       // query heads per task
   constexpr int KS = (D + 31) / 32;      // scores: 32-dim matrix-core steps (the last
                                          // masked past D when D is not a multiple of 32)
   constexpr int NC = D / 16;             // P.V: 16-dim output chunks
@@ -127,17 +131,6 @@ __global__ __launch_bounds__(kWave * kWavesPerTask) void decode_mm_kernel(TiledP
   // 5.8 / 5.9 TB/s against 3.9 / 3.7 / 4.7 / 5.5 / 5.2 non-temporal, and
   // D = 64 / 128 at 5.6 / 6.0 against 6.1 / 6.2.
   constexpr int POL = (D == 64 || D == 128) ? kKvLoadPolicy : kKvLoadKeep;
-
-  __shared__ MmLds<D> lds;
-
-  const int lane = threadIdx.x & (kWave - 1);
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  Task t;
-  if (!decode_task<COLS, TWO, CG == 1>(p, t)) return;
-  if (t.nb == 0 || t.range_bad) {
-    if (t.split == 0 && wave == 0) write_empty<T, D, COLS>(p, t, lane);
-    return;
-  }
 
   const int col = lane & 15;  // K: token row of the A operand; scores: column
   const int R = lane >> 4;    // K: dims 8R..+7 of each step; scores: tokens 4R..4R+3
@@ -159,7 +152,7 @@ __global__ __launch_bounds__(kWave * kWavesPerTask) void decode_mm_kernel(TiledP
   // row-major in LDS it sits at element 8 c. Byte offsets inside one (block,
   // head) run, per tier: K step ks at koff + 64*ks, V load j at voff[j].
   int vtok[NLD];
-  const TierParams& t0 = p.tier[0];
+  const TierParams& t0 = p.tier[SOLO ? 1 : 0];
   const uint32_t koff0 = (uint32_t)(((int64_t)col * t0.st + R * 8) * 2);
   uint32_t voff0[NLD], voff1[NLD];
 #pragma unroll
@@ -196,10 +189,10 @@ __global__ __launch_bounds__(kWave * kWavesPerTask) void decode_mm_kernel(TiledP
     for (int c = 0; c < NC; ++c) acc[g][c] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
 
-  const WaveBlocks wb = wave_blocks<TWO>(p, t, wave, lane);
+  const WaveBlocks wb = wave_blocks<TS>(p, t, wave, lane);
   const int nw = wb.nw;
   auto ntok_of = [&](int k) -> int {
-    return block_tokens<TWO>(t, wb.first + wb.stride * k);
+    return block_tokens<TS>(t, wb.first + wb.stride * k);
   };
 
   // K and V double-buffered in registers: block k+1's loads are issued right
@@ -208,27 +201,27 @@ __global__ __launch_bounds__(kWave * kWavesPerTask) void decode_mm_kernel(TiledP
   // shapes: HBM is already busy and the extra requests only queue.)
   Vec8 kb[2][KS], vb[2][NLD];
   auto load_block = [&](int slot, int k) {
-    const BlockSrc src = block_src<TWO>(p, wb, t, k);
-    if (TWO && src.t1) {
+    const BlockSrc src = block_src<TS>(p, wb, t, k);
+    if (SOLO || (TWO && src.t1)) {
       // tier 1's K in whole rows, as V: over the link a wave's 1 KiB in one
       // run reads 15 % faster than 64 bytes of every row; block_scores turns
       // it into the A operand through LDS
 #pragma unroll
-      for (int j = 0; j < KS; ++j) kb[slot][j] = buffer_ld16<POL>(src.k, voff1[j]);
+      for (int j = 0; j < KS; ++j) kb[slot][j] = buffer_ld16<POL>(src.k, SOLO ? voff0[j] : voff1[j]);
     } else {
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) kb[slot][ks] = buffer_ld16<POL>(src.k, koff0, 64 * ks);
     }
 #pragma unroll
     for (int j = 0; j < NLD; ++j)
-      vb[slot][j] = buffer_ld16<POL>(src.v, src.t1 ? voff1[j] : voff0[j]);
+      vb[slot][j] = buffer_ld16<POL>(src.v, TWO && src.t1 ? voff1[j] : voff0[j]);
     __builtin_amdgcn_sched_barrier(0);
   };
 
   // Scores of the K block in `slot` for every group (log2 domain, masked
   // past ntok).
   auto block_scores = [&](int slot, int k, int ntok, float (*s)[4]) {
-    if (TWO && k >= wb.k1) {
+    if (SOLO || (TWO && k >= wb.k1)) {
       // rows to A operand, through the LDS slot that takes the block's V next
       // (DS operations of a wave run in order)
       uint16_t* st = stage + (k & 1) * kTileTokens * D;
@@ -363,12 +356,17 @@ __global__ __launch_bounds__(kWave * kWavesPerTask) void decode_mm_kernel(TiledP
   // columns w, w+4, w+8, w+12 of the group, each over LPC lanes of 8 dims
   constexpr int LPC = D / 8;           // lanes per column
   constexpr int CPP = kWave / LPC;     // columns per pass of the wave
+  constexpr int QN = SOLO ? kCols : kCols / kWavesPerTask;  // columns of the wave
+  constexpr int WN = SOLO ? 1 : kWavesPerTask;              // states they are merged from
+  const int w0 = SOLO ? wave : 0;
   auto& mg = lds.merge;
   const bool write_final = t.nsplit == 1;
 #pragma unroll
   for (int g = 0; g < CG; ++g) {
     const float lt = xor_sum<16>(l[g]);
-    __syncthreads();  // the V staging (g = 0) or the previous group's merge is done
+    // the V staging (g = 0) or the previous group's merge is done (a host
+    // worker wave keeps to its own parts of the LDS)
+    if (!SOLO) __syncthreads();
     if (CG > 1 || 4 * R < t.gcount) {  // rows of real columns
 #pragma unroll
       for (int c = 0; c < NC; ++c) {
@@ -382,30 +380,33 @@ __global__ __launch_bounds__(kWave * kWavesPerTask) void decode_mm_kernel(TiledP
       mg.l[wave][lane] = lt;
     }
     if (lane == 0) mg.bad[wave] = wb.bad ? 1 : 0;
-    __syncthreads();
+    if (SOLO)
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    else
+      __syncthreads();
 
     bool bad = false;
 #pragma unroll
-    for (int w = 0; w < kWavesPerTask; ++w) bad |= mg.bad[w] != 0;
+    for (int w = 0; w < WN; ++w) bad |= mg.bad[w0 + w] != 0;
 #pragma unroll
-    for (int pass = 0; pass < (4 + CPP - 1) / CPP; ++pass) {
-      const int q = pass * CPP + lane / LPC;  // which of the wave's 4 columns
-      if (q >= 4) break;
-      const int cc = wave + 4 * q;
+    for (int pass = 0; pass < (QN + CPP - 1) / CPP; ++pass) {
+      const int q = pass * CPP + lane / LPC;  // which of the wave's columns
+      if (q >= QN || (SOLO && pass * CPP >= t.gcount)) break;
+      const int cc = SOLO ? q : wave + 4 * q;
       const int d0 = (lane % LPC) * 8;
-      float M = mg.m[0][cc];
+      float M = mg.m[w0][cc];
 #pragma unroll
-      for (int w = 1; w < kWavesPerTask; ++w) M = fmaxf(M, mg.m[w][cc]);
+      for (int w = 1; w < WN; ++w) M = fmaxf(M, mg.m[w0 + w][cc]);
       const float Ms = M == neg_inf() ? 0.f : M;
       float ltot = 0.f, o[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) o[e] = 0.f;
 #pragma unroll
-      for (int w = 0; w < kWavesPerTask; ++w) {
-        const float sc = fast_exp2(mg.m[w][cc] - Ms);  // 0 for a wave without blocks
-        ltot += sc * mg.l[w][cc];
-        const float4 a = *reinterpret_cast<const float4*>(&mg.acc[w][cc][d0]);
-        const float4 b = *reinterpret_cast<const float4*>(&mg.acc[w][cc][d0 + 4]);
+      for (int w = 0; w < WN; ++w) {
+        const float sc = fast_exp2(mg.m[w0 + w][cc] - Ms);  // 0 for a wave without blocks
+        ltot += sc * mg.l[w0 + w][cc];
+        const float4 a = *reinterpret_cast<const float4*>(&mg.acc[w0 + w][cc][d0]);
+        const float4 b = *reinterpret_cast<const float4*>(&mg.acc[w0 + w][cc][d0 + 4]);
         o[0] += sc * a.x;
         o[1] += sc * a.y;
         o[2] += sc * a.z;
@@ -437,15 +438,60 @@ __global__ __launch_bounds__(kWave * kWavesPerTask) void decode_mm_kernel(TiledP
     }
   }
   // a balanced launch (one column group): the row's last task merges its parts
-  if constexpr (CG == 1) {
+  if constexpr (SOLO) {
+    end_solo_part<T, D>(p, t, lane);
+  } else if constexpr (CG == 1) {
     if (p.bal_parts == 0 || t.nsplit == 1) return;
-    if (last_to_arrive(p, t, &mg.last)) merge_parts<T, D>(p, t);
+    if (last_to_arrive(p, t, &mg.last)) merge_parts<T, D>(p, t, threadIdx.x, kWave * kWavesPerTask);
+  }
+}
+
+template <typename T, int D, int CG, bool TWO>
+__global__ __launch_bounds__(kWave * kWavesPerTask) void decode_mm_kernel(TiledParams p) {
+  __shared__ MmLds<D> lds;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  Task t;
+  if (!decode_task<kCols * CG, TWO, CG == 1>(p, t)) return;
+  if (t.nb == 0 || t.range_bad) {
+    if (t.split == 0 && wave == 0) write_empty<T, D, kCols * CG>(p, t, lane);
+    return;
+  }
+  mm_task<T, D, CG, TWO ? kBothTiers : kFirstTier>(p, t, lds, wave, lane);
+}
+
+// Two tiers with host workers (balanced_task in decode_tiled.h): the first
+// host_wgs workgroups' waves take tier 1's parts one after another, the other
+// workgroups a part of tier 0 each.
+template <typename T, int D>
+__global__ __launch_bounds__(kWave * kWavesPerTask) void decode_mm_tiers_kernel(TiledParams p) {
+  __shared__ MmLds<D> lds;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  Task t;
+  auto task = [&](int f, bool host) -> bool {
+    return balanced_task<kCols, true, true, 1>(p, t, f, host);  // at most 64 rows
+  };
+  if ((int)blockIdx.x < p.host_wgs) {
+    for (int f = (int)blockIdx.x * kWavesPerTask + wave; task(f, true);
+         f += kWavesPerTask * p.host_wgs)
+      mm_task<T, D, 1, kSecondTier>(p, t, lds, wave, lane);
+  } else {
+    if (!task((int)blockIdx.x - p.host_wgs, false)) return;
+    if (t.nb == 0 || t.range_bad) {
+      if (wave == 0) write_empty<T, D, kCols>(p, t, lane);
+      return;
+    }
+    mm_task<T, D, 1, kFirstTier>(p, t, lds, wave, lane);
   }
 }
 
 template <typename T, int D, int CG>
 hipError_t launch_dc(const TiledParams& tp, unsigned tasks, const SplitPlan& sp, bool two,
                      hipStream_t s) {
+  if constexpr (CG == 1) {
+    if (tp.host_wgs > 0) return launch_capped<&decode_mm_tiers_kernel<T, D>>(tp, tasks, sp, s);
+  }
   return two ? launch_capped<&decode_mm_kernel<T, D, CG, true>>(tp, tasks, sp, s)
              : launch_capped<&decode_mm_kernel<T, D, CG, false>>(tp, tasks, sp, s);
 }

@@ -193,7 +193,8 @@ __global__ __launch_bounds__(kWave) void decode_generic_kernel(GenericParams p) 
 //   FD_WAVE_BLOCKS=<b>   blocks per working wave (0: every wave works);
 //   FD_WG_CAP=<k>        at most k workgroups per CU (0: no cap);
 //   FD_BALANCE=<w>       balanced cuts aiming at w workgroups wherever they can be made
-//                        (0: none).
+//                        (0: none);
+//   FD_HOST_WGS=<w>      w workgroups for a host tier in pinned memory (0: none).
 // Like getenv, the first definition of a name counts.
 struct Tuning {
   const char* split_blocks = nullptr;
@@ -202,6 +203,7 @@ struct Tuning {
   const char* wave_blocks = nullptr;
   const char* wg_cap = nullptr;
   const char* balance = nullptr;
+  const char* host_wgs = nullptr;
 
   bool kernel_forced(const char* name) const {
     return kernel != nullptr && strcmp(kernel, name) == 0;
@@ -226,6 +228,7 @@ Tuning read_tuning() {
     else if (!t.wave_blocks && (v = value(s, "WAVE_BLOCKS"))) t.wave_blocks = v;
     else if (!t.wg_cap && (v = value(s, "WG_CAP"))) t.wg_cap = v;
     else if (!t.balance && (v = value(s, "BALANCE"))) t.balance = v;
+    else if (!t.host_wgs && (v = value(s, "HOST_WGS"))) t.host_wgs = v;
   }
   return t;
 }
@@ -478,6 +481,37 @@ constexpr double kBalMerge = 20.0;        // blocks one task streams in the time
 constexpr double kBalRates = 1.65;        // a task's own rate (45 GB/s) over a 256th of HBM's
 constexpr double kBalMinBlocks = 8.0;     // smallest part (4: 9.2 us instead of 9.1 above, 16: 10.5)
 
+// Fills in the cuts aiming at `want` workgroups; false where nothing can be cut.
+bool cut_balanced(SplitPlan& sp, const Tuning& tune, int32_t n, int32_t H, int32_t D,
+                  int32_t kv_tasks, int32_t wt, int32_t least, int32_t whole, int64_t want,
+                  int cus, int32_t host_wgs = 0) {
+  const int64_t parts = std::max<int64_t>(n, want / kv_tasks);
+  // parts the lengths can make at most: see balanced_task (a part holds at
+  // most kMaxSplitBlocks blocks), and a row of the table's width alone
+  const int64_t over = ((int64_t)n * wt + kMaxSplitBlocks - 1) / kMaxSplitBlocks;
+  const int64_t grid = std::min(std::max(parts, over) + n, (int64_t)n * ((wt + least - 1) / least));
+  if (grid <= n && host_wgs == 0) return false;  // no row can be cut
+  // host workers' parts: ceil(N1 P / waves) blocks, at most a wave's ids
+  int64_t slots = grid;
+  if (host_wgs > 0)
+    slots += std::max<int64_t>((kWavesPerTask * host_wgs + kv_tasks - 1) / kv_tasks,
+                               ((int64_t)n * wt + kMaxWaveBlocks - 1) / kMaxWaveBlocks) + n;
+  // a row's partials have 32-bit byte offsets, the grid divides as small_div does
+  if (slots * H * D >= (1 << 28) || slots * kv_tasks >= (1 << 22)) return false;
+  sp.bal_parts = (int32_t)parts;
+  sp.bal_min = least;
+  sp.bal_grid = (int32_t)grid;
+  sp.bal_slots = (int32_t)slots;
+  sp.host_wgs = host_wgs;
+  // (forced cuts, for comparison runs and tests, cut what they can)
+  sp.bal_whole = tune.balance != nullptr ? -kMaxBalBlocks : whole;
+  sp.bal_share = (float)(kBalRates * kv_tasks / cus);
+  const int64_t cap = (parts * kv_tasks + host_wgs + cus - 1) / cus;
+  sp.bal_cap = cap <= 4 ? (int32_t)cap : 0;
+  if (tune.wg_cap != nullptr && *tune.wg_cap != 0) sp.bal_cap = std::max(0, atoi(tune.wg_cap));
+  return true;
+}
+
 void plan_balanced(SplitPlan& sp, const Tuning& tune, int32_t n, int32_t H, int32_t D,
                    int32_t kv_tasks, int32_t G, int32_t wt, int32_t elt, int cus) {
   if (cus <= 0 || n <= 0 || n > kMaxBalRows || G > 16 || wt <= 0 || wt > kMaxBalBlocks) return;
@@ -494,23 +528,7 @@ void plan_balanced(SplitPlan& sp, const Tuning& tune, int32_t n, int32_t H, int3
     want = 5 * pairs <= 2LL * cus ? cus : 2LL * cus;
   }
   if (want <= 0 || pairs > kMaxBalPairs) return;
-  const int64_t parts = std::max<int64_t>(n, want / kv_tasks);
-  // parts the lengths can make at most: see balanced_task (a part holds at
-  // most kMaxSplitBlocks blocks), and a row of the table's width alone
-  const int64_t over = ((int64_t)n * wt + kMaxSplitBlocks - 1) / kMaxSplitBlocks;
-  const int64_t grid = std::min(std::max(parts, over) + n, (int64_t)n * ((wt + least - 1) / least));
-  if (grid <= n) return;  // no row can be cut
-  // a row's partials have 32-bit byte offsets, the grid divides as small_div does
-  if (grid * H * D >= (1 << 28) || grid * kv_tasks >= (1 << 22)) return;
-  sp.bal_parts = (int32_t)parts;
-  sp.bal_min = least;
-  sp.bal_grid = (int32_t)grid;
-  // (forced cuts, for comparison runs and tests, cut what they can)
-  sp.bal_whole = tune.balance != nullptr ? -kMaxBalBlocks : whole;
-  sp.bal_share = (float)(kBalRates * kv_tasks / cus);
-  const int64_t cap = (parts * kv_tasks + cus - 1) / cus;
-  sp.bal_cap = cap <= 4 ? (int32_t)cap : 0;
-  if (tune.wg_cap != nullptr && *tune.wg_cap != 0) sp.bal_cap = std::max(0, atoi(tune.wg_cap));
+  cut_balanced(sp, tune, n, H, D, kv_tasks, wt, least, whole, want, cus);
 }
 
 }  // namespace
@@ -706,9 +724,55 @@ size_t decode_workspace_bytes(const SplitPlan& sp, int32_t n, int32_t H, int32_t
   return parts * D * sizeof(float) + parts * sizeof(float) + 256;
 }
 
+// Host workers: two-tier launches of up to 64 rows (the lengths one wave
+// holds) on decode_mm_kernel's shapes. A CU returns its vector loads in order,
+// so tasks that read both tiers took about the sum of the HBM and link times;
+// with the host tier on 32 workgroups of its own the two overlap, and the HBM
+// parts are cut by the rows' lengths, not by tables that are as wide as the
+// whole context for both tiers. Measured (HIP graph replay, us; HBM + link
+// time in brackets), against the same build without workers: 64 x U[500, 1500],
+// 32/8, a host block each [38 + 40] 82 -> 66; 64/8, 2 % host [37 + 57] 98 -> 77; a
+// layer of 33 x U[40, 1800] with full-width tables 50 -> 42; 8 x 32 heads, 10 %
+// [10 + 119] 133 -> 127; with narrow tables 33 rows 35 -> 38; 24 rows 60 % host
+// [4 + 697] 685 -> 696. 16 workgroups are too few for one-block parts (33 rows:
+// 49), 48 take CUs from the HBM parts (64 rows: 70).
+bool plan_host_workers(SplitPlan& sp, int32_t n, int32_t H, int32_t KVH, int32_t D, int32_t BS,
+                       int32_t bt_width, int32_t kv_dtype) {
+  const int cus = device_cus();
+  const int32_t G = H / KVH;
+  // decode_mm_kernel's head sizes and groups (of those of 1 to 3 heads, which
+  // take the VALU kernel else, at D = 128)
+  if (!sp.fast || kv_dtype == FD_F32 || cus <= 0 || n <= 0 || n > kWave || bt_width <= 0 ||
+      G > 16 || !(sp.mm || (D == 128 && G < 4)))
+    return false;
+  const Tuning tune = read_tuning();
+  if ((tune.split_blocks != nullptr && atoi(tune.split_blocks) > 0) ||
+      (tune.balance != nullptr && atoi(tune.balance) <= 0) ||
+      (tune.kernel != nullptr && !tune.kernel_forced("mm")))
+    return false;
+  const int32_t wgs = tune.host_wgs != nullptr ? atoi(tune.host_wgs) : 32;
+  const int64_t wt = (int64_t)bt_width * (BS / kTileTokens);
+  const int64_t pairs = (int64_t)n * KVH;
+  if (wgs <= 0 || wt > kMaxBalBlocks || pairs > kMaxBalPairs) return false;
+  const double units = 2.0 * kTileTokens * D * 2 / kBalTileBytes;
+  int64_t want = (5 * pairs <= 2LL * cus ? cus : 2LL * cus) - wgs;
+  if (tune.balance != nullptr) want = atoi(tune.balance);
+  SplitPlan hw = sp;
+  if (!cut_balanced(hw, tune, n, H, D, KVH, (int32_t)wt,
+                    std::max(2, (int32_t)(kBalMinBlocks / units)), (int32_t)(kBalMerge / units),
+                    want, cus, wgs))
+    return false;
+  hw.mm = true;
+  hw.mfma = false;
+  hw.kernel_g = 16;
+  hw.passes = 1;
+  sp = hw;
+  return true;
+}
+
 size_t balanced_partial_bytes(const SplitPlan& sp, int32_t H, int32_t D) {
   if (sp.bal_parts <= 0) return 0;
-  const size_t parts = (size_t)sp.bal_grid * H;
+  const size_t parts = (size_t)sp.bal_slots * H;
   return (parts * (D + 1) * sizeof(float) + 255) / 256 * 256;
 }
 
@@ -812,13 +876,14 @@ int launch_decode(const DecodeArgs& a, const SplitPlan& sp, hipStream_t s) {
   const bool balanced = sp.bal_parts > 0;
   const size_t parts = (size_t)a.n * a.H * sp.max_splits;
   if (balanced) {
-    const size_t bparts = (size_t)sp.bal_grid * a.H;
+    const size_t bparts = (size_t)sp.bal_slots * a.H;
     tp.part_o = static_cast<float*>(a.workspace);
     tp.part_lse = tp.part_o + bparts * a.D;
     tp.bal_parts = sp.bal_parts;
     tp.bal_min = sp.bal_min;
     tp.bal_whole = sp.bal_whole;
     tp.bal_share = sp.bal_share;
+    tp.host_wgs = sp.host_wgs;
     tp.order = a.order;
     tp.wave_blocks = 0;
     tp.counters = a.counters;
@@ -836,7 +901,7 @@ int launch_decode(const DecodeArgs& a, const SplitPlan& sp, hipStream_t s) {
     tp.part_o = reinterpret_cast<float*>(ws);
     tp.part_lse = reinterpret_cast<float*>(ws + parts * a.D * sizeof(float));
   }
-  const int64_t tasks = balanced ? (int64_t)sp.bal_grid * a.KVH * sp.passes
+  const int64_t tasks = balanced ? (int64_t)sp.bal_grid * a.KVH * sp.passes + sp.host_wgs
                                  : (int64_t)a.n * a.KVH * sp.passes * sp.max_splits;
   if (tasks > INT32_MAX) return set_error(FD_ERR_UNSUPPORTED, "decode: too many tasks");
   if (a.timeline != nullptr && tasks > a.timeline_tasks)

@@ -84,6 +84,8 @@ struct TiledParams {
   int32_t bal_parts;  // > 0: balanced cuts (balanced_task()): parts per kv-head pass aimed at
   int32_t bal_min;    // balanced cuts: blocks per part at least
   int32_t bal_whole;  // balanced cuts: blocks a cut has to save (whole rows otherwise)
+  int32_t host_wgs;   // balanced cuts of two tiers: workgroups that take tier 1's blocks alone
+                      // (balanced_task()), 0: tasks over both tiers' blocks
   float bal_share;    // balanced cuts: blocks of one task's own rate in the time in which HBM
                       // delivers one block of every row of all kv-head passes together
   uint32_t* counters; // balanced cuts: arrivals per (sequence, kv-head pass), zero between launches
@@ -318,6 +320,16 @@ __device__ __forceinline__ int xcd_task(int b, int tasks) {
 // rows), or N / 256 + n when parts reach the 256 blocks a task can hold: the
 // grid's bound. Workgroups past the last part return.
 //
+// Two tiers, tier 1 over the link (p.host_wgs > 0): a CU returns vector loads
+// in order, so a wave that waits for the link holds up every HBM load of its
+// CU, and a launch whose tasks read both took about the sum of both times.
+// There the first host_wgs workgroups take all of tier 1's blocks, each of
+// their waves a part of its own at a time (adjacent waves adjacent kv heads
+// of the same blocks, one run in the host tier's layout), and the parts above
+// are cut from tier 0's blocks alone. A row's parts of both kinds merge the
+// same way. Parts of tier 1 hold ceil(N1 P / waves) blocks of its N1 blocks
+// and P kv-head passes, at most the 64 ids a wave holds.
+//
 // Every wave works the cut out by itself from the n lengths (one load per 64
 // rows, all in flight together, then DPP scans): the same chain of dependent
 // loads as a task with a dispatch order, lengths -> block ids -> K.
@@ -347,13 +359,13 @@ __device__ __forceinline__ int wave_max_int(int x) {  // of values >= 0
   return __builtin_amdgcn_readlane(x, kWave - 1);
 }
 
-// Blocks of a row of la / lb tokens (0 when a length is past its table: such
-// a row is one part, which writes its NaN).
+// Blocks of a row of la / lb tokens, of tier 0 alone or of both (0 when a
+// length is past its table: such a row is one part, which writes its NaN).
 template <bool TWO>
-__device__ __forceinline__ int row_blocks(const TiledParams& p, int la, int lb) {
+__device__ __forceinline__ int row_blocks(const TiledParams& p, int la, int lb, bool both) {
   if (la > p.tier[0].bt_width * p.BS || (TWO && lb > p.tier[1].bt_width * p.BS)) return 0;
   return (max(la, 0) + kTileTokens - 1) / kTileTokens +
-         (TWO ? (max(lb, 0) + kTileTokens - 1) / kTileTokens : 0);
+         (TWO && both ? (max(lb, 0) + kTileTokens - 1) / kTileTokens : 0);
 }
 
 // a / d for 0 <= a < 2^22 and d > 0, rcp = 1 / d within a few ulp: the
@@ -371,11 +383,16 @@ __device__ __forceinline__ float fast_rcp(int d) { return __builtin_amdgcn_rcpf(
 constexpr int kMaxBalBlocks = 1 << 20;  // table width of a balanced launch, in 16-token tiles
 constexpr int kBalTries = 6;            // part sizes tried
 
-template <int G, bool TWO, int kBalChunks>
-__device__ __forceinline__ bool balanced_task(const TiledParams& p, Task& t) {
+// Task f of a balanced launch: part f / P of kv-head pass f % P. TIERED: the
+// launch has host workers; tier 0's parts, or with `host` set tier 1's, their
+// blocks counted within the tier.
+template <int G, bool TWO, bool TIERED, int kBalChunks>
+__device__ __forceinline__ bool balanced_task(const TiledParams& p, Task& t, int f, bool host) {
   const int lane = threadIdx.x & (kWave - 1);
-  int row[kBalChunks], la[kBalChunks], lb[kBalChunks], nb[kBalChunks], parts[kBalChunks];
-  bool skips = false;  // the caller's order lists an entry outside [0, n)
+  static_assert(TWO || !TIERED, "host workers take a second tier");
+  int row[kBalChunks], la[kBalChunks], lb[kBalChunks];
+  int parts[kBalChunks];  // of the row's blocks (tiered: of tier 0's)
+  bool skips = false;     // the caller's order lists an entry outside [0, n)
 #pragma unroll
   for (int c = 0; c < kBalChunks; ++c) {
     row[c] = c * kWave + lane;
@@ -388,8 +405,8 @@ __device__ __forceinline__ bool balanced_task(const TiledParams& p, Task& t) {
     }
   }
   const int P = p.KVH * p.passes;
-  const int j = small_div(blockIdx.x, P, fast_rcp(P));  // part; kv-head passes run fastest
-  t.kp = blockIdx.x - j * P;
+  const int j = small_div(f, P, fast_rcp(P));  // part; kv-head passes run fastest
+  t.kp = f - j * P;
   const int pass = small_div(t.kp, p.KVH, fast_rcp(p.KVH));
   t.kh = t.kp - pass * p.KVH;
   t.h0 = t.kh * p.hpk + pass * G;
@@ -406,14 +423,25 @@ __device__ __forceinline__ bool balanced_task(const TiledParams& p, Task& t) {
     }
   }
   auto listed = [&](int c) -> bool { return (unsigned)row[c] < (unsigned)p.n; };
-  int sum = 0, longest = 0;
+  // blocks of lane's row of chunk c: those the parts are cut from, and tier
+  // 1's where it has parts of its own
+  auto blocks = [&](int c) -> int {
+    return listed(c) ? row_blocks<TWO>(p, la[c], lb[c], !TIERED) : 0;
+  };
+  auto host_blocks = [&](int c) -> int {
+    return TIERED && listed(c) && row_blocks<TWO>(p, la[c], lb[c], true) > 0
+               ? (max(lb[c], 0) + kTileTokens - 1) / kTileTokens
+               : 0;
+  };
+  int sum = 0, longest = 0, hsum = 0;
 #pragma unroll
   for (int c = 0; c < kBalChunks; ++c) {
-    nb[c] = parts[c] = 0;
+    parts[c] = 0;
     if (c == 0 || c * kWave < p.n) {
-      nb[c] = listed(c) ? row_blocks<TWO>(p, la[c], lb[c]) : 0;
-      sum += nb[c];
-      longest = max(longest, nb[c]);
+      const int nb = blocks(c);
+      sum += nb;
+      longest = max(longest, nb);
+      if constexpr (TIERED) hsum += host_blocks(c);
     }
   }
   const int total = __builtin_amdgcn_readlane(wave_scan(sum), kWave - 1);
@@ -434,7 +462,9 @@ __device__ __forceinline__ bool balanced_task(const TiledParams& p, Task& t) {
 #pragma unroll
     for (int c = 0; c < kBalChunks; ++c) {
       if (c == 0 || c * kWave < p.n) {
-        parts[c] = listed(c) ? max(1, small_div(nb[c] + size - 1, size, rcp)) : 0;
+        // (a row all in tier 1 has no part of tier 0; an empty one has one part)
+        const int least = listed(c) && (!TIERED || host_blocks(c) == 0) ? 1 : 0;
+        parts[c] = max(least, small_div(blocks(c) + size - 1, size, rcp));
         count += parts[c];
       }
     }
@@ -443,31 +473,53 @@ __device__ __forceinline__ bool balanced_task(const TiledParams& p, Task& t) {
     const float grow = (float)size * (float)(all - want) * __builtin_amdgcn_rcpf((float)want);
     size = __builtin_amdgcn_readfirstlane(min(size + 1 + (int)(0.5f * grow), kMaxSplitBlocks));
   }
-  int base = 0;  // parts of the rows before chunk c
+  int hsize = 1;  // tier 1's blocks per part
+  if constexpr (TIERED) {
+    const int htotal = __builtin_amdgcn_readlane(wave_scan(hsum), kWave - 1);
+    hsize = (int)((float)htotal * (float)P *
+                  __builtin_amdgcn_rcpf((float)(kWavesPerTask * p.host_wgs))) + 1;
+    hsize = __builtin_amdgcn_readfirstlane(min(max(hsize, 1), kMaxWaveBlocks));
+  }
+  const float hrcp = fast_rcp(hsize);
+  int base = 0, hbase = 0;  // parts of the rows before chunk c, of either kind
 #pragma unroll
   for (int c = 0; c < kBalChunks; ++c) {
     if (c > 0 && c * kWave >= p.n) break;
+    const int nh = TIERED ? host_blocks(c) : 0;
+    const int hparts = TIERED ? small_div(nh + hsize - 1, hsize, hrcp) : 0;
     const int upto = base + wave_scan(parts[c]);  // parts up to and with this lane's row
+    const int hupto = TIERED ? hbase + wave_scan(hparts) : 0;
     const int end = __builtin_amdgcn_readlane(upto, kWave - 1);
-    if (j < end) {
-      const int at = __popcll(__ballot(upto <= j));  // the lane of part j's row
+    const int hend = TIERED ? __builtin_amdgcn_readlane(hupto, kWave - 1) : 0;
+    if (j < (host ? hend : end)) {
+      // the lane of part j's row
+      const int at = __popcll(host ? __ballot(hupto <= j) : __ballot(upto <= j));
       t.i = __builtin_amdgcn_readlane(row[c], at);
       t.la = __builtin_amdgcn_readlane(la[c], at);
       t.lb = __builtin_amdgcn_readlane(lb[c], at);
-      t.nb = __builtin_amdgcn_readlane(nb[c], at);
-      t.nsplit = __builtin_amdgcn_readlane(parts[c], at);
-      t.slot0 = __builtin_amdgcn_readlane(upto, at) - t.nsplit;
-      t.split = j - t.slot0;
       t.nba = t.la > 0 ? (t.la + kTileTokens - 1) / kTileTokens : 0;
-      // the row's first `more` parts hold one block more than the others
-      const int each = small_div(t.nb, t.nsplit, fast_rcp(t.nsplit));
-      const int more = t.nb - each * t.nsplit;
-      t.b_begin = t.split * each + min(t.split, more);
-      t.b_end = t.b_begin + each + (t.split < more ? 1 : 0);
+      const int np = __builtin_amdgcn_readlane(parts[c], at);
+      const int nhp = TIERED ? __builtin_amdgcn_readlane(hparts, at) : 0;
+      const int first = __builtin_amdgcn_readlane(upto, at) - np;
+      const int hfirst = TIERED ? __builtin_amdgcn_readlane(hupto, at) - nhp : 0;
+      const int nbh = TIERED ? __builtin_amdgcn_readlane(nh, at) : 0;
+      const int nb0 = __builtin_amdgcn_readlane(blocks(c), at);  // blocks the np parts are cut from
+      t.nb = nb0 + nbh;
+      t.nsplit = np + nhp;
+      t.slot0 = first + hfirst;
+      const int k = host ? j - hfirst : j - first;
+      const int of = host ? nhp : np, nbk = host ? nbh : nb0;
+      t.split = host ? np + k : k;
+      // the first `more` parts hold one block more than the others
+      const int each = small_div(nbk, of, fast_rcp(of));
+      const int more = nbk - each * of;
+      t.b_begin = k * each + min(k, more);
+      t.b_end = t.b_begin + each + (k < more ? 1 : 0);
       t.range_bad = t.la > p.tier[0].bt_width * p.BS || (TWO && t.lb > p.tier[1].bt_width * p.BS);
       return true;
     }
     base = end;
+    hbase = hend;
   }
   return false;
 }
@@ -476,7 +528,8 @@ __device__ __forceinline__ bool balanced_task(const TiledParams& p, Task& t) {
 template <int G, bool TWO, bool BAL = true>
 __device__ __forceinline__ bool decode_task(const TiledParams& p, Task& t) {
   if (BAL && p.bal_parts > 0)
-    return p.n <= kWave ? balanced_task<G, TWO, 1>(p, t) : balanced_task<G, TWO, kBalChunks>(p, t);
+    return p.n <= kWave ? balanced_task<G, TWO, false, 1>(p, t, blockIdx.x, false)
+                        : balanced_task<G, TWO, false, kBalChunks>(p, t, blockIdx.x, false);
   const int task = p.xcd_group ? xcd_task(blockIdx.x, gridDim.x) : (int)blockIdx.x;
   t.kh = task % p.KVH;
   int rest = task / p.KVH;
@@ -506,9 +559,15 @@ __device__ __forceinline__ bool decode_task(const TiledParams& p, Task& t) {
   return true;
 }
 
+// Which of the launch's tiers a task's blocks lie in (the kernels' TWO, false
+// or true, is the first or second).
+enum TierSet { kFirstTier = 0, kBothTiers = 1, kSecondTier = 2 };
+
 // Valid tokens of the row's block u (< 16 only for the last block of a tier).
-template <bool TWO>
+template <int TS>
 __device__ __forceinline__ int block_tokens(const Task& t, int u) {
+  constexpr bool TWO = TS == kBothTiers;
+  if (TS == kSecondTier) return min(kTileTokens, t.lb - u * kTileTokens);
   if (TWO && u >= t.nba) return min(kTileTokens, t.lb - (u - t.nba) * kTileTokens);
   return min(kTileTokens, t.la - u * kTileTokens);
 }
@@ -550,12 +609,18 @@ struct WaveBlocks {
 // each about that many blocks (at least one, at most four); the rest only
 // take part in the merge. A short row then keeps fewer blocks in flight than
 // a long one.
-template <bool TWO>
+// A host worker wave (TS == kSecondTier) has its task to itself.
+template <int TS>
 __device__ __forceinline__ WaveBlocks wave_blocks(const TiledParams& p, const Task& t, int wave,
                                                   int lane) {
+  constexpr bool TWO = TS == kBothTiers;
   WaveBlocks w;
   int ws = kWavesPerTask;
-  if (p.wave_blocks > 0) {
+  if (TS == kSecondTier) {
+    ws = 1;
+    wave = 0;
+  }
+  if (TS != kSecondTier && p.wave_blocks > 0) {
     // (each wave's block ids fit its 64 lanes: nblk <= split_blocks <= 256)
     const int nblk = t.b_end - t.b_begin;
     ws = max((nblk + p.wave_blocks - 1) / p.wave_blocks,
@@ -601,7 +666,7 @@ __device__ __forceinline__ WaveBlocks wave_blocks(const TiledParams& p, const Ta
       sub = ut % p.tpb;
       my_bad = bid < 0 || (int64_t)bid >= tp.num_blocks;
     } else {
-      const TierParams& tp = p.tier[0];
+      const TierParams& tp = p.tier[TS == kSecondTier ? 1 : 0];
       bid = tp.bt[(int64_t)t.i * tp.bt_stride + u / p.tpb];
       sub = u % p.tpb;
       my_bad = bid < 0 || (int64_t)bid >= tp.num_blocks;
@@ -762,6 +827,17 @@ __device__ __forceinline__ void finish_task(const TiledParams& p, const Task& t,
 }
 
 
+// Counts one part of a row as written; true for the row's last, which leaves
+// the counter at zero. One thread.
+__device__ __forceinline__ bool count_arrival(const TiledParams& p, const Task& t) {
+  uint32_t* c = p.counters + (int64_t)t.i * p.KVH * p.passes + t.kp;
+  const uint32_t before =
+      __hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const bool done = before == (uint32_t)t.nsplit - 1;
+  if (done) __hip_atomic_store(c, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return done;
+}
+
 // Whether the tasks of this row still to come leave the merge to this one: a
 // balanced launch has no combine pass; the last of a row's parts to arrive
 // merges them. Called by the whole workgroup once its partial is written;
@@ -773,33 +849,27 @@ __device__ __forceinline__ void finish_task(const TiledParams& p, const Task& t,
 __device__ __forceinline__ bool last_to_arrive(const TiledParams& p, const Task& t, int* last) {
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's partial stores are done
   __syncthreads();
-  if (threadIdx.x == 0) {
-    uint32_t* c = p.counters + (int64_t)t.i * p.KVH * p.passes + t.kp;
-    const uint32_t before =
-        __hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const bool done = before == (uint32_t)t.nsplit - 1;
-    if (done) __hip_atomic_store(c, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    *last = done ? 1 : 0;
-  }
+  if (threadIdx.x == 0) *last = count_arrival(p, t) ? 1 : 0;
   __syncthreads();
   return __builtin_amdgcn_readfirstlane(*last) != 0;
 }
 
-// Merges the row's parts and writes its result (the whole workgroup of the
-// row's last task): a thread takes 4 dims of a head and folds the parts in
+// Merges the row's parts and writes its result (thread `tid` of `threads`: the
+// workgroup, or host worker wave, of the row's last task): a thread takes 4 dims of a head and folds the parts in
 // order, kPartsInFlight of them read together, as each round of reads is a
 // trip past the L2. The order is fixed, whichever task arrives last.
 constexpr int kPartsInFlight = 8;
 
 template <typename T, int D>
-__device__ __forceinline__ void merge_parts(const TiledParams& p, const Task& t) {
+__device__ __forceinline__ void merge_parts(const TiledParams& p, const Task& t, int tid,
+                                            int threads) {
   constexpr int LPT = D / 4;  // threads per head
   const int64_t first = (int64_t)t.slot0 * p.H + t.h0;
   const __amdgpu_buffer_rsrc_t ro =
       part_rsrc(p.part_o + first * p.D, ((int64_t)(t.nsplit - 1) * p.H + t.gcount) * p.D);
   const __amdgpu_buffer_rsrc_t rl =
       part_rsrc(p.part_lse + first, (int64_t)(t.nsplit - 1) * p.H + t.gcount);
-  for (int it = threadIdx.x; it < t.gcount * LPT; it += kWave * kWavesPerTask) {
+  for (int it = tid; it < t.gcount * LPT; it += threads) {
     const int g = it / LPT;
     const int d0 = (it % LPT) * 4;
     if (d0 >= p.D) continue;
@@ -856,7 +926,19 @@ __device__ __forceinline__ void end_task(const TiledParams& p, const Task& t, Wa
   __syncthreads();
   if (wave == 0) finish_task<T, D, G>(p, t, ws, lane);
   if (p.bal_parts == 0 || t.nsplit == 1) return;
-  if (last_to_arrive(p, t, &ws.last)) merge_parts<T, D>(p, t);
+  if (last_to_arrive(p, t, &ws.last))
+    merge_parts<T, D>(p, t, threadIdx.x, kWave * kWavesPerTask);
+}
+
+// After a host worker wave's part is written: merges the row if it was the
+// row's last.
+template <typename T, int D>
+__device__ __forceinline__ void end_solo_part(const TiledParams& p, const Task& t, int lane) {
+  if (t.nsplit == 1) return;
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), as in last_to_arrive
+  int last = 0;
+  if (lane == 0) last = count_arrival(p, t) ? 1 : 0;
+  if (__builtin_amdgcn_readfirstlane(last) != 0) merge_parts<T, D>(p, t, lane, kWave);
 }
 
 // Query head of the task's head slot g: slots past the task's heads repeat
@@ -880,10 +962,11 @@ struct BlockSrc {
 // rows with one host block each, 2.2 -> 1.2 MB over the link). In HBM the
 // extra scalar work per block costs more than the bytes (full batch of 256
 // grouped-query rows: 387 -> 401 us), so tier 0 keeps whole blocks.
-template <bool TWO>
+template <int TS>
 __device__ __forceinline__ BlockSrc block_src(const TiledParams& p, const WaveBlocks& wb,
                                               const Task& t, int k) {
-  const bool t1 = TWO && k >= wb.k1;
+  constexpr bool TWO = TS != kFirstTier;
+  const bool t1 = TS == kSecondTier || (TS == kBothTiers && k >= wb.k1);
   const int bid = __builtin_amdgcn_readlane(wb.my_bid, k);
   const int sub = __builtin_amdgcn_readlane(wb.my_sub, k);
   const TierParams& a = p.tier[0];
@@ -892,7 +975,7 @@ __device__ __forceinline__ BlockSrc block_src(const TiledParams& p, const WaveBl
                        (int64_t)sub * kTileTokens * (t1 ? b.st : a.st);
   uint32_t cut = 0;  // bytes of the block's rows past its tokens
   if (t1)
-    cut = (uint32_t)(kTileTokens - block_tokens<TWO>(t, wb.first + wb.stride * k)) *
+    cut = (uint32_t)(kTileTokens - block_tokens<TS>(t, wb.first + wb.stride * k)) *
           (uint32_t)b.st * 2;
   BlockSrc s;
   s.k = make_rsrc((t1 ? b.k : a.k) + base, (t1 ? b.k_run_bytes : a.k_run_bytes) - cut);

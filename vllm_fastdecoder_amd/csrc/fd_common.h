@@ -276,6 +276,8 @@ struct SplitPlan {
   int32_t bal_min;       // 16-token tiles per part at least,
   int32_t bal_grid;      // the parts the grid holds per kv-head pass,
   int32_t bal_cap;       // its wg_cap,
+  int32_t bal_slots;     // partials per query head (the grid's parts, and host workers'),
+  int32_t host_wgs;      // workgroups that take tier 1's blocks alone (two tiers; 0: none),
   int32_t bal_whole;     // and balanced_task's figures for leaving rows whole
   float bal_share;
   int* occupancy_query;  // planner only: when set, the tiled launchers store the selected
@@ -289,6 +291,10 @@ struct SplitPlan {
 SplitPlan plan_decode(int32_t n, int32_t H, int32_t KVH, int32_t D, int32_t BS,
                       int32_t bt_width, int32_t kv_dtype, bool aligned, bool matrix = true,
                       double fill = 0.0);
+// The plan of a two-tier launch with tier 1, in pinned host memory, on
+// workgroups of its own; false, with sp unchanged, where that does not apply.
+bool plan_host_workers(SplitPlan& sp, int32_t n, int32_t H, int32_t KVH, int32_t D, int32_t BS,
+                       int32_t bt_width, int32_t kv_dtype);
 size_t decode_workspace_bytes(const SplitPlan& sp, int32_t n, int32_t H,
                               int32_t D);
 // Workspace of a plan's balanced launch (0 when it has none): the partials,
