@@ -187,3 +187,40 @@ def test_entry_points_without_counters(gpu):
         if size:
             assert torch.equal(out, ref[0]) and torch.equal(lse, ref[1])
         _check(case, out, lse)
+
+
+@pytest.mark.parametrize("native", [True, False])
+def test_graphs_that_share_an_unreserved_workspace(gpu, native, monkeypatch):
+    """Two graphs captured on one stream with no workspace reserved: the second
+    uses the buffer the first capture allocated, and is replayed first, then
+    in turn with eager calls on that stream; every result is the eager one."""
+    if not native:
+        monkeypatch.setattr(ops, "_NATIVE", False)
+    case = _case([900, 2500, 64, 700], 32, 8, 128, torch.bfloat16, seed=21)
+    q, kc, vc, bt, lens = (x.to(gpu) for x in case)
+    outs = [(torch.empty(4, 32, 128, device=gpu), torch.empty(32, 4, device=gpu)) for _ in range(3)]
+
+    def step(k):
+        ops.decode_attn(q, kc, vc, bt, lens, 1 / math.sqrt(128), *outs[k])
+        kv = kc.transpose(1, 2), vc.transpose(1, 2)
+        ops.paged_decode(q, *kv, bt, lens, 1 / math.sqrt(128), out=outs[k][0], lse=outs[k][1])
+
+    step(2)
+    torch.cuda.synchronize()
+    ref = [t.clone() for t in outs[2]]
+    side = torch.cuda.Stream(device=gpu)
+    graphs = [torch.cuda.CUDAGraph() for _ in range(2)]
+    for k, g in enumerate(graphs):
+        with torch.cuda.graph(g, stream=side):
+            step(k)
+    for k in (1, 0, 1, 2, 1, 0):
+        for t in (t for pair in outs for t in pair):
+            t.fill_(7.0)
+        if k < 2:
+            graphs[k].replay()
+        else:
+            torch.cuda.synchronize()
+            with torch.cuda.stream(side):
+                step(2)
+        torch.cuda.synchronize()
+        assert torch.equal(outs[k][0], ref[0]) and torch.equal(outs[k][1], ref[1]), k

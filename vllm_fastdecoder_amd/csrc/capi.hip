@@ -260,12 +260,15 @@ int fd_decode_workspace_need(int32_t n, int32_t num_heads, int32_t num_kv_heads,
   const SplitPlan sp = plan_decode(n, num_heads, num_kv_heads, head_size, block_size, bt_width,
                                    kv_dtype, true, host_tier == 0,
                                    row_fill(total_tokens, n, bt_width, block_size));
-  *bytes = sp.bal_parts > 0 ? balanced_partial_bytes(sp, num_heads, head_size)
+  // (with room for counters, should the caller have none beside its workspace)
+  *bytes = sp.bal_parts > 0 ? balanced_partial_bytes(sp, num_heads, head_size) +
+                                  balanced_counter_bytes(sp, n, num_kv_heads)
                             : decode_workspace_bytes(sp, n, num_heads, head_size);
   SplitPlan hw = sp;
   if (host_tier != 0 && plan_host_workers(hw, n, num_heads, num_kv_heads, head_size, block_size,
                                           bt_width, kv_dtype))
-    *bytes = std::max(*bytes, balanced_partial_bytes(hw, num_heads, head_size));
+    *bytes = std::max(*bytes, balanced_partial_bytes(hw, num_heads, head_size) +
+                                  balanced_counter_bytes(hw, n, num_kv_heads));
   return FD_OK;
 }
 

@@ -102,8 +102,8 @@ bool current_stream(int64_t idx, void** stream) {
 }
 
 // The stream's workspace of at least `need` bytes and the counters behind it
-// (ops._counters_ptr: on the next 256-byte boundary); `hold` keeps it alive
-// over the launch. False with a Python error set.
+// (ops._counters_ptr: on the next 256-byte boundary, where the buffer has
+// them); `hold` keeps it alive over the launch. False with a Python error set.
 bool workspace(const at::Tensor& q, size_t need, PyRef& hold, void** ws, size_t* bytes,
                uint32_t** counters) {
   *ws = nullptr;
@@ -119,7 +119,9 @@ bool workspace(const at::Tensor& q, size_t need, PyRef& hold, void** ws, size_t*
   const at::Tensor& buf = THPVariable_Unpack(hold.p);
   *ws = buf.data_ptr();
   *bytes = (size_t)buf.numel();
-  *counters = reinterpret_cast<uint32_t*>(static_cast<char*>(*ws) + (*bytes + 255) / 256 * 256);
+  const size_t head = (*bytes + 255) / 256 * 256;
+  if (buf.storage().nbytes() >= head + 4 * FD_DECODE_COUNTERS)
+    *counters = reinterpret_cast<uint32_t*>(static_cast<char*>(*ws) + head);
   return true;
 }
 

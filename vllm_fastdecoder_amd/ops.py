@@ -139,12 +139,17 @@ class _Workspace:
     def _allocate(key: tuple[int, int], nbytes: int) -> torch.Tensor:
         """nbytes of scratch followed, on the next 256-byte boundary, by the
         stream's arrival counters (fd_paged_decode_counted), cleared on the
-        stream that will use them."""
+        stream that will use them. Without the counters under a stream
+        capture: the clearing would only be recorded, and another graph, or an
+        eager call, could use them before the graph that holds it has run
+        (launches then clear counters of their own in the workspace)."""
         device, stream = key
         head = _counters_offset(nbytes)
         size = head + 4 * _lib.DECODE_COUNTERS
 
         def make():
+            if torch.cuda.is_current_stream_capturing():
+                return torch.empty(nbytes, dtype=torch.uint8, device=torch.device("cuda", device))
             t = torch.empty(size, dtype=torch.uint8, device=torch.device("cuda", device))
             t[head:].zero_()
             return t[:nbytes]
@@ -166,8 +171,13 @@ def _counters_offset(nbytes: int) -> int:
 
 
 def _counters_ptr(buf: torch.Tensor | None) -> int | None:
-    """The arrival counters behind a buffer of WORKSPACE."""
-    return None if buf is None else buf.data_ptr() + _counters_offset(buf.numel())
+    """The arrival counters behind a buffer of WORKSPACE, where it has them."""
+    if buf is None:
+        return None
+    head = _counters_offset(buf.numel())
+    if buf.untyped_storage().nbytes() < head + 4 * _lib.DECODE_COUNTERS:
+        return None
+    return buf.data_ptr() + head
 
 
 WORKSPACE = _Workspace()
