@@ -191,9 +191,9 @@ def test_entry_points_without_counters(gpu):
 
 @pytest.mark.parametrize("native", [True, False])
 def test_graphs_that_share_an_unreserved_workspace(gpu, native, monkeypatch):
-    """Two graphs captured on one stream with no workspace reserved: the second
-    uses the buffer the first capture allocated, and is replayed first, then
-    in turn with eager calls on that stream; every result is the eager one."""
+    """Two graphs captured on one stream with no workspace reserved, so each
+    with scratch of its own: the second is replayed first, then they are in
+    turn with eager calls on that stream; every result is the eager one."""
     if not native:
         monkeypatch.setattr(ops, "_NATIVE", False)
     case = _case([900, 2500, 64, 700], 32, 8, 128, torch.bfloat16, seed=21)
@@ -224,3 +224,51 @@ def test_graphs_that_share_an_unreserved_workspace(gpu, native, monkeypatch):
                 step(2)
         torch.cuda.synchronize()
         assert torch.equal(outs[k][0], ref[0]) and torch.equal(outs[k][1], ref[1]), k
+
+
+@pytest.mark.parametrize("native", [True, False])
+def test_unreserved_graphs_keep_their_scratch(gpu, native, monkeypatch):
+    """Two graphs captured on one stream without a reservation, rows cut by
+    length: a larger eager call grows the stream's workspace, fresh tensors
+    take whatever memory that freed, and both graphs replay at once on two
+    streams. They write into none of those tensors and give the eager bits."""
+    if not native:
+        monkeypatch.setattr(ops, "_NATIVE", False)
+    case = _case([900, 2500, 64, 700], 32, 8, 128, torch.bfloat16, seed=22)
+    q, kc, vc, bt, lens = (x.to(gpu) for x in case)
+    kv = kc.transpose(1, 2), vc.transpose(1, 2)
+    outs = [(torch.empty(4, 32, 128, device=gpu), torch.empty(32, 4, device=gpu)) for _ in range(3)]
+
+    def step(k, rep=1):
+        out, lse = outs[k] if rep == 1 else (None, None)
+        ops.paged_decode(q.repeat(rep, 1, 1), *kv, bt.repeat(rep, 1), lens.repeat(rep),
+                         1 / math.sqrt(128), out=out, lse=lse)
+
+    side, other = (torch.cuda.Stream(device=gpu) for _ in range(2))
+    with torch.cuda.stream(side):
+        step(2)
+    torch.cuda.synchronize()
+    ref = [t.clone() for t in outs[2]]
+    graphs = [torch.cuda.CUDAGraph() for _ in range(2)]
+    for k, g in enumerate(graphs):
+        with torch.cuda.graph(g, stream=side):
+            step(k)
+    size = ops.workspace_bytes(4, 32, 8, 128, 16, bt.shape[1])
+    with torch.cuda.stream(side):
+        step(2, rep=4)
+        assert ops.workspace_bytes(16, 32, 8, 128, 16, bt.shape[1]) > size
+        markers = [torch.full((size + 4 * _lib.DECODE_COUNTERS,), 77, dtype=torch.uint8, device=gpu)
+                   for _ in range(8)]
+    torch.cuda.synchronize()
+    for _ in range(3):
+        for pair in outs[:2]:
+            for t in pair:
+                t.fill_(7.0)
+        torch.cuda.synchronize()
+        for s, g in zip((side, other), graphs):
+            with torch.cuda.stream(s):
+                g.replay()
+        torch.cuda.synchronize()
+        for pair in outs[:2]:
+            assert torch.equal(pair[0], ref[0]) and torch.equal(pair[1], ref[1])
+        assert all(bool((m == 77).all()) for m in markers)

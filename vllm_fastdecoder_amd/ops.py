@@ -96,7 +96,11 @@ class _Workspace:
     capture): a captured graph keeps the raw address of the buffer its
     launches were given, so a pinned stream's buffers are never dropped,
     neither by the eviction above nor when growth replaces one, until the
-    reservation is released (release_workspace)."""
+    reservation is released (release_workspace). A launch captured on a stream
+    that is not pinned gets scratch of its own instead, allocated from the
+    graph's memory pool like any tensor of the captured code: it lives as long
+    as the graph, no other call is ever given it, and growth, eviction and
+    other graphs of the same stream leave it alone."""
 
     def __init__(self, max_streams: int = 16) -> None:
         self._bufs: dict[tuple[int, int], torch.Tensor] = {}
@@ -118,6 +122,10 @@ class _Workspace:
         if nbytes == 0 and not pin:
             return None
         key = self._key(device, stream)
+        if not pin and _capturing() and key not in self._pinned:
+            # (freed when the caller drops it, to the pool that torch keeps for
+            # this graph: only its later captured work uses that)
+            return self._allocate(key, nbytes)
         with self._lock:
             buf = self._bufs.pop(key, None)  # re-inserted below: most recent last
             if buf is None or buf.numel() < nbytes:
@@ -140,15 +148,14 @@ class _Workspace:
         """nbytes of scratch followed, on the next 256-byte boundary, by the
         stream's arrival counters (fd_paged_decode_counted), cleared on the
         stream that will use them. Without the counters under a stream
-        capture: the clearing would only be recorded, and another graph, or an
-        eager call, could use them before the graph that holds it has run
-        (launches then clear counters of their own in the workspace)."""
+        capture, where the clearing would only be recorded (launches then
+        clear counters of their own in the workspace)."""
         device, stream = key
         head = _counters_offset(nbytes)
         size = head + 4 * _lib.DECODE_COUNTERS
 
         def make():
-            if torch.cuda.is_current_stream_capturing():
+            if _capturing():
                 return torch.empty(nbytes, dtype=torch.uint8, device=torch.device("cuda", device))
             t = torch.empty(size, dtype=torch.uint8, device=torch.device("cuda", device))
             t[head:].zero_()
@@ -164,6 +171,15 @@ class _Workspace:
         (and may be evicted again)."""
         with self._lock:
             self._pinned.pop(self._key(device, stream), None)
+
+
+_IS_CAPTURING = getattr(torch._C, "_cuda_isCurrentStreamCapturing", None)
+
+
+def _capturing() -> bool:
+    """Whether the current stream records a graph (the raw query: this is
+    asked on every call that takes a workspace)."""
+    return _IS_CAPTURING is not None and _IS_CAPTURING()
 
 
 def _counters_offset(nbytes: int) -> int:
@@ -218,8 +234,9 @@ def reserve_workspace(stream: torch.cuda.Stream, nbytes: int) -> torch.Tensor:
     (workspace_bytes of the largest shape to come), and pins it. For HIP
     graph capture: torch.cuda.graph captures on its own stream, so a
     workspace reserved for that stream before capture keeps the captured
-    launches from allocating (otherwise the first captured launch of a shape
-    that splits rows allocates it from the graph's memory pool). The graph
+    launches from allocating (otherwise each captured launch that needs a
+    workspace allocates its own from the graph's memory pool, and clears its
+    arrival counters in a launch of its own). The graph
     keeps the buffer's raw address, so while the reservation holds, the
     buffer is neither evicted nor freed when a later, larger call on the
     same stream grows the workspace. Returns the buffer; call
