@@ -135,6 +135,22 @@ def test_order_entries_outside_the_rows_are_skipped(gpu, monkeypatch):
     assert torch.all(out[[1, 2]] == 7.0) and torch.all(lse[:, [1, 2]] == 7.0)
 
 
+@pytest.mark.parametrize("H,KVH,D", [(8, 2, 128), (2, 2, 128), (8, 2, 256)])
+def test_a_row_listed_twice_beside_a_skipped_entry(gpu, H, KVH, D, monkeypatch):
+    """Each listing is cut and merged by itself; the launches after it are
+    whole again."""
+    monkeypatch.setenv("FD_BALANCE", "64")
+    case = _case([900, 500, 64, 700, 0], H, KVH, D, torch.bfloat16, seed=13)
+    for _ in range(3):
+        out = torch.full((5, H, D), 7.0, device=gpu)
+        lse = torch.full((H, 5), 7.0, device=gpu)
+        _run(case, gpu, out, lse, row_order=torch.tensor([3, -1, 3, 0, 0], dtype=torch.int32))
+        _check(case, out, lse, rows=[0, 3])
+        rest = [1, 2, 4]
+        assert torch.all(out[rest] == 7.0) and torch.all(lse[:, rest] == 7.0)
+        _check(case, *_run(case, gpu))
+
+
 def test_range_errors_stay_in_their_rows(gpu, monkeypatch):
     """A bad block id and a length past the table: NaN in those rows only."""
     monkeypatch.setenv("FD_BALANCE", "96")

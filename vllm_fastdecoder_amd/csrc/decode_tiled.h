@@ -274,7 +274,8 @@ struct Task {
   int nba, nb;
   int b_begin, b_end, nsplit;
   bool range_bad;  // a length needs more blocks than its table has
-  int kp, slot0;   // balanced cuts: kv-head pass of the task, first part of its row
+  int kp, slot0;   // balanced cuts: kv-head pass of the task, first part of its row,
+  int pos;         // and the row's place in the launch's list of rows
 };
 
 // blockIdx.x -> task: kv head fastest, then head group (one unless a kv head
@@ -495,6 +496,7 @@ __device__ __forceinline__ bool balanced_task(const TiledParams& p, Task& t, int
       // the lane of part j's row
       const int at = __popcll(host ? __ballot(hupto <= j) : __ballot(upto <= j));
       t.i = __builtin_amdgcn_readlane(row[c], at);
+      t.pos = c * kWave + at;
       t.la = __builtin_amdgcn_readlane(la[c], at);
       t.lb = __builtin_amdgcn_readlane(lb[c], at);
       t.nba = t.la > 0 ? (t.la + kTileTokens - 1) / kTileTokens : 0;
@@ -828,9 +830,11 @@ __device__ __forceinline__ void finish_task(const TiledParams& p, const Task& t,
 
 
 // Counts one part of a row as written; true for the row's last, which leaves
-// the counter at zero. One thread.
+// the counter at zero. One thread. Rows are counted by their place in the
+// launch's list: an order with entries outside [0, n) may list a row twice,
+// and each listing is cut, counted and merged by itself.
 __device__ __forceinline__ bool count_arrival(const TiledParams& p, const Task& t) {
-  uint32_t* c = p.counters + (int64_t)t.i * p.KVH * p.passes + t.kp;
+  uint32_t* c = p.counters + (int64_t)t.pos * p.KVH * p.passes + t.kp;
   const uint32_t before =
       __hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   const bool done = before == (uint32_t)t.nsplit - 1;
