@@ -168,13 +168,16 @@ int fd_paged_decode_partial_hint(
     void* workspace, size_t workspace_bytes,
     void* stream, int64_t total_tokens);
 
-/* Entries of the arrival-counter array below. */
+/* uint32 words of the arrival-counter array below. */
 #define FD_DECODE_COUNTERS 4096
 
 /* fd_paged_decode_partial_hint for a caller that keeps arrival counters
- * beside its workspace: a device array of FD_DECODE_COUNTERS uint32, all zero
- * before its first call (every call leaves it zero). Launches that may
- * overlap need one each, like the workspace. Launches whose rows are cut by
+ * beside its workspace: a device array of FD_DECODE_COUNTERS uint32 (8-byte
+ * aligned; ignored where it is not), all zero before its first call and the
+ * library's from then on. Launches that may overlap need one each, like the
+ * workspace; what an overlap leaves there reaches no later launch (only
+ * replays of a graph captured before it, until the array is cleared or an
+ * ungraphed launch has used it). Launches whose rows are cut by
  * their lengths count each row's finished tasks there, so that the last one
  * merges the row; without the array (the other entry points, or NULL) such a
  * launch takes the counters from its workspace and clears them with a small

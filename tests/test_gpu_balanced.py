@@ -179,30 +179,56 @@ def test_two_tiers(gpu, H, KVH, dtype, monkeypatch):
     torch.testing.assert_close(lse, ref_lse, atol=1e-5, rtol=1e-5)
 
 
+def _c_call(case, dev, size, counters=None):
+    """The C entry point without counters, or with the given ones, a
+    workspace of `size` bytes full of ones."""
+    q, kc, vc, bt, lens = (x.to(dev) for x in case)
+    n, H, D = q.shape
+    KVH = kc.shape[1]
+    lib = _lib.load_lib()
+    ws = torch.full((max(size, 1),), 0xFF, dtype=torch.uint8, device=dev)
+    out, lse = torch.empty(n, H, D, device=dev), torch.empty(H, n, device=dev)
+    args = (q.data_ptr(), q.stride(0), q.stride(1), kc.data_ptr(), vc.data_ptr(), kc.stride(0),
+            kc.stride(1), kc.stride(2), kc.shape[0], bt.data_ptr(), bt.stride(0), bt.shape[1],
+            lens.data_ptr(), None, n, H, KVH, D, 16, 1 / math.sqrt(D), _lib.FD_BF16,
+            out.data_ptr(), out.stride(0), out.stride(1), _lib.FD_F32, lse.data_ptr(),
+            lse.stride(0), ws.data_ptr() if size else None, ctypes.c_size_t(size),
+            torch.cuda.current_stream().cuda_stream)
+    if counters is None:
+        _lib.check(lib.fd_paged_decode_partial(*args))
+    else:
+        _lib.check(lib.fd_paged_decode_counted(*args, 0, counters.data_ptr()))
+    torch.cuda.synchronize()
+    return out, lse
+
+
 def test_entry_points_without_counters(gpu):
     """The C entry points that bring no counters: a workspace of the query's
     size, full of ones, gives the counted call's bits; one that only covers
     the cut by table width (here none) is still taken."""
     case = _case([900, 500, 64], 32, 8, 128, torch.bfloat16, seed=12, spare=0)
-    q, kc, vc, bt, lens = (x.to(gpu) for x in case)
     ref = _run(case, gpu)
-    lib = _lib.load_lib()
-    need = ops.workspace_bytes(3, 32, 8, 128, 16, bt.shape[1])
+    need = ops.workspace_bytes(3, 32, 8, 128, 16, case[3].shape[1])
     assert need > 0
     for size in (need, 0):
-        ws = torch.full((max(size, 1),), 0xFF, dtype=torch.uint8, device=gpu)
-        out, lse = torch.empty(3, 32, 128, device=gpu), torch.empty(32, 3, device=gpu)
-        _lib.check(lib.fd_paged_decode_partial(
-            q.data_ptr(), q.stride(0), q.stride(1), kc.data_ptr(), vc.data_ptr(), kc.stride(0),
-            kc.stride(1), kc.stride(2), kc.shape[0], bt.data_ptr(), bt.stride(0), bt.shape[1],
-            lens.data_ptr(), None, 3, 32, 8, 128, 16, 1 / math.sqrt(128), _lib.FD_BF16,
-            out.data_ptr(), out.stride(0), out.stride(1), _lib.FD_F32, lse.data_ptr(),
-            lse.stride(0), ws.data_ptr() if size else None, ctypes.c_size_t(size),
-            torch.cuda.current_stream().cuda_stream))
-        torch.cuda.synchronize()
+        out, lse = _c_call(case, gpu, size)
         if size:
             assert torch.equal(out, ref[0]) and torch.equal(lse, ref[1])
         _check(case, out, lse)
+
+
+@pytest.mark.parametrize("left", [1, 2, 1000])
+def test_counts_an_earlier_launch_left_do_not_reach_the_next(gpu, left):
+    """Every counter starts with arrivals in it, as launches that overlapped
+    on them may leave."""
+    case = _case([900, 500, 64], 32, 8, 128, torch.bfloat16, seed=12, spare=0)
+    ref = _run(case, gpu)
+    need = ops.workspace_bytes(3, 32, 8, 128, 16, case[3].shape[1])
+    counters = torch.zeros(_lib.DECODE_COUNTERS // 2, dtype=torch.int64, device=gpu)
+    counters += left
+    for _ in range(2):
+        out, lse = _c_call(case, gpu, need, counters)
+        assert torch.equal(out, ref[0]) and torch.equal(lse, ref[1])
 
 
 @pytest.mark.parametrize("native", [True, False])

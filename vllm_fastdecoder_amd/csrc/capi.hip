@@ -61,6 +61,12 @@ bool in_host_memory(const void* p) {
   return host;
 }
 
+// The caller's arrival counters as the kernels' 64-bit words (none where they
+// do not lie so).
+uint64_t* counter_array(uint32_t* c) {
+  return reinterpret_cast<uintptr_t>(c) % 8 == 0 ? reinterpret_cast<uint64_t*>(c) : nullptr;
+}
+
 // Blocks made by fd_host_alloc and the device that was current then: the
 // device whose queued work fd_host_free waits for.
 std::mutex g_host_mu;
@@ -369,7 +375,7 @@ int fd_paged_decode_counted(
   a.tier[0] = KvTier{k_cache, v_cache, kv_stride_block, kv_stride_head, kv_stride_token,
                      num_blocks, block_table, bt_stride, bt_width, lens};
   a.ntiers = 1;
-  a.counters = counters;
+  a.counters = counter_array(counters);
   return run_decode(a, "decode", q, q_stride_seq, q_stride_head, row_order, n, num_heads,
                     num_kv_heads, head_size, block_size, scale, kv_dtype, out, out_stride_seq,
                     out_stride_head, out_dtype, lse, lse_stride_head, workspace,
@@ -418,7 +424,7 @@ int fd_split_decode_counted(const void* q, int64_t q_stride_seq, int64_t q_strid
                        d.num_blocks, d.block_table, d.bt_stride, d.bt_width, d.lens};
   }
   a.ntiers = 2;
-  a.counters = counters;
+  a.counters = counter_array(counters);
   return run_decode(a, "split_decode", q, q_stride_seq, q_stride_head, row_order, n, num_heads,
                     num_kv_heads, head_size, block_size, scale, kv_dtype, out, out_stride_seq,
                     out_stride_head, out_dtype, lse, lse_stride_head, workspace,

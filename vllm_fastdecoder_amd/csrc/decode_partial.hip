@@ -776,15 +776,23 @@ size_t balanced_partial_bytes(const SplitPlan& sp, int32_t H, int32_t D) {
   return (parts * (D + 1) * sizeof(float) + 255) / 256 * 256;
 }
 
+// 64-bit words from one of `pairs` arrival counters to the next: up to 256
+// bytes, as far as the caller's array reaches.
+static int32_t counter_stride(int64_t pairs) {
+  return (int32_t)std::min<int64_t>(32, kMaxBalPairs / std::max<int64_t>(pairs, 1));
+}
+
 size_t balanced_counter_bytes(const SplitPlan& sp, int32_t n, int32_t KVH) {
-  return sp.bal_parts > 0 ? (size_t)n * KVH * sp.passes * sizeof(uint32_t) : 0;
+  const int64_t pairs = (int64_t)n * KVH * sp.passes;
+  return sp.bal_parts > 0 ? (size_t)pairs * counter_stride(pairs) * sizeof(uint64_t) : 0;
 }
 
 // Clears a balanced launch's arrival counters where the caller keeps none.
 // (A kernel, not a memset: the call may be captured in a graph.)
-__global__ __launch_bounds__(256) void clear_counters_kernel(uint32_t* c, int32_t count) {
+__global__ __launch_bounds__(256) void clear_counters_kernel(uint64_t* c, int32_t count,
+                                                             int32_t stride) {
   const int32_t k = blockIdx.x * 256 + threadIdx.x;
-  if (k < count) c[k] = 0;
+  if (k < count) c[k * stride] = 0;
 }
 
 int launch_decode(const DecodeArgs& a, const SplitPlan& sp, hipStream_t s) {
@@ -886,13 +894,16 @@ int launch_decode(const DecodeArgs& a, const SplitPlan& sp, hipStream_t s) {
     tp.host_wgs = sp.host_wgs;
     tp.order = a.order;
     tp.wave_blocks = 0;
+    static std::atomic<uint64_t> launches{0};
+    tp.launch = ++launches << kArrivalBits;
     tp.counters = a.counters;
+    const int32_t count = a.n * a.KVH * sp.passes;
+    tp.counter_stride = counter_stride(count);
     if (tp.counters == nullptr) {
-      const int32_t count = a.n * a.KVH * sp.passes;
-      tp.counters = reinterpret_cast<uint32_t*>(static_cast<char*>(a.workspace) +
+      tp.counters = reinterpret_cast<uint64_t*>(static_cast<char*>(a.workspace) +
                                                 balanced_partial_bytes(sp, a.H, a.D));
       hipLaunchKernelGGL(clear_counters_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256),
-                         0, s, tp.counters, count);
+                         0, s, tp.counters, count, tp.counter_stride);
       const hipError_t e = hipGetLastError();
       if (e != hipSuccess) return hip_error(e, "clear_counters_kernel launch");
     }

@@ -248,8 +248,8 @@ struct DecodeArgs {
   int64_t lse_sh;
   void* workspace;
   size_t workspace_bytes;
-  uint32_t* counters;  // balanced launches' arrival counters, all zero (NULL: taken from the
-                       // workspace and cleared by a launch of their own)
+  uint64_t* counters;  // balanced launches' arrival counters (NULL: taken from the workspace
+                       // and cleared by a launch of their own)
   // measurement only (fd_paged_decode_timeline): per-workgroup time stamps
   // of a VALU-kernel launch, kTimelineSlots words per workgroup; NULL in
   // every other call

@@ -101,20 +101,20 @@ bool current_stream(int64_t idx, void** stream) {
   return !(PyErr_Occurred());
 }
 
-// The stream's workspace of at least `need` bytes and the counters behind it
+// The (current) stream's workspace of at least `need` bytes and the counters behind it
 // (ops._counters_ptr: on the next 256-byte boundary, where the buffer has
 // them); `hold` keeps it alive over the launch. False with a Python error set.
-bool workspace(const at::Tensor& q, size_t need, PyRef& hold, void** ws, size_t* bytes,
-               uint32_t** counters) {
+bool workspace(const at::Tensor& q, size_t need, void* stream, PyRef& hold, void** ws,
+               size_t* bytes, uint32_t** counters) {
   *ws = nullptr;
   *bytes = 0;
   *counters = nullptr;
   if (need == 0) return true;
   PyRef dev(THPDevice_New(q.device()));
   if (dev.p == nullptr) return false;
-  PyRef n(PyLong_FromSize_t(need));
-  if (n.p == nullptr) return false;
-  hold.p = PyObject_CallFunctionObjArgs(g_workspace_get, dev.p, n.p, nullptr);
+  PyRef n(PyLong_FromSize_t(need)), s(PyLong_FromVoidPtr(stream));
+  if (n.p == nullptr || s.p == nullptr) return false;
+  hold.p = PyObject_CallFunctionObjArgs(g_workspace_get, dev.p, n.p, s.p, nullptr);
   if (hold.p == nullptr) return false;
   const at::Tensor& buf = THPVariable_Unpack(hold.p);
   *ws = buf.data_ptr();
@@ -276,7 +276,7 @@ PyObject* paged_decode(PyObject*, PyObject* const* a, Py_ssize_t na) {
     size_t ws_bytes;
     uint32_t* counters;
     if (!current_stream(q->get_device(), &stream) ||
-        !workspace(*q, need, hold, &ws, &ws_bytes, &counters))
+        !workspace(*q, need, stream, hold, &ws, &ws_bytes, &counters))
       return nullptr;
     const int status = without_gil([&] { return fd_paged_decode_counted(
         q->data_ptr(), q->stride(0), q->stride(1), k->data_ptr(), v->data_ptr(), k->stride(0),
@@ -349,7 +349,7 @@ PyObject* split_decode(PyObject*, PyObject* const* a, Py_ssize_t na) {
     size_t ws_bytes;
     uint32_t* counters;
     if (!current_stream(q->get_device(), &stream) ||
-        !workspace(*q, need, hold, &ws, &ws_bytes, &counters))
+        !workspace(*q, need, stream, hold, &ws, &ws_bytes, &counters))
       return nullptr;
     const int status = without_gil([&] { return fd_split_decode_counted(
         q->data_ptr(), q->stride(0), q->stride(1), &t0, &t1, order, (int32_t)n, (int32_t)H,

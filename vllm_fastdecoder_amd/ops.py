@@ -116,13 +116,13 @@ class _Workspace:
 
     def get(self, device: torch.device, nbytes: int, stream: int | None = None,
             pin: bool = False) -> torch.Tensor | None:
-        """The workspace of `stream` (a raw handle; default: the current
-        stream on `device`, the one the caller's launch goes on), at least
-        nbytes long. pin: keep this stream's buffers alive (see above)."""
+        """The workspace of `stream` (a raw handle; the current stream on
+        `device`, the one the caller's launch goes on, unless only room is
+        made for it), at least nbytes long. pin: keep this stream's buffers alive (see above)."""
         if nbytes == 0 and not pin:
             return None
         key = self._key(device, stream)
-        if not pin and _capturing() and key not in self._pinned:
+        if not pin and key not in self._pinned and _capturing():
             # (freed when the caller drops it, to the pool that torch keeps for
             # this graph: only its later captured work uses that)
             return self._allocate(key, nbytes)
