@@ -110,6 +110,44 @@ def test_rows_past_one_tasks_blocks(gpu, monkeypatch):
     _check(case, *_run(case, gpu))
 
 
+@pytest.mark.parametrize("H,KVH,D,dtype,bar_out,bar_lse", [
+    (8, 8, 128, torch.float16, 2.0e-7, 3.55e-8), (8, 4, 64, torch.bfloat16, 2.1e-7, 3.9e-8),
+    (8, 2, 256, torch.bfloat16, 2.4e-7, 3.2e-8), (8, 2, 128, torch.float32, 2.05e-7, 3.8e-8)])
+def test_merged_rows_keep_fp32_precision(gpu, H, KVH, D, dtype, bar_out, bar_lse, monkeypatch):
+    """Rows of many parts, kernels whose weights are fp32 throughout: distances
+    from 64 bits in the 2-norm (2^-24 is 6e-8; the last rounding of a number
+    alone is up to 3e-8). Measured with the parts kept as sums: 1.7, 1.6, 2.2,
+    1.9e-7 and 3.2, 3.5, 2.9, 3.7e-8; kept as normalised outputs and LSEs: 2.3,
+    2.7, 2.7, 2.2e-7 and 3.9, 4.4, 3.5, 4.0e-8. The bars lie between."""
+    monkeypatch.setenv("FD_BALANCE", str(16 * 8 * KVH))
+    case = _case([1200 + 37 * i for i in range(8)], H, KVH, D, dtype, seed=D + H)
+    out, lse = _run(case, gpu)
+    q, kc, vc, bt, lens = case
+    ref_out, ref_lse = oracle.decode_attn_host_layout_f64(q, kc, vc, bt, lens, 1 / math.sqrt(D))
+    assert float((out.cpu().double() - ref_out).norm() / ref_out.norm()) < bar_out
+    assert float((lse.cpu().double() - ref_lse).norm() / ref_lse.norm()) < bar_lse
+
+
+@pytest.mark.parametrize("H,KVH,D,dtype", [(2, 2, 128, torch.float16), (8, 2, 128, torch.bfloat16),
+                                           (8, 2, 256, torch.bfloat16), (2, 2, 128, torch.float32)])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_bad_values_of_a_weightless_part_show(gpu, H, KVH, D, dtype, bad, monkeypatch):
+    """A V entry that is no number in a part whose weight underflows: as in a
+    row of one task (and in 64 bits), its dimension is no number either."""
+    q, kc, vc, bt, lens = _case([640], H, KVH, D, dtype, seed=6)
+    q.fill_(1.0)
+    kc.fill_(14.0)
+    for b in bt[0, :8]:  # the row's first 128 tokens: scores about 300 lower
+        kc[int(b)] = -14.0
+    vc[int(bt[0, 3]), :, 5, 9] = bad
+    for parts in ("0", str(8 * KVH)):
+        monkeypatch.setenv("FD_BALANCE", parts)
+        out, lse = _run((q, kc, vc, bt, lens), gpu)
+        assert not torch.isfinite(out[..., 9]).any() and torch.isfinite(lse).all()
+        keep = torch.arange(D) != 9
+        assert torch.isfinite(out[..., keep]).all()
+
+
 def test_chosen_by_the_plan(gpu):
     """A small grouped-query batch takes the cut by itself, and gives the same
     bits on every call (the counters are back at zero) and in any order; a

@@ -416,23 +416,16 @@ __device__ __forceinline__ void mm_task(const TiledParams& p, const Task& t, MmL
         o[6] += sc * b.z;
         o[7] += sc * b.w;
       }
-      const float inv = 1.f / ltot;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) o[e] *= inv;
-      float lse2 = M + fast_log2(ltot);
-      if (bad) {
-        lse2 = qnan();
-#pragma unroll
-        for (int e = 0; e < 8; ++e) o[e] = qnan();
-      }
+      if (bad) ltot = qnan();  // and with it the row's output and LSE
       const int hc = kCols * g + cc;  // the task's head slot
       if (hc < t.gcount && d0 < p.D) {
         const int h = t.h0 + hc;
         if (write_final) {
+          normalise(o, ltot);
           store8<T>(p.out, (int64_t)t.i * p.out_ss + (int64_t)h * p.out_sh + d0, p.out_f32, o);
-          if (d0 == 0) p.lse[(int64_t)h * p.lse_sh + t.i] = lse2 * kLn2;
+          if (d0 == 0) p.lse[(int64_t)h * p.lse_sh + t.i] = (M + fast_log2(ltot)) * kLn2;
         } else {
-          store_partial<CG == 1>(p, t, h, d0, o, lse2);
+          store_partial<CG == 1>(p, t, h, d0, o, M, ltot);
         }
       }
     }

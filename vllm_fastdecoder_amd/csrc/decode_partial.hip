@@ -773,7 +773,7 @@ bool plan_host_workers(SplitPlan& sp, int32_t n, int32_t H, int32_t KVH, int32_t
 size_t balanced_partial_bytes(const SplitPlan& sp, int32_t H, int32_t D) {
   if (sp.bal_parts <= 0) return 0;
   const size_t parts = (size_t)sp.bal_slots * H;
-  return (parts * (D + 1) * sizeof(float) + 255) / 256 * 256;
+  return (parts * (D + 2) * sizeof(float) + 255) / 256 * 256;
 }
 
 // 64-bit words from one of `pairs` arrival counters to the next: up to 256

@@ -78,6 +78,7 @@ struct TiledParams {
   int64_t lse_sh;
   float* part_o;    // [n, H, S, D] fp32 (normalised partial outputs)
   float* part_lse;  // [n, H, S] fp32 (natural-log LSE of each partial)
+  // balanced cuts: [slots, H, D] sums of p V and [slots, H, 2] (max, sum of p)
   int32_t S;        // max splits per (sequence, kv head)
   int32_t split_blocks;
   int32_t wave_blocks;  // blocks per working wave (0: every wave works; wave_blocks())
@@ -734,32 +735,53 @@ __device__ __forceinline__ void publish_wave_state(WaveStates<D, G>& ws, int wav
 // past the XCD's own L2), as a row's tasks run on several XCDs.
 constexpr int kAgentScope = 16;
 typedef unsigned int part_u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int part_u32x2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t part_rsrc(const float* base, int64_t elems) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), (short)0, (int)(elems * 4),
                                            0x00020000);
 }
 
-// Writes a split task's partial of 8 dims of query head h: the normalised
-// output and, with d0 == 0, the LSE (lse2: log2 domain).
+__device__ __forceinline__ void normalise(float (&o)[8], float l) {
+  const float inv = 1.f / l;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) o[e] *= inv;
+}
+
+// Writes a split task's partial of 8 dims of query head h from its sums of
+// p V, running max M (log2 domain) and sum of p. Cut by table width: the
+// normalised output and, with d0 == 0, the LSE. Balanced cuts keep the sums
+// and (M, l) as they are: a weight exp2(M - max) made from an LSE, a number
+// of about 10 in fp32, has its rounding in every bit of the merged row.
+// Distance from 64 bits (fp32 out; kept as LSEs, then as sums): 12 x
+// U[64, 1500], 32/8, fp32 KV 2.0 -> 1.7e-7 (LSE 4.8 -> 3.9e-8); 4 x
+// U[3000, 9000], 32/32, fp16 3.1 -> 2.2e-7. A part whose weight underflows
+// still shows a NaN or infinity in its V, as in a row of one task.
 template <bool BAL = true>
 __device__ __forceinline__ void store_partial(const TiledParams& p, const Task& t, int h, int d0,
-                                              const float* o, float lse2) {
+                                              float (&o)[8], float M, float l) {
   if (BAL && p.bal_parts > 0) {
-    const int64_t pidx = (int64_t)(t.slot0 + t.split) * p.H + h;
-    const __amdgpu_buffer_rsrc_t ro = part_rsrc(p.part_o + pidx * p.D, p.D);
+    // (resources of the whole task: one of each lane's head would not be
+    // uniform, and cost a loop over the heads per store)
+    const int64_t pidx = (int64_t)(t.slot0 + t.split) * p.H + t.h0;
+    const __amdgpu_buffer_rsrc_t ro = part_rsrc(p.part_o + pidx * p.D, (int64_t)t.gcount * p.D);
+    const int off = (h - t.h0) * p.D + d0;
 #pragma unroll
     for (int e = 0; e < 8; e += 4) {
       const part_u32x4 u = {__float_as_uint(o[e]), __float_as_uint(o[e + 1]),
                             __float_as_uint(o[e + 2]), __float_as_uint(o[e + 3])};
-      __builtin_amdgcn_raw_buffer_store_b128(u, ro, (d0 + e) * 4, 0, kAgentScope);
+      __builtin_amdgcn_raw_buffer_store_b128(u, ro, (off + e) * 4, 0, kAgentScope);
     }
-    if (d0 == 0)
-      __hip_atomic_store(p.part_lse + pidx, lse2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (d0 == 0) {
+      const part_u32x2 u = {__float_as_uint(M), __float_as_uint(l)};
+      __builtin_amdgcn_raw_buffer_store_b64(u, part_rsrc(p.part_lse + pidx * 2, 2 * t.gcount),
+                                            (h - t.h0) * 8, 0, kAgentScope);
+    }
   } else {
     const int64_t pidx = ((int64_t)t.i * p.H + h) * p.S + t.split;
+    normalise(o, l);
     store8<F32>(p.part_o, pidx * p.D + d0, true, o);
-    if (d0 == 0) p.part_lse[pidx] = lse2 * kLn2;
+    if (d0 == 0) p.part_lse[pidx] = (M + fast_log2(l)) * kLn2;
   }
 }
 
@@ -808,23 +830,16 @@ __device__ __forceinline__ void finish_task(const TiledParams& p, const Task& t,
       o[6] += sc * sb[w].z;
       o[7] += sc * sb[w].w;
     }
-    const float inv = 1.f / lt;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] *= inv;
-    float lse2 = M + fast_log2(lt);
-    if (bad) {
-      lse2 = qnan();
-#pragma unroll
-      for (int e = 0; e < 8; ++e) o[e] = qnan();
-    }
+    if (bad) lt = qnan();  // and with it the row's output and LSE
     const int h = t.h0 + g;
     if (g < t.gcount && lane < LPT && chunk * 8 < p.D) {
       if (write_final) {
+        normalise(o, lt);
         store8<T>(p.out, (int64_t)t.i * p.out_ss + (int64_t)h * p.out_sh + chunk * 8,
                   p.out_f32, o);
-        if (lane == 0) p.lse[(int64_t)h * p.lse_sh + t.i] = lse2 * kLn2;
+        if (lane == 0) p.lse[(int64_t)h * p.lse_sh + t.i] = (M + fast_log2(lt)) * kLn2;
       } else {
-        store_partial(p, t, h, chunk * 8, o, lse2);
+        store_partial(p, t, h, chunk * 8, o, M, lt);
       }
     }
   }
@@ -876,9 +891,10 @@ __device__ __forceinline__ bool last_to_arrive(const TiledParams& p, const Task&
 }
 
 // Merges the row's parts and writes its result (thread `tid` of `threads`: the
-// workgroup, or host worker wave, of the row's last task): a thread takes 4 dims of a head and folds the parts in
-// order, kPartsInFlight of them read together, as each round of reads is a
-// trip past the L2. The order is fixed, whichever task arrives last.
+// workgroup, or host worker wave, of the row's last task): a thread takes 4
+// dims of a head and folds the parts in order, kPartsInFlight of them read
+// together, as each round of reads is a trip past the L2. The order is fixed,
+// whichever task arrives last.
 constexpr int kPartsInFlight = 8;
 
 template <typename T, int D>
@@ -886,32 +902,28 @@ __device__ __forceinline__ void merge_parts(const TiledParams& p, const Task& t,
                                             int threads) {
   constexpr int LPT = D / 4;  // threads per head
   const int64_t first = (int64_t)t.slot0 * p.H + t.h0;
-  const __amdgpu_buffer_rsrc_t ro =
-      part_rsrc(p.part_o + first * p.D, ((int64_t)(t.nsplit - 1) * p.H + t.gcount) * p.D);
-  const __amdgpu_buffer_rsrc_t rl =
-      part_rsrc(p.part_lse + first, (int64_t)(t.nsplit - 1) * p.H + t.gcount);
+  const int64_t heads = (int64_t)(t.nsplit - 1) * p.H + t.gcount;
+  const __amdgpu_buffer_rsrc_t ro = part_rsrc(p.part_o + first * p.D, heads * p.D);
+  const __amdgpu_buffer_rsrc_t rl = part_rsrc(p.part_lse + first * 2, heads * 2);
   for (int it = tid; it < t.gcount * LPT; it += threads) {
     const int g = it / LPT;
     const int d0 = (it % LPT) * 4;
     if (d0 >= p.D) continue;
     float M = neg_inf(), l = 0.f, acc[4] = {0.f, 0.f, 0.f, 0.f};
     for (int k0 = 0; k0 < t.nsplit; k0 += kPartsInFlight) {
-      float lv[kPartsInFlight];
+      part_u32x2 ml[kPartsInFlight];
       part_u32x4 x[kPartsInFlight];
 #pragma unroll
       for (int u = 0; u < kPartsInFlight; ++u) {
-        // a part past the last reads the last one again, weightless
+        // a part past the last reads the last one again, to no effect
         const uint32_t pi = (uint32_t)(min(k0 + u, t.nsplit - 1) * p.H + g);
-        lv[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rl, pi * 4, 0, kAgentScope));
+        ml[u] = __builtin_amdgcn_raw_buffer_load_b64(rl, pi * 8, 0, kAgentScope);
         x[u] = __builtin_amdgcn_raw_buffer_load_b128(
             ro, (pi * (uint32_t)p.D + (uint32_t)d0) * 4, 0, kAgentScope);
       }
       float mn = M;
 #pragma unroll
-      for (int u = 0; u < kPartsInFlight; ++u) {
-        lv[u] = k0 + u < t.nsplit ? lv[u] : neg_inf();
-        mn = fmaxf(mn, lv[u]);
-      }
+      for (int u = 0; u < kPartsInFlight; ++u) mn = fmaxf(mn, __uint_as_float(ml[u][0]));
       const float ms = mn == neg_inf() ? 0.f : mn;
       const float alpha = fast_exp2(M - ms);
       l *= alpha;
@@ -919,14 +931,12 @@ __device__ __forceinline__ void merge_parts(const TiledParams& p, const Task& t,
       for (int e = 0; e < 4; ++e) acc[e] *= alpha;
 #pragma unroll
       for (int u = 0; u < kPartsInFlight; ++u) {
-        const float w = fast_exp2(lv[u] - ms);
-        l += w;
+        const bool on = k0 + u < t.nsplit;
+        const float w = fast_exp2(__uint_as_float(ml[u][0]) - ms);
+        l = __builtin_fmaf(w, on ? __uint_as_float(ml[u][1]) : 0.f, l);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          // a part of weight 0 (read again, or all its scores -inf) may hold NaN
-          const float o = w == 0.f ? 0.f : __uint_as_float(x[u][e]);
-          acc[e] = __builtin_fmaf(w, o, acc[e]);
-        }
+        for (int e = 0; e < 4; ++e)
+          acc[e] = __builtin_fmaf(w, on ? __uint_as_float(x[u][e]) : 0.f, acc[e]);
       }
       M = mn;
     }
@@ -935,7 +945,9 @@ __device__ __forceinline__ void merge_parts(const TiledParams& p, const Task& t,
     for (int e = 0; e < 4; ++e) acc[e] *= inv;
     const int h = t.h0 + g;
     store4<T>(p.out, (int64_t)t.i * p.out_ss + (int64_t)h * p.out_sh + d0, p.out_f32, acc);
-    if (d0 == 0) p.lse[(int64_t)h * p.lse_sh + t.i] = (M + fast_log2(l)) * kLn2;
+    // (M, about 10, is rounded once: with the product)
+    if (d0 == 0)
+      p.lse[(int64_t)h * p.lse_sh + t.i] = __builtin_fmaf(M, kLn2, fast_log2(l) * kLn2);
   }
 }
 
