@@ -25,6 +25,12 @@
 //           and p_lo = (p - p_hi) rounded, so the products keep about 16 bits
 //           of p (one part alone keeps 8 for bf16, 11 for fp16); fp16 p is
 //           scaled by 2^7 first (p <= 2^15) so small weights stay normal.
+//           Two-tier launches add a third part, the rounding of what is left:
+//           all 24 bits of an fp32 p, as on the VALU kernel, which takes them
+//           where this one does not. Distance from 64 bits of an fp32 out, two
+//           parts, three, VALU: 33 x U[40, 1800], 32/8, bf16 20, 1.6 and
+//           1.8e-7; 24 x U[256, 1024], 32/32, bf16 24, 1.9 and 1.8e-7. It
+//           costs 0-3 % (64 x U[500, 1500], 32/8: 66.5 -> 67.3 us).
 //           The B operand needs 4 consecutive tokens of one dim per lane:
 //           each wave writes its V block row-major to LDS (lane l of load j
 //           carries 16-byte chunk 64 j + l of the block, so the loads stay
@@ -80,12 +86,15 @@ __device__ __forceinline__ f32x4 mfma_pv<BF16>(s16x4 a, s16x4 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
 }
 
-// p split into its 16-bit rounding and the rounding of the remainder.
-template <typename T>
-__device__ __forceinline__ void split16(float x, short& hi, short& lo) {
-  const uint16_t h = from_f32(T{}, x);
-  hi = (short)h;
-  lo = (short)from_f32(T{}, x - lo_f32(T{}, (uint32_t)h));
+// p split into its 16-bit rounding and the roundings of the remainders.
+template <typename T, int N>
+__device__ __forceinline__ void split16(float x, short (&part)[N]) {
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    const uint16_t h = from_f32(T{}, x);
+    part[k] = (short)h;
+    x -= lo_f32(T{}, (uint32_t)h);
+  }
 }
 
 // LDS of one workgroup: the waves' V staging (two slots each) during the
@@ -107,8 +116,8 @@ struct __align__(16) MmLds {  // 16-byte V rows, float4 merge reads
 };
 
 // One task of the kernel, over tier 0's blocks, both tiers' or (one wave, a
-// host worker's) tier 1's.
-template <typename T, int D, int CG, int TS>
+// host worker's) tier 1's; P in PN parts.
+template <typename T, int D, int CG, int TS, int PN>
 __device__ __forceinline__ void mm_task(const TiledParams& p, const Task& t, MmLds<D>& lds,
                                         int wave, int lane) {
   constexpr bool TWO = TS == kBothTiers;
@@ -281,7 +290,7 @@ __device__ __forceinline__ void mm_task(const TiledParams& p, const Task& t, MmL
             make_uint4(x.w[0], x.w[1], x.w[2], x.w[3]);
       }
     }
-    s16x4 phi[CG], plo[CG];
+    s16x4 ps[CG][PN];
 #pragma unroll
     for (int g = 0; g < CG; ++g) {
       float bmax = fmaxf(fmaxf(s[g][0], s[g][1]), fmaxf(s[g][2], s[g][3]));
@@ -305,10 +314,10 @@ __device__ __forceinline__ void mm_task(const TiledParams& p, const Task& t, MmL
       for (int r = 0; r < 4; ++r) {
         const float pr = fast_exp2(s[g][r] - ms);
         l[g] += pr;
-        short h, lo;
-        split16<T>(pr * kPScale, h, lo);
-        phi[g][r] = h;
-        plo[g][r] = lo;
+        short part[PN];
+        split16<T>(pr * kPScale, part);
+#pragma unroll
+        for (int k = 0; k < PN; ++k) ps[g][k][r] = part[k];
       }
     }
     // the block's V rows are in LDS before any lane reads them transposed
@@ -318,8 +327,19 @@ __device__ __forceinline__ void mm_task(const TiledParams& p, const Task& t, MmL
       const s16x4 bv = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(st + tr_off + 16 * c));
 #pragma unroll
       for (int g = 0; g < CG; ++g) {
-        acc[g][c] = mfma_pv<T>(phi[g], bv, acc[g][c]);
-        acc[g][c] = mfma_pv<T>(plo[g], bv, acc[g][c]);
+        if constexpr (PN == 2) {
+          acc[g][c] = mfma_pv<T>(ps[g][0], bv, acc[g][c]);
+          acc[g][c] = mfma_pv<T>(ps[g][1], bv, acc[g][c]);
+        } else {
+          // the block's sum by itself, least parts first: each instruction
+          // rounds several times, and only the last addition rounds at the
+          // accumulator's size
+          f32x4 sum = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int k = PN - 1; k >= 0; --k) sum = mfma_pv<T>(ps[g][k], bv, sum);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[g][c][e] += sum[e];
+        }
       }
     }
   };
@@ -450,7 +470,7 @@ __global__ __launch_bounds__(kWave * kWavesPerTask) void decode_mm_kernel(TiledP
     if (t.split == 0 && wave == 0) write_empty<T, D, kCols * CG>(p, t, lane);
     return;
   }
-  mm_task<T, D, CG, TWO ? kBothTiers : kFirstTier>(p, t, lds, wave, lane);
+  mm_task<T, D, CG, TWO ? kBothTiers : kFirstTier, TWO ? 3 : 2>(p, t, lds, wave, lane);
 }
 
 // Two tiers with host workers (balanced_task in decode_tiled.h): the first
@@ -468,14 +488,14 @@ __global__ __launch_bounds__(kWave * kWavesPerTask) void decode_mm_tiers_kernel(
   if ((int)blockIdx.x < p.host_wgs) {
     for (int f = (int)blockIdx.x * kWavesPerTask + wave; task(f, true);
          f += kWavesPerTask * p.host_wgs)
-      mm_task<T, D, 1, kSecondTier>(p, t, lds, wave, lane);
+      mm_task<T, D, 1, kSecondTier, 3>(p, t, lds, wave, lane);
   } else {
     if (!task((int)blockIdx.x - p.host_wgs, false)) return;
     if (t.nb == 0 || t.range_bad) {
       if (wave == 0) write_empty<T, D, kCols>(p, t, lane);
       return;
     }
-    mm_task<T, D, 1, kFirstTier>(p, t, lds, wave, lane);
+    mm_task<T, D, 1, kFirstTier, 3>(p, t, lds, wave, lane);
   }
 }
 
