@@ -27,10 +27,13 @@
 //           scaled by 2^7 first (p <= 2^15) so small weights stay normal.
 //           Two-tier launches add a third part, the rounding of what is left:
 //           all 24 bits of an fp32 p, as on the VALU kernel, which takes them
-//           where this one does not. Distance from 64 bits of an fp32 out, two
-//           parts, three, VALU: 33 x U[40, 1800], 32/8, bf16 20, 1.6 and
-//           1.8e-7; 24 x U[256, 1024], 32/32, bf16 24, 1.9 and 1.8e-7. It
-//           costs 0-3 % (64 x U[500, 1500], 32/8: 66.5 -> 67.3 us).
+//           where this one does not; and they add up the steps of a score
+//           and the parts of a block by themselves, as each matrix
+//           instruction rounds several times at its accumulator's size.
+//           Distance from 64 bits of an fp32 out, two parts, so, VALU: 33 x
+//           U[40, 1800], 32/8, bf16 20, 1.5 and 1.8e-7; 24 x U[256, 1024],
+//           32/32, bf16 24, 1.7 and 1.8e-7, fp16 2.8, 1.7 and 1.9e-7. It
+//           costs 0-3 % (64 x U[500, 1500], 32/8: 66.5 -> 68.5 us).
 //           The B operand needs 4 consecutive tokens of one dim per lane:
 //           each wave writes its V block row-major to LDS (lane l of load j
 //           carries 16-byte chunk 64 j + l of the block, so the loads stay
@@ -255,7 +258,15 @@ __device__ __forceinline__ void mm_task(const TiledParams& p, const Task& t, MmL
       // q could still be NaN: zero it too
       const Vec8 kv = (32 * (ks + 1) <= D || k_dims_on(ks)) ? kb[slot][ks] : Vec8{{0u, 0u, 0u, 0u}};
 #pragma unroll
-      for (int g = 0; g < CG; ++g) sv[g] = mfma_qk<T>(kv, qb[g][ks], sv[g]);
+      for (int g = 0; g < CG; ++g) {
+        if constexpr (PN == 2) {
+          sv[g] = mfma_qk<T>(kv, qb[g][ks], sv[g]);
+        } else {  // (each step by itself, as the sums of P.V below)
+          const f32x4 part = mfma_qk<T>(kv, qb[g][ks], f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+          for (int e = 0; e < 4; ++e) sv[g][e] += part[e];
+        }
+      }
     }
 #pragma unroll
     for (int g = 0; g < CG; ++g) {
