@@ -298,7 +298,7 @@ def _current_device() -> int:
     return torch.cuda.current_device() if torch.cuda.is_available() else -1
 
 
-_ENV_NAMES = ("FD_SPLIT_BLOCKS", "FD_DECODE_KERNEL", "FD_BALANCE")
+_ENV_NAMES = ("FD_SPLIT_BLOCKS", "FD_DECODE_KERNEL", "FD_BALANCE", "FD_HOST_WGS")
 # os.environ encodes the name on every lookup (~0.6 us each, on every decode
 # call); on POSIX its own dict is keyed by the encoded names
 _ENV_DATA = getattr(os.environ, "_data", None)
@@ -312,14 +312,14 @@ def _planner_env() -> tuple:
     if _ENV_DATA is None:
         return tuple(os.environ.get(k) for k in _ENV_NAMES)
     get = _ENV_DATA.get
-    a, b, c = _ENV_KEYS
-    return get(a), get(b), get(c)
+    a, b, c, d = _ENV_KEYS
+    return get(a), get(b), get(c), get(d)
 
 
 def workspace_bytes(n: int, H: int, KVH: int, D: int, BS: int, width: int) -> int:
     """Workspace a decode call of this shape needs on the current device
     (remembered per shape, device and the planner overrides it depends on:
-    FD_SPLIT_BLOCKS, FD_BALANCE, and FD_DECODE_KERNEL, which can allow more
+    FD_SPLIT_BLOCKS, FD_BALANCE, FD_HOST_WGS, and FD_DECODE_KERNEL, which can allow more
     splits; the device's CU count sets the split bounds)."""
     key = (n, H, KVH, D, BS, width, _planner_env(), _current_device())
     size = _WS_SIZES.get(key)
