@@ -79,4 +79,4 @@ for name, values in (("FD_HOST_WGS", "0 32 128 512"), ("FD_BALANCE", "0 64 400")
     del os.environ[name]
 done(out)
 """)
-    assert all(a == b for a, b in got) and len({b for _, b in got[:4]}) > 2
+    assert all(a == b for a, b in got) and len({b for _, b in got[:4]}) > 1
