@@ -68,7 +68,9 @@ enum fd_status {
  * (the reference reports errors as RuntimeError via TORCH_CHECK). */
 const char* fd_last_error(void);
 
-/* Library ABI version (bumped when a signature changes). */
+/* Library ABI version (bumped when a signature changes): of this header, and
+ * of the library that is loaded. */
+#define FD_ABI_VERSION 14
 int fd_abi_version(void);
 
 /* ------------------------------------------------------------------------
@@ -237,14 +239,21 @@ int fd_paged_decode_workspace_size(
     int32_t block_size, int32_t bt_width, size_t* bytes);
 
 /* Bytes of workspace one fd_paged_decode_counted / fd_split_decode_counted
- * call with these sizes needs: the exact figure for one kv dtype and token
- * total, where fd_paged_decode_workspace_size covers them all. host_tier: 1 if
- * a tier lies in pinned host memory (a two-tier call asks for both and takes
- * the larger). No counterpart in the reference. */
+ * call with these sizes (bt_width: of both tiers' tables together) may need,
+ * for one kv dtype and token total, where fd_paged_decode_workspace_size
+ * covers them all. host_tier: 0 if the caches lie in HBM (the launch's own
+ * figure), 1 if one lies in pinned host memory or may (enough for each launch
+ * the call may become; a two-tier call over a pinned host tier asks for 1).
+ * No counterpart in the reference. */
 int fd_decode_workspace_need(int32_t n, int32_t num_heads, int32_t num_kv_heads,
                              int32_t head_size, int32_t block_size, int32_t bt_width,
                              int32_t kv_dtype, int32_t host_tier, int64_t total_tokens,
                              size_t* bytes);
+
+/* *host: 1 if p lies in pinned host memory by the decode calls' own lookup, in
+ * which each thread remembers the addresses it saw last. No counterpart in the
+ * reference. */
+int fd_in_host_memory(const void* p, int32_t* host);
 
 /* Which kernel a decode launch of these sizes takes, and how it is cut into
  * tasks (the planner of fd_paged_decode_partial / fd_split_decode, on the
@@ -255,8 +264,8 @@ int fd_decode_workspace_need(int32_t n, int32_t num_heads, int32_t num_kv_heads,
  *               (16-byte aligned q, out and caches; strides multiples of 8
  *               elements), else 0 (the generic kernel)
  *   host_tier   1 if the cache lies in pinned host memory (16-bit partials
- *               then take the VALU kernel; a two-tier launch with only its
- *               host tier there takes the matrix-core kernel where 0 gives it)
+ *               then take the VALU kernel); two-tier launches:
+ *               fd_split_decode_plan_info
  *   total_tokens the rows' token total, as given to
  *               fd_paged_decode_partial_hint (0: unknown)
  * FD_DECODE_KERNEL and FD_SPLIT_BLOCKS are honoured as in a launch. */
@@ -283,8 +292,20 @@ int fd_decode_plan_info(int32_t n, int32_t num_heads, int32_t num_kv_heads, int3
                         int32_t block_size, int32_t bt_width, int32_t kv_dtype, int32_t aligned,
                         int32_t host_tier, int64_t total_tokens, FdDecodePlan* plan);
 
-/* Whether a decode launch of these sizes (aligned, with the workspace the size
- * query asks for) is cut by the rows' lengths on the device instead of by the
+/* What an aligned two-tier call (fd_split_decode_counted; counted 0:
+ * fd_split_decode) of these sizes launches with a workspace of that size:
+ * host_pinned 1 if the host tier lies in pinned memory. *parts as below;
+ * *host_workgroups: the workgroups that take the host tier's blocks alone (0:
+ * tasks over both tiers' blocks). FD_ERR_WORKSPACE where the call would be
+ * refused for its workspace. No counterpart in the reference. */
+int fd_split_decode_plan_info(int32_t n, int32_t num_heads, int32_t num_kv_heads,
+                              int32_t head_size, int32_t block_size, int32_t hbm_width,
+                              int32_t host_width, int32_t kv_dtype, int32_t host_pinned,
+                              size_t workspace_bytes, int32_t counted, FdDecodePlan* plan,
+                              int32_t* parts, int32_t* host_workgroups);
+
+/* Whether a one-tier decode launch of these sizes (aligned, with the workspace
+ * the size query asks for) is cut by the rows' lengths on the device instead of by the
  * table width: *parts is the number of tasks aimed at per kv head and
  * head-group pass, 0 if the cut by table width that fd_decode_plan_info
  * describes is launched (kernel, heads_per_task and passes hold either way).

@@ -80,3 +80,54 @@ for name, values in (("FD_HOST_WGS", "0 32 128 512"), ("FD_BALANCE", "0 64 400")
 done(out)
 """)
     assert all(a == b for a, b in got) and len({b for _, b in got[:4]}) > 1
+
+
+SHAPES = """
+rng = random.Random(5)
+def shape():
+    H, KVH, D = rng.choice(((32, 8, 128), (32, 32, 128), (64, 8, 128), (16, 8, 256), (28, 4, 128),
+                            (40, 8, 112), (14, 2, 64), (24, 8, 128), (71, 1, 64), (8, 1, 80)))
+    return rng.randint(1, 80), H, KVH, D
+"""
+
+
+def test_two_tier_need_covers_the_launch(planner):
+    """A workspace of exactly fd_decode_workspace_need's bytes gives a two-tier
+    call the plan that an unlimited one gives it, counters or not."""
+    got = planner(SHAPES + """
+need, bad, workers = ctypes.c_size_t(), [], 0
+for _ in range(1500):
+    n, H, KVH, D = shape()
+    a, b = rng.randint(1, 300), rng.choice((1, 3, 20, 300))
+    dt = rng.choice((torch.float16, torch.bfloat16, torch.float32))
+    _lib.check(lib.fd_decode_workspace_need(n, H, KVH, D, 16, a + b, ops._DT[dt], 1, 0,
+                                            ctypes.byref(need)))
+    for counted in (True, False):
+        free = ops.split_plan_info(n, H, KVH, D, 16, a, b, dt, 1 << 40, counted)
+        workers += free["host_workgroups"] > 0
+        if ops.split_plan_info(n, H, KVH, D, 16, a, b, dt, need.value, counted) != free:
+            bad.append((n, H, KVH, D, a, b, str(dt), counted))
+done([len(bad), bad[:3], workers])
+""")
+    assert got[0] == 0, got
+    assert got[2] > 500
+
+
+def test_a_cache_found_in_host_memory_is_not_refused_its_hbm_workspace(planner):
+    """One tier at a pinned address (or one the lookup takes for it) with the
+    workspace of the HBM launch: planned again only where that fits. The calls
+    here pass every check and end at the launch, for want of a GPU."""
+    got = planner(SHAPES + """
+need, status = ctypes.c_size_t(), {}
+for _ in range(1500):
+    n, H, KVH, D = shape()
+    W = rng.randint(1, 600)
+    _lib.check(lib.fd_decode_workspace_need(n, H, KVH, D, 16, W, 0, 0, 0, ctypes.byref(need)))
+    p = 1 << 20
+    rc = lib.fd_paged_decode_counted(
+        p, H * D, D, 1 << 41, 1 << 41, KVH * 16 * D, 16 * D, D, 4, p, W, W, p, None, n, H, KVH, D,
+        16, 0.1, 0, p, H * D, D, 0, p, n, p if need.value else None, need.value, None, 0, p)
+    status[rc] = status.get(rc, 0) + 1
+done(status)
+""")
+    assert set(got) == {"4"}, got  # FD_ERR_HIP

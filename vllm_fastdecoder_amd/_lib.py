@@ -19,7 +19,7 @@ FD_F16, FD_BF16, FD_F32 = 0, 1, 2
 FD_OK = 0
 FD_ERR_INVALID, FD_ERR_RANGE, FD_ERR_WORKSPACE, FD_ERR_HIP, FD_ERR_UNSUPPORTED = 1, 2, 3, 4, 5
 FD_ERR_RESOURCE = 6
-ABI_VERSION = 13
+ABI_VERSION = 14
 DECODE_COUNTERS = 4096  # FD_DECODE_COUNTERS
 NOALLOC_SCRATCH_BYTES = 32 << 20  # FD_NOALLOC_SCRATCH_BYTES of include/fdattn.h
 
@@ -157,12 +157,19 @@ SIGNATURES: dict[str, tuple] = {
          c_int32, c_int32, c_int64,                             # kv_dtype, host_tier, total_tokens
          POINTER(c_size_t)],
     ),
+    "fd_in_host_memory": (c_int, [c_void_p, POINTER(c_int32)]),
     "fd_decode_plan_info": (
         c_int,
         [c_int32, c_int32, c_int32, c_int32, c_int32, c_int32,  # n, H, KVH, D, BS, bt_width
          c_int32, c_int32, c_int32,                             # kv_dtype, aligned, host_tier
          c_int64,                                               # total_tokens
          POINTER(FdDecodePlan)],
+    ),
+    "fd_split_decode_plan_info": (
+        c_int,
+        [c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32,  # n, H, KVH, D, BS, widths
+         c_int32, c_int32, c_size_t, c_int32,                            # kv_dtype, pinned, bytes, counted
+         POINTER(FdDecodePlan), POINTER(c_int32), POINTER(c_int32)],
     ),
     "fd_decode_balanced_parts": (
         c_int,

@@ -41,7 +41,9 @@ bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0;
 // Whether p points into pinned host memory, which the GPU reads over the link.
 // The answer for each recently seen pointer is kept per thread (a lookup
 // costs ~1 us; a layer's caches keep their addresses), and a stale entry
-// after a free can only change which of two correct kernels runs.
+// after a free can only change which of two correct kernels runs: a launch
+// whose workspace holds only the other's partials takes that one
+// (choose_plan).
 bool in_host_memory(const void* p) {
   struct Entry {
     const void* p;
@@ -81,6 +83,64 @@ double row_fill(int64_t total_tokens, int32_t n, int64_t width, int32_t block_si
   if (total_tokens <= 0 || n <= 0 || width <= 0) return 0.0;
   const double cap = (double)n * (double)width * block_size;
   return std::min(1.0, (double)total_tokens / cap);
+}
+
+struct CallSizes {
+  int32_t n, H, KVH, D, BS;
+  int ntiers;
+  int64_t width;  // of the tiers' tables together
+  int32_t kv_dtype;
+  bool aligned;
+  double fill;
+};
+
+size_t balanced_bytes(const SplitPlan& sp, const CallSizes& c, bool counted) {
+  return balanced_partial_bytes(sp, c.H, c.D) +
+         (counted ? 0 : balanced_counter_bytes(sp, c.n, c.KVH));
+}
+
+// What a decode call launches, given the workspace it brings (0: none that is
+// aligned), whether it brings counters, and pinned(t), whether tier t lies in
+// pinned host memory (asked only where the answer matters). *need: the
+// workspace the plan cannot do without.
+template <typename Pinned>
+SplitPlan choose_plan(const CallSizes& c, bool counted, size_t ws_bytes, bool timeline,
+                      Pinned&& pinned, size_t* need) {
+  // Balanced cuts need a workspace for whatever the rows' lengths make of
+  // them. A caller that brings less (it planned without them) gets the cuts
+  // by table width; a timeline is of those, as its buffer is sized for them.
+  auto planned = [&](bool matrix) -> SplitPlan {
+    SplitPlan sp = plan_decode(c.n, c.H, c.KVH, c.D, c.BS, (int32_t)c.width, c.kv_dtype, c.aligned,
+                               matrix, c.fill);
+    if (timeline || balanced_bytes(sp, c, counted) > ws_bytes) sp.bal_parts = 0;
+    return sp;
+  };
+  auto needs = [&](const SplitPlan& sp) -> size_t {
+    return sp.bal_parts > 0 ? 0 : decode_workspace_bytes(sp, c.n, c.H, c.D);
+  };
+  SplitPlan sp = planned(true);
+  // Over the link the matrix-core kernels' K tiles (16 token rows of 16 bytes
+  // per lane group) read slower than the VALU kernel's whole rows (measured
+  // on a GQA-4 host tier: 47.9 against 55.9 GB/s), so partials over pinned
+  // host memory take the VALU kernel. A two-tier launch on decode_mm_kernel
+  // reads its host blocks in whole rows and stays there for its HBM blocks,
+  // most of which the VALU kernel's per-head work holds up (33 rows of
+  // U[40, 1800], 32/8, one host block each: 44 -> 39 us; 64 of U[500, 1500]: 96 -> 85).
+  bool host = false;
+  const int read_in_rows = c.ntiers > 1 && sp.mm ? 1 : 0;  // of the tiers, the last
+  for (int t = 0; (sp.mfma || sp.mm) && t < c.ntiers - read_in_rows; ++t) host = host || pinned(t);
+  if (host) {
+    const SplitPlan rows = planned(false);
+    if (needs(rows) <= ws_bytes || needs(sp) > ws_bytes) sp = rows;
+  }
+  if (c.ntiers > 1 && pinned(1) && !pinned(0)) {
+    SplitPlan hw = sp;
+    if (plan_host_workers(hw, c.n, c.H, c.KVH, c.D, c.BS, (int32_t)c.width, c.kv_dtype) &&
+        balanced_bytes(hw, c, counted) <= ws_bytes)
+      sp = hw;
+  }
+  *need = needs(sp);
+  return sp;
 }
 
 // Validates a decode call over a.ntiers tiers (tiers already filled in),
@@ -139,41 +199,13 @@ int run_decode(DecodeArgs& a, const char* who, const void* q, int64_t q_stride_s
                   (1ll << 31);
   }
   const double fill = row_fill(total_tokens, n, width, block_size);
-  SplitPlan sp = plan_decode(n, num_heads, num_kv_heads, head_size, block_size,
-                             (int32_t)width, kv_dtype, aligned, true, fill);
-  // Over the link the matrix-core kernels' K tiles (16 token rows of 16 bytes
-  // per lane group) read slower than the VALU kernel's whole rows (measured
-  // on a GQA-4 host tier: 47.9 against 55.9 GB/s), so partials over pinned
-  // host memory take the VALU kernel. A two-tier launch on decode_mm_kernel
-  // reads its host blocks in whole rows and stays there for its HBM blocks,
-  // most of which the VALU kernel's per-head work holds up (33 rows of
-  // U[40, 1800], 32/8, one host block each: 45 -> 35 us; 64 of U[500, 1500]: 97 -> 80).
-  bool host = false;
-  const int read_in_rows = a.ntiers > 1 && sp.mm ? 1 : 0;  // of the tiers, the last
-  for (int t = 0; (sp.mfma || sp.mm) && t < a.ntiers - read_in_rows; ++t)
-    host = host || in_host_memory(a.tier[t].k);
-  if (host)
-    sp = plan_decode(n, num_heads, num_kv_heads, head_size, block_size, (int32_t)width, kv_dtype,
-                     aligned, false, fill);
-  // Balanced cuts need a workspace for whatever the rows' lengths make of
-  // them. A caller that brings less (it planned without them) gets the cuts
-  // by table width.
-  auto fits_workspace = [&](const SplitPlan& c) -> bool {
-    const size_t bal = balanced_partial_bytes(c, num_heads, head_size) +
-                       (a.counters == nullptr ? balanced_counter_bytes(c, n, num_kv_heads) : 0);
-    return bal == 0 || (workspace != nullptr && workspace_bytes >= bal && aligned16(workspace));
-  };
-  if (a.ntiers > 1 && in_host_memory(a.tier[1].k) && !in_host_memory(a.tier[0].k)) {
-    SplitPlan hw = sp;
-    if (plan_host_workers(hw, n, num_heads, num_kv_heads, head_size, block_size, (int32_t)width,
-                          kv_dtype) &&
-        fits_workspace(hw))
-      sp = hw;
-  }
-  if (!fits_workspace(sp)) sp.bal_parts = 0;
-  // a timeline is of whole tasks by table width, as its buffer is sized for
-  if (a.timeline != nullptr) sp.bal_parts = 0;
-  const size_t need = sp.bal_parts > 0 ? 0 : decode_workspace_bytes(sp, n, num_heads, head_size);
+  const CallSizes sizes{n,       num_heads, num_kv_heads, head_size, block_size,
+                        a.ntiers, width,     kv_dtype,     aligned,   fill};
+  size_t need = 0;
+  const SplitPlan sp = choose_plan(
+      sizes, a.counters != nullptr,
+      workspace != nullptr && aligned16(workspace) ? workspace_bytes : 0, a.timeline != nullptr,
+      [&](int t) { return in_host_memory(a.tier[t].k); }, &need);
   if (need > 0 && (workspace == nullptr || workspace_bytes < need || !aligned16(workspace)))
     return set_error(FD_ERR_WORKSPACE,
                      "%s: workspace of %zu bytes (16-byte aligned) required, got %zu", who, need,
@@ -237,6 +269,23 @@ int workspace_size(int32_t n, int32_t num_heads, int32_t num_kv_heads, int32_t h
   return FD_OK;
 }
 
+namespace {
+
+void fill_plan_info(const SplitPlan& sp, int32_t kv_dtype, FdDecodePlan* plan) {
+  plan->kernel = !sp.fast ? FD_KERNEL_GENERIC
+                 : kv_dtype == FD_F32 ? FD_KERNEL_F32
+                 : sp.mm ? FD_KERNEL_MM
+                 : sp.mfma ? FD_KERNEL_MFMA
+                           : FD_KERNEL_VALU;
+  plan->heads_per_task = sp.fast ? sp.kernel_g : 1;
+  plan->passes = sp.fast ? sp.passes : 1;
+  plan->split_blocks = sp.split_blocks;
+  plan->max_splits = sp.max_splits;
+  plan->wg_cap = sp.fast ? sp.wg_cap : 0;
+  plan->wave_blocks = sp.fast ? sp.wave_blocks : 0;
+}
+
+}  // namespace
 }  // namespace fd
 
 using namespace fd;
@@ -245,7 +294,7 @@ extern "C" {
 
 const char* fd_last_error(void) { return g_err; }
 
-int fd_abi_version(void) { return 13; }
+int fd_abi_version(void) { return FD_ABI_VERSION; }
 
 int fd_paged_decode_workspace_size(int32_t n, int32_t num_heads, int32_t num_kv_heads,
                                    int32_t head_size, int32_t block_size, int32_t bt_width,
@@ -263,18 +312,27 @@ int fd_decode_workspace_need(int32_t n, int32_t num_heads, int32_t num_kv_heads,
       head_size <= 0 || block_size <= 0 || bt_width < 0 || total_tokens < 0 ||
       !valid_dtype(kv_dtype))
     return set_error(FD_ERR_INVALID, "workspace_need: bad sizes");
-  const SplitPlan sp = plan_decode(n, num_heads, num_kv_heads, head_size, block_size, bt_width,
-                                   kv_dtype, true, host_tier == 0,
-                                   row_fill(total_tokens, n, bt_width, block_size));
   // (with room for counters, should the caller have none beside its workspace)
-  *bytes = sp.bal_parts > 0 ? balanced_partial_bytes(sp, num_heads, head_size) +
-                                  balanced_counter_bytes(sp, n, num_kv_heads)
-                            : decode_workspace_bytes(sp, n, num_heads, head_size);
-  SplitPlan hw = sp;
-  if (host_tier != 0 && plan_host_workers(hw, n, num_heads, num_kv_heads, head_size, block_size,
-                                          bt_width, kv_dtype))
-    *bytes = std::max(*bytes, balanced_partial_bytes(hw, num_heads, head_size) +
-                                  balanced_counter_bytes(hw, n, num_kv_heads));
+  const CallSizes c{n,        num_heads, num_kv_heads, head_size, block_size, 1,
+                    bt_width, kv_dtype,  true,         row_fill(total_tokens, n, bt_width, block_size)};
+  size_t most = 0;
+  for (int matrix = 1; matrix >= (host_tier == 0 ? 1 : 0); --matrix) {
+    const SplitPlan sp = plan_decode(n, num_heads, num_kv_heads, head_size, block_size, bt_width,
+                                     kv_dtype, true, matrix != 0, c.fill);
+    most = std::max(most, sp.bal_parts > 0 ? balanced_bytes(sp, c, false)
+                                           : decode_workspace_bytes(sp, n, num_heads, head_size));
+    SplitPlan hw = sp;
+    if (host_tier != 0 && plan_host_workers(hw, n, num_heads, num_kv_heads, head_size, block_size,
+                                            bt_width, kv_dtype))
+      most = std::max(most, balanced_bytes(hw, c, false));
+  }
+  *bytes = most;
+  return FD_OK;
+}
+
+int fd_in_host_memory(const void* p, int32_t* host) {
+  if (host == nullptr) return set_error(FD_ERR_INVALID, "in_host_memory: host is NULL");
+  *host = p != nullptr && in_host_memory(p) ? 1 : 0;
   return FD_OK;
 }
 
@@ -295,17 +353,32 @@ int fd_decode_plan_info(int32_t n, int32_t num_heads, int32_t num_kv_heads, int3
   if (host_tier != 0 && (sp.mfma || sp.mm))
     sp = plan_decode(n, num_heads, num_kv_heads, head_size, block_size, bt_width, kv_dtype,
                      aligned != 0, false, fill);
-  plan->kernel = !sp.fast ? FD_KERNEL_GENERIC
-                 : kv_dtype == FD_F32 ? FD_KERNEL_F32
-                 : sp.mm ? FD_KERNEL_MM
-                 : sp.mfma ? FD_KERNEL_MFMA
-                           : FD_KERNEL_VALU;
-  plan->heads_per_task = sp.fast ? sp.kernel_g : 1;
-  plan->passes = sp.fast ? sp.passes : 1;
-  plan->split_blocks = sp.split_blocks;
-  plan->max_splits = sp.max_splits;
-  plan->wg_cap = sp.fast ? sp.wg_cap : 0;
-  plan->wave_blocks = sp.fast ? sp.wave_blocks : 0;
+  fill_plan_info(sp, kv_dtype, plan);
+  return FD_OK;
+}
+
+int fd_split_decode_plan_info(int32_t n, int32_t num_heads, int32_t num_kv_heads,
+                              int32_t head_size, int32_t block_size, int32_t hbm_width,
+                              int32_t host_width, int32_t kv_dtype, int32_t host_pinned,
+                              size_t workspace_bytes, int32_t counted, FdDecodePlan* plan,
+                              int32_t* parts, int32_t* host_workgroups) {
+  if (plan == nullptr || parts == nullptr || host_workgroups == nullptr)
+    return set_error(FD_ERR_INVALID, "split_plan_info: NULL result");
+  if (n < 0 || num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads != 0 ||
+      head_size <= 0 || block_size <= 0 || hbm_width < 0 || host_width < 0 ||
+      (int64_t)hbm_width + host_width > INT32_MAX || !valid_dtype(kv_dtype))
+    return set_error(FD_ERR_INVALID, "split_plan_info: bad sizes");
+  const CallSizes c{n, num_heads, num_kv_heads, head_size, block_size,
+                    2, (int64_t)hbm_width + host_width, kv_dtype, true, 0.0};
+  size_t need = 0;
+  const SplitPlan sp = choose_plan(c, counted != 0, workspace_bytes, false,
+                                   [&](int t) { return t == 1 && host_pinned != 0; }, &need);
+  if (need > workspace_bytes)
+    return set_error(FD_ERR_WORKSPACE, "split_plan_info: workspace of %zu bytes required, got %zu",
+                     need, workspace_bytes);
+  fill_plan_info(sp, kv_dtype, plan);
+  *parts = sp.bal_parts;
+  *host_workgroups = sp.host_wgs;
   return FD_OK;
 }
 

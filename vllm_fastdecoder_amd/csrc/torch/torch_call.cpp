@@ -267,8 +267,10 @@ PyObject* paged_decode(PyObject*, PyObject* const* a, Py_ssize_t na) {
     const int kv = dtype_code(q->scalar_type());
     const float scale = (float)PyFloat_AS_DOUBLE(a[5]);
     size_t need = 0;
-    if (fd_decode_workspace_need((int32_t)n, (int32_t)H, (int32_t)KVH, (int32_t)D, (int32_t)BS,
-                                 (int32_t)width, kv, 0, total, &need) != FD_OK)
+    int32_t host = 0;  // a GPU tensor may lie over mapped host memory
+    if (fd_in_host_memory(k->data_ptr(), &host) != FD_OK ||
+        fd_decode_workspace_need((int32_t)n, (int32_t)H, (int32_t)KVH, (int32_t)D, (int32_t)BS,
+                                 (int32_t)width, kv, host, total, &need) != FD_OK)
       return not_here();  // sizes the call refuses: with Python's message
     if (!o.allocate(*q)) return not_here();
     PyRef hold;

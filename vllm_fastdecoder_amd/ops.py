@@ -263,16 +263,39 @@ def decode_plan_info(n: int, H: int, KVH: int, D: int, BS: int, width: int, dtyp
     kernel's own occupancy), "capped" (wg_cap > 0), "wave_blocks" (tiles per
     working wave, 0 = every wave works)}. total_tokens: the rows' token total
     a paged_decode call is given (None: unknown). Honours FD_DECODE_KERNEL /
-    FD_SPLIT_BLOCKS / FD_WG_CAP / FD_WAVE_BLOCKS."""
+    FD_SPLIT_BLOCKS / FD_WG_CAP / FD_WAVE_BLOCKS. A launch that balanced_parts
+    says is cut by the rows' lengths uses its workspace also where max_splits
+    is 1 here."""
     plan = _lib.FdDecodePlan()
     _lib.check(_lib.load_lib().fd_decode_plan_info(n, H, KVH, D, BS, width, _DT[dtype],
                                                    int(aligned), int(host_tier),
                                                    int(total_tokens or 0),
                                                    ctypes.byref(plan)))
+    return _plan_dict(plan)
+
+
+def _plan_dict(plan: _lib.FdDecodePlan) -> dict:
     return {"kernel": _lib.FD_KERNEL_NAMES[plan.kernel], "heads_per_task": plan.heads_per_task,
             "passes": plan.passes, "split_blocks": plan.split_blocks,
             "max_splits": plan.max_splits, "wg_cap": plan.wg_cap, "capped": plan.wg_cap > 0,
             "wave_blocks": plan.wave_blocks}
+
+
+def split_plan_info(n: int, H: int, KVH: int, D: int, BS: int, hbm_width: int, host_width: int,
+                    dtype: torch.dtype, workspace: int | None = None, counted: bool = True,
+                    host_pinned: bool = True) -> dict:
+    """What a split_decode call of these sizes launches
+    (fd_split_decode_plan_info): decode_plan_info's keys, "balanced_parts" (as
+    balanced_parts gives it) and "host_workgroups" (workgroups that take the
+    pinned host tier alone, 0: none). workspace: its bytes (None: what
+    workspace_bytes asks for); counted: with arrival counters."""
+    if workspace is None:
+        workspace = workspace_bytes(n, H, KVH, D, BS, hbm_width + host_width)
+    plan, parts, wgs = _lib.FdDecodePlan(), ctypes.c_int32(), ctypes.c_int32()
+    _lib.check(_lib.load_lib().fd_split_decode_plan_info(
+        n, H, KVH, D, BS, hbm_width, host_width, _DT[dtype], int(host_pinned), workspace,
+        int(counted), ctypes.byref(plan), ctypes.byref(parts), ctypes.byref(wgs)))
+    return {**_plan_dict(plan), "balanced_parts": parts.value, "host_workgroups": wgs.value}
 
 
 def balanced_parts(n: int, H: int, KVH: int, D: int, BS: int, width: int, dtype: torch.dtype,
