@@ -119,14 +119,15 @@ def test_a_cache_found_in_host_memory_is_not_refused_its_hbm_workspace(planner):
     here pass every check and end at the launch, for want of a GPU."""
     got = planner(SHAPES + """
 need, status = ctypes.c_size_t(), {}
-for _ in range(1500):
+for _ in range(6000):
     n, H, KVH, D = shape()
-    W = rng.randint(1, 600)
-    _lib.check(lib.fd_decode_workspace_need(n, H, KVH, D, 16, W, 0, 0, 0, ctypes.byref(need)))
+    n, W = 4 * n, rng.randint(1, 600)
+    total = int(rng.random() * n * W * 16)
+    _lib.check(lib.fd_decode_workspace_need(n, H, KVH, D, 16, W, 0, 0, total, ctypes.byref(need)))
     p = 1 << 20
     rc = lib.fd_paged_decode_counted(
         p, H * D, D, 1 << 41, 1 << 41, KVH * 16 * D, 16 * D, D, 4, p, W, W, p, None, n, H, KVH, D,
-        16, 0.1, 0, p, H * D, D, 0, p, n, p if need.value else None, need.value, None, 0, p)
+        16, 0.1, 0, p, H * D, D, 0, p, n, p if need.value else None, need.value, None, total, p)
     status[rc] = status.get(rc, 0) + 1
 done(status)
 """)
