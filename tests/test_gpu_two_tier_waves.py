@@ -65,6 +65,12 @@ def _run(gpu, H, KVH, D, dtype, rows, row_order=None, bad_row=None):
     return out, lse, ref_out, ref_lse, lens
 
 
+def _plan(H, KVH, D, dtype, rows):
+    """The launch of _run's call (tables as wide as the longest row)."""
+    W = max(a + b for a, b, _ in rows)
+    return ops.split_plan_info(len(rows), H, KVH, D, 16, W, W, dtype)
+
+
 def _check(got, dtype, rows=None):
     out, lse, ref_out, ref_lse, lens = got
     rows = list(range(len(lens))) if rows is None else rows
@@ -89,18 +95,29 @@ def test_tier_shares(gpu, H, KVH, D, dtype, split, monkeypatch):
     (7, 1, 48, torch.float16), (16, 1, 64, torch.bfloat16), (10, 2, 80, torch.float16)])
 def test_host_workers(gpu, H, KVH, D, dtype, workers, monkeypatch):
     """Rows of every tier share, one row, and 64 (the most the workers take);
-    the same bits on a second call and in any order."""
+    the same bits on a second call and in any order, from a workspace of the
+    call's own size as from a larger one."""
     monkeypatch.setenv("FD_HOST_WGS", workers)
+    for rows in (ROWS, ROWS[:1], ROWS * 5):
+        wgs = _plan(H, KVH, D, dtype, rows)["host_workgroups"]
+        assert wgs == (int(workers) if len(rows) <= 64 else 0), rows
+    monkeypatch.setattr(ops, "WORKSPACE", ops._Workspace())
     first = _run(gpu, H, KVH, D, dtype, ROWS)
     _check(first, dtype)
     order = torch.randperm(len(ROWS), generator=torch.Generator().manual_seed(2)).int()
     again = _run(gpu, H, KVH, D, dtype, ROWS, row_order=order)
     assert torch.equal(again[0], first[0]) and torch.equal(again[1], first[1])
+    ops.WORKSPACE.get(gpu, 1 << 24)
+    again = _run(gpu, H, KVH, D, dtype, ROWS)
+    assert torch.equal(again[0], first[0]) and torch.equal(again[1], first[1])
     _check(_run(gpu, H, KVH, D, dtype, [(30, 9, 4)]), dtype)
     _check(_run(gpu, H, KVH, D, dtype, [(i % 5, (3 * i) % 7, 1 + i % 16) for i in range(64)]), dtype)
 
 
-def test_host_workers_leave_out_and_range_errors(gpu):
+def test_host_workers_leave_out_and_range_errors(gpu, monkeypatch):
+    monkeypatch.setenv("FD_HOST_WGS", "32")
+    monkeypatch.setattr(ops, "WORKSPACE", ops._Workspace())
+    assert _plan(4, 1, 128, torch.bfloat16, ROWS)["host_workgroups"] == 32
     rows = list(range(len(ROWS)))
     order = torch.tensor([r if r not in (2, 5) else -1 for r in rows], dtype=torch.int32)
     got = _run(gpu, 4, 1, 128, torch.bfloat16, ROWS, row_order=order)

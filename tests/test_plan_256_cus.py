@@ -103,6 +103,7 @@ for _ in range(1500):
     _lib.check(lib.fd_decode_workspace_need(n, H, KVH, D, 16, a + b, ops._DT[dt], 1, 0,
                                             ctypes.byref(need)))
     for counted in (True, False):
+        os.environ.pop("FD_HOST_WGS", None)
         free = ops.split_plan_info(n, H, KVH, D, 16, a, b, dt, 1 << 40, counted)
         workers += free["host_workgroups"] > 0
         if ops.split_plan_info(n, H, KVH, D, 16, a, b, dt, need.value, counted) != free:
@@ -132,3 +133,17 @@ for _ in range(6000):
 done(status)
 """)
     assert set(got) == {"4"}, got  # FD_ERR_HIP
+
+
+def test_host_workers_go_by_the_tables_widths(planner):
+    """On both sides of each line of the rule (plan_host_workers)."""
+    got = planner("""
+def workers(n, H, KVH, a, b, D=128):
+    return ops.split_plan_info(n, H, KVH, D, 16, a, b, torch.bfloat16)["host_workgroups"] > 0
+done([
+    workers(33, 32, 8, 112, 1), workers(33, 32, 8, 100, 2), workers(33, 32, 8, 112, 112),
+    workers(40, 8, 1, 178, 10), workers(12, 16, 8, 88, 5), workers(12, 16, 8, 59, 5),
+    workers(1, 32, 8, 46, 11), workers(1, 32, 8, 22, 11), workers(64, 16, 16, 60, 1),
+    workers(64, 32, 32, 60, 1), workers(65, 32, 8, 112, 1)])
+""")
+    assert got == [True, True, True, False, True, False, False, True, True, False, False]

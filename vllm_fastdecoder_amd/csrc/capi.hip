@@ -92,6 +92,7 @@ struct CallSizes {
   int32_t kv_dtype;
   bool aligned;
   double fill;
+  int32_t tier_width[2];  // of each (two tiers)
 };
 
 size_t balanced_bytes(const SplitPlan& sp, const CallSizes& c, bool counted) {
@@ -135,7 +136,8 @@ SplitPlan choose_plan(const CallSizes& c, bool counted, size_t ws_bytes, bool ti
   }
   if (c.ntiers > 1 && pinned(1) && !pinned(0)) {
     SplitPlan hw = sp;
-    if (plan_host_workers(hw, c.n, c.H, c.KVH, c.D, c.BS, (int32_t)c.width, c.kv_dtype) &&
+    if (plan_host_workers(hw, c.n, c.H, c.KVH, c.D, c.BS, (int32_t)c.width, c.tier_width[0],
+                          c.tier_width[1], c.kv_dtype) &&
         balanced_bytes(hw, c, counted) <= ws_bytes)
       sp = hw;
   }
@@ -200,7 +202,8 @@ int run_decode(DecodeArgs& a, const char* who, const void* q, int64_t q_stride_s
   }
   const double fill = row_fill(total_tokens, n, width, block_size);
   const CallSizes sizes{n,       num_heads, num_kv_heads, head_size, block_size,
-                        a.ntiers, width,     kv_dtype,     aligned,   fill};
+                        a.ntiers, width,     kv_dtype,     aligned,   fill,
+                        {a.tier[0].bt_width, a.tier[1].bt_width}};
   size_t need = 0;
   const SplitPlan sp = choose_plan(
       sizes, a.counters != nullptr,
@@ -260,7 +263,7 @@ int workspace_size(int32_t n, int32_t num_heads, int32_t num_kv_heads, int32_t h
                               balanced_counter_bytes(sp, n, num_kv_heads));
     // a two-tier launch with its host tier in pinned memory
     SplitPlan hw = sp;
-    if (plan_host_workers(hw, n, num_heads, num_kv_heads, head_size, block_size, bt_width,
+    if (plan_host_workers(hw, n, num_heads, num_kv_heads, head_size, block_size, bt_width, -1, -1,
                           dts[c]))
       most = std::max(most, balanced_partial_bytes(hw, num_heads, head_size) +
                                 balanced_counter_bytes(hw, n, num_kv_heads));
@@ -314,7 +317,8 @@ int fd_decode_workspace_need(int32_t n, int32_t num_heads, int32_t num_kv_heads,
     return set_error(FD_ERR_INVALID, "workspace_need: bad sizes");
   // (with room for counters, should the caller have none beside its workspace)
   const CallSizes c{n,        num_heads, num_kv_heads, head_size, block_size, 1,
-                    bt_width, kv_dtype,  true,         row_fill(total_tokens, n, bt_width, block_size)};
+                    bt_width, kv_dtype,  true,         row_fill(total_tokens, n, bt_width, block_size),
+                    {bt_width, 0}};
   size_t most = 0;
   for (int matrix = 1; matrix >= (host_tier == 0 ? 1 : 0); --matrix) {
     const SplitPlan sp = plan_decode(n, num_heads, num_kv_heads, head_size, block_size, bt_width,
@@ -323,7 +327,7 @@ int fd_decode_workspace_need(int32_t n, int32_t num_heads, int32_t num_kv_heads,
                                            : decode_workspace_bytes(sp, n, num_heads, head_size));
     SplitPlan hw = sp;
     if (host_tier != 0 && plan_host_workers(hw, n, num_heads, num_kv_heads, head_size, block_size,
-                                            bt_width, kv_dtype))
+                                            bt_width, -1, -1, kv_dtype))
       most = std::max(most, balanced_bytes(hw, c, false));
   }
   *bytes = most;
@@ -369,7 +373,8 @@ int fd_split_decode_plan_info(int32_t n, int32_t num_heads, int32_t num_kv_heads
       (int64_t)hbm_width + host_width > INT32_MAX || !valid_dtype(kv_dtype))
     return set_error(FD_ERR_INVALID, "split_plan_info: bad sizes");
   const CallSizes c{n, num_heads, num_kv_heads, head_size, block_size,
-                    2, (int64_t)hbm_width + host_width, kv_dtype, true, 0.0};
+                    2, (int64_t)hbm_width + host_width, kv_dtype, true, 0.0,
+                    {hbm_width, host_width}};
   size_t need = 0;
   const SplitPlan sp = choose_plan(c, counted != 0, workspace_bytes, false,
                                    [&](int t) { return t == 1 && host_pinned != 0; }, &need);

@@ -728,16 +728,34 @@ size_t decode_workspace_bytes(const SplitPlan& sp, int32_t n, int32_t H, int32_t
 // holds) on decode_mm_kernel's shapes. A CU returns its vector loads in order,
 // so tasks that read both tiers took about the sum of the HBM and link times;
 // with the host tier on 32 workgroups of its own the two overlap, and the HBM
-// parts are cut by the rows' lengths, not by tables that are as wide as the
-// whole context for both tiers. Measured (HIP graph replay, us; HBM + link
-// time in brackets), against the same build without workers: 64 x U[500, 1500],
-// 32/8, a host block each [38 + 40] 82 -> 66; 64/8, 2 % host [37 + 57] 98 -> 77; a
-// layer of 33 x U[40, 1800] with full-width tables 50 -> 42; 8 x 32 heads, 10 %
-// [10 + 119] 133 -> 127; with narrow tables 33 rows 35 -> 38; 24 rows 60 % host
-// [4 + 697] 685 -> 696. 16 workgroups are too few for one-block parts (33 rows:
-// 49), 48 take CUs from the HBM parts (64 rows: 70).
+// parts are cut by the rows' lengths, not by tables that may be as wide as the
+// whole context for both tiers. 16 workgroups are too few for one-block parts
+// (33 rows: 49 us), 48 take CUs from the HBM parts (64 rows: 70).
+//
+// What it gains is the shorter of the two times, and what it costs is that few
+// waves work on the link; the lengths are not known here, the tables' widths
+// are. Measured without -> with (HIP graph replay, us; rows of the given
+// lengths, the share of their blocks in the host tier, "1": the newest):
+//                                       1       5 %        20 %        60 %
+//   64 x U[500, 1500], 32/8          85 -> 67  234 -> 208  893 -> 891  2757 -> 2732
+//   20 x U[200, 900], 64/32          84 -> 72  174 -> 155  653 -> 651  2035 -> 1998
+//   33 x U[40, 1800], 32/8           39 -> 37   95 -> 94   365 -> 383  1109 -> 1128
+//   12 x U[300, 1500], 16/8          23 -> 17   44 -> 40   160 -> 166   488 -> 476
+//   16 x U[300, 2000], 32/8          26 -> 23   69 -> 71   257 -> 265   799 -> 783
+//   40 x U[500, 3000], 8/1           20 -> 15   44 -> 54   148 -> 164   451 -> 460
+//   8 x U[128, 1024], 32/8           16 -> 14   23 -> 23    70 -> 73    221 -> 212
+//   1 x 900, 32/8                    11 -> 10   12 -> 13    21 -> 24     47 -> 49
+//   64 x U[100, 500], 32/32         175 -> 180 192 -> 196  983 -> 1003 3225 -> 3165
+// So: not past 4 (row, kv head) pairs per CU; with a host table of at most a
+// 50th of the HBM table's width, or of half of it and more (rows mostly in the
+// host tier, or tables that hold the whole context for either tier, as a step
+// planned on the device has them: most often the newest blocks spilled);
+// between those from 3/8 of a pair per CU on, down to a 12th. Widths given as
+// -1: whether any widths of bt_width together take it (workspace sizes).
+// FD_HOST_WGS=<w> forces the workers wherever they can be made.
 bool plan_host_workers(SplitPlan& sp, int32_t n, int32_t H, int32_t KVH, int32_t D, int32_t BS,
-                       int32_t bt_width, int32_t kv_dtype) {
+                       int32_t bt_width, int32_t hbm_width, int32_t host_width,
+                       int32_t kv_dtype) {
   const int cus = device_cus();
   const int32_t G = H / KVH;
   // decode_mm_kernel's head sizes and groups (of those of 1 to 3 heads, which
@@ -754,6 +772,12 @@ bool plan_host_workers(SplitPlan& sp, int32_t n, int32_t H, int32_t KVH, int32_t
   const int64_t wt = (int64_t)bt_width * (BS / kTileTokens);
   const int64_t pairs = (int64_t)n * KVH;
   if (wgs <= 0 || wt > kMaxBalBlocks || pairs > kMaxBalPairs) return false;
+  if (tune.host_wgs == nullptr) {
+    const int64_t w0 = hbm_width, w1 = host_width;
+    const bool widths = w0 < 0 || w0 >= 50 * w1 || 2 * w1 >= w0 ||
+                        (8 * pairs >= 3LL * cus && w0 >= 12 * w1);
+    if (pairs > 4LL * cus || !widths) return false;
+  }
   const double units = 2.0 * kTileTokens * D * 2 / kBalTileBytes;
   int64_t want = (5 * pairs <= 2LL * cus ? cus : 2LL * cus) - wgs;
   if (tune.balance != nullptr) want = atoi(tune.balance);

@@ -294,7 +294,7 @@ SplitPlan plan_decode(int32_t n, int32_t H, int32_t KVH, int32_t D, int32_t BS,
 // The plan of a two-tier launch with tier 1, in pinned host memory, on
 // workgroups of its own; false, with sp unchanged, where that does not apply.
 bool plan_host_workers(SplitPlan& sp, int32_t n, int32_t H, int32_t KVH, int32_t D, int32_t BS,
-                       int32_t bt_width, int32_t kv_dtype);
+                       int32_t bt_width, int32_t hbm_width, int32_t host_width, int32_t kv_dtype);
 size_t decode_workspace_bytes(const SplitPlan& sp, int32_t n, int32_t H,
                               int32_t D);
 // Workspace of a plan's balanced launch (0 when it has none): the partials,
