@@ -183,7 +183,8 @@ int fd_paged_decode_partial_hint(
  * their lengths count each row's finished tasks there, so that the last one
  * merges the row; without the array (the other entry points, or NULL) such a
  * launch takes the counters from its workspace and clears them with a small
- * launch of its own first. Same results either way. No counterpart in the
+ * launch of its own first, or, where that costs more than the cut gains, is
+ * cut by table width (the same results within rounding). No counterpart in the
  * reference. */
 int fd_paged_decode_counted(
     const void* q, int64_t q_stride_seq, int64_t q_stride_head,
@@ -304,8 +305,8 @@ int fd_split_decode_plan_info(int32_t n, int32_t num_heads, int32_t num_kv_heads
                               size_t workspace_bytes, int32_t counted, FdDecodePlan* plan,
                               int32_t* parts, int32_t* host_workgroups);
 
-/* Whether a one-tier decode launch of these sizes (aligned, with the workspace
- * the size query asks for) is cut by the rows' lengths on the device instead of by the
+/* Whether a one-tier decode launch of these sizes (aligned, with counters and
+ * the workspace the size query asks for) is cut by the rows' lengths on the device instead of by the
  * table width: *parts is the number of tasks aimed at per kv head and
  * head-group pass, 0 if the cut by table width that fd_decode_plan_info
  * describes is launched (kernel, heads_per_task and passes hold either way).

@@ -147,3 +147,15 @@ done([
     workers(64, 32, 32, 60, 1), workers(65, 32, 8, 112, 1)])
 """)
     assert got == [True, True, True, False, True, False, False, True, True, False, False]
+
+
+def test_uncounted_launches_are_cut_by_length_where_that_pays_for_the_clearing(planner):
+    """A launch that the cut by width leaves whole, counted and not: a table
+    of 28, 48 and 49 blocks; one whose rows it splits."""
+    got = planner("""
+def parts(n, H, KVH, W, counted):
+    return ops.split_plan_info(n, H, KVH, 128, 16, W, 0, torch.float16, counted=counted,
+                               host_pinned=False)["balanced_parts"] > 0
+done([parts(2, 32, 32, w, c) for w in (28, 44, 48, 49, 512) for c in (True, False)])
+""")
+    assert got == [False, False, True, False, True, False, True, True, True, True]

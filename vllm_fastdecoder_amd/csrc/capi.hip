@@ -113,7 +113,8 @@ SplitPlan choose_plan(const CallSizes& c, bool counted, size_t ws_bytes, bool ti
   auto planned = [&](bool matrix) -> SplitPlan {
     SplitPlan sp = plan_decode(c.n, c.H, c.KVH, c.D, c.BS, (int32_t)c.width, c.kv_dtype, c.aligned,
                                matrix, c.fill);
-    if (timeline || balanced_bytes(sp, c, counted) > ws_bytes) sp.bal_parts = 0;
+    if (timeline || !(counted || sp.bal_uncounted) || balanced_bytes(sp, c, counted) > ws_bytes)
+      sp.bal_parts = 0;
     return sp;
   };
   auto needs = [&](const SplitPlan& sp) -> size_t {

@@ -475,9 +475,18 @@ int32_t quarter_row_blocks(int32_t n, int32_t kv_tasks, int32_t D, bool f32, boo
 //     ~0.8 us for the cut itself): checked here against the table width,
 //     which bounds the row, and in the kernel against the row. 8 x 32 rows of
 //     U[128, 1024] (whole rows 15.7 us) lose cut (16.5).
+//   * without the caller's arrival counters a launch clears its own first, in
+//     a launch that costs 1.5 us in a graph and up to 4 us between eager
+//     calls. Where the cut by width splits rows, a combine launch goes in
+//     return; where it does not (one launch before), the table has to be
+//     kBalClear blocks wider. By width / cleared / counted: 2 x U[500, 700],
+//     32/32, fp16 (44 blocks) 10.2 / 10.7 / 8.6; 3 x U[300, 900], 32/8 (57)
+//     11.8 / 9.0 / 7.6; 1 x 900 (57) 13.0 / 8.8 / 7.4; 8 x U[128, 1024], 32/8
+//     (64) 17.1 / 10.5 / 9.0; 16 of them 17.8 / 14.0 / 12.4.
 // FD_SPLIT_BLOCKS (forced tasks) turns the cuts off.
 constexpr double kBalTileBytes = 8192.0;  // the unit of the figures below
 constexpr double kBalMerge = 20.0;        // blocks one task streams in the time a merge adds
+constexpr double kBalClear = 20.0;        // and in the time that clearing counters may add
 constexpr double kBalRates = 1.65;        // a task's own rate (45 GB/s) over a 256th of HBM's
 constexpr double kBalMinBlocks = 8.0;     // smallest part (4: 9.2 us instead of 9.1 above, 16: 10.5)
 
@@ -529,6 +538,8 @@ void plan_balanced(SplitPlan& sp, const Tuning& tune, int32_t n, int32_t H, int3
   }
   if (want <= 0 || pairs > kMaxBalPairs) return;
   cut_balanced(sp, tune, n, H, D, kv_tasks, wt, least, whole, want, cus);
+  sp.bal_uncounted = tune.balance != nullptr || sp.max_splits > 1 ||
+                     wt > least + whole + (int32_t)(kBalClear / units);
 }
 
 }  // namespace

@@ -278,6 +278,7 @@ struct SplitPlan {
   int32_t bal_cap;       // its wg_cap,
   int32_t bal_slots;     // partials per query head (the grid's parts, and host workers'),
   int32_t host_wgs;      // workgroups that take tier 1's blocks alone (two tiers; 0: none),
+  bool bal_uncounted;    // the cuts also gain where the launch clears its own counters,
   int32_t bal_whole;     // and balanced_task's figures for leaving rows whole
   float bal_share;
   int* occupancy_query;  // planner only: when set, the tiled launchers store the selected
