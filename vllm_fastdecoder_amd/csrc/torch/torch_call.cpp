@@ -1,5 +1,5 @@
-// The ordinary form of ops.paged_decode, ops.split_decode and the cache write
-// taken from torch tensors straight to the C ABI, in one native call.
+// The ordinary form of ops.paged_decode and of the cache writes taken from
+// torch tensors straight to the C ABI, in one native call.
 //
 // What bounds a small launch is the host: through ctypes a decode call took
 // 13-15 us (about forty attribute reads and checks in Python, two tensor
@@ -291,77 +291,6 @@ PyObject* paged_decode(PyObject*, PyObject* const* a, Py_ssize_t na) {
   });
 }
 
-// split_decode(q, hbm_k, hbm_v, hbm_bt, hbm_lens, host_k, host_v, host_bt,
-//              host_lens, scale, out, lse, row_order)
-PyObject* split_decode(PyObject*, PyObject* const* a, Py_ssize_t na) {
-  return guarded([&]() -> PyObject* {
-    if (na != 13 || modes_active()) return not_here();
-    const at::Tensor* q = query(a[0]);
-    const at::Tensor* k = plain(a[1]);
-    const at::Tensor* v = plain(a[2]);
-    const at::Tensor* hk = plain(a[5]);
-    const at::Tensor* hv = plain(a[6]);
-    const at::Tensor *bt, *lens, *hbt, *hlens;
-    if (q == nullptr || k == nullptr || v == nullptr || hk == nullptr || hv == nullptr ||
-        k->dim() != 4 || hk->dim() != 4 || !same_layout(*k, *v) || !same_layout(*hk, *hv) ||
-        !index_pair(*q, a[3], a[4], &bt, &lens) || !index_pair(*q, a[7], a[8], &hbt, &hlens) ||
-        !PyFloat_CheckExact(a[9]))
-      return not_here();
-    for (const at::Tensor* t : {k, v, hk, hv})
-      if (t->scalar_type() != q->scalar_type() || t->stride(3) != 1 ||
-          !(t->is_cuda() ? t->device() == q->device() : t->is_cpu()))
-        return not_here();
-    const int64_t n = q->size(0), H = q->size(1), D = q->size(2);
-    const int64_t BS = k->size(1), KVH = k->size(2);
-    if (k->size(3) != D || hk->size(3) != D || hk->size(1) != KVH || hk->size(2) != BS ||
-        KVH == 0 || H % KVH != 0 || !fits32(H) || !fits32(D) || !fits32(BS) || BS == 0)
-      return not_here();
-    const int32_t* order;
-    if (!order_of(*q, a[12], &order)) return not_here();
-    Outputs o(*q, a[10], a[11]);
-    const int64_t width = bt->size(1) + hbt->size(1);
-    if (!o.ok || !fits32(width)) return not_here();
-    const int kv = dtype_code(q->scalar_type());
-    size_t need = 0, need_hbm = 0;
-    for (int host = 0; host < 2; ++host)  // a tier in pinned memory takes other kernels
-      if (fd_decode_workspace_need((int32_t)n, (int32_t)H, (int32_t)KVH, (int32_t)D, (int32_t)BS,
-                                   (int32_t)width, kv, host, 0, host ? &need : &need_hbm) != FD_OK)
-        return not_here();
-    need = std::max(need, need_hbm);
-    fd_kv_tier t0{}, t1{};
-    if (!cache_ptr(a[1], *k, &t0.k_cache) || !cache_ptr(a[2], *v, &t0.v_cache) ||
-        !cache_ptr(a[5], *hk, &t1.k_cache) || !cache_ptr(a[6], *hv, &t1.v_cache))
-      return nullptr;
-    auto fill = [](fd_kv_tier& t, const at::Tensor& c, int head, int token, const at::Tensor& b,
-                   const at::Tensor& l) {
-      t.stride_block = c.stride(0);
-      t.stride_head = c.stride(head);
-      t.stride_token = c.stride(token);
-      t.num_blocks = c.size(0);
-      t.block_table = b.data_ptr<int32_t>();
-      t.bt_stride = b.stride(0);
-      t.bt_width = (int32_t)b.size(1);
-      t.lens = l.data_ptr<int32_t>();
-    };
-    fill(t0, *k, 2, 1, *bt, *lens);
-    fill(t1, *hk, 1, 2, *hbt, *hlens);
-    if (!o.allocate(*q)) return not_here();
-    PyRef hold;
-    void *ws, *stream;
-    size_t ws_bytes;
-    uint32_t* counters;
-    if (!current_stream(q->get_device(), &stream) ||
-        !workspace(*q, need, stream, hold, &ws, &ws_bytes, &counters))
-      return nullptr;
-    const int status = without_gil([&] { return fd_split_decode_counted(
-        q->data_ptr(), q->stride(0), q->stride(1), &t0, &t1, order, (int32_t)n, (int32_t)H,
-        (int32_t)KVH, (int32_t)D, (int32_t)BS, (float)PyFloat_AS_DOUBLE(a[9]), kv,
-        o.out.data_ptr(), o.out.stride(0), o.out.stride(1), dtype_code(o.out.scalar_type()),
-        o.lse.data_ptr<float>(), o.lse.stride(0), ws, ws_bytes, stream, counters); });
-    return result(status, o);
-  });
-}
-
 // key and value rows [T, KVH, D] of one shape, T given by the slots.
 bool kv_rows(const at::Tensor* key, const at::Tensor* value) {
   return key != nullptr && value != nullptr && key->is_cuda() && value->device() == key->device() &&
@@ -481,8 +410,6 @@ PyObject* init(PyObject*, PyObject* args) {
 PyMethodDef methods[] = {
     {"init", init, METH_VARARGS, nullptr},
     {"paged_decode", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(paged_decode)),
-     METH_FASTCALL, nullptr},
-    {"split_decode", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(split_decode)),
      METH_FASTCALL, nullptr},
     {"cache_write", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(cache_write)),
      METH_FASTCALL, nullptr},
