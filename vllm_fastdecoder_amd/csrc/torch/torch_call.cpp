@@ -214,13 +214,15 @@ PyObject* result(int status, const Outputs& o) {
 }
 
 // Runs a library call without the GIL: a launch may wait for room in its
-// queue, as torch's own launches do without it.
+// queue, as torch's own launches do without it. The GIL is back before an
+// exception (a tensor's data_ptr may throw) leaves.
 template <typename F>
 int without_gil(F&& f) {
-  PyThreadState* save = PyEval_SaveThread();
-  const int status = f();
-  PyEval_RestoreThread(save);
-  return status;
+  struct Released {
+    PyThreadState* save = PyEval_SaveThread();
+    ~Released() { PyEval_RestoreThread(save); }
+  } released;
+  return f();
 }
 
 // No C++ exception leaves an entry point: it becomes a Python RuntimeError.
