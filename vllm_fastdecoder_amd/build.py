@@ -54,10 +54,13 @@ TORCH_CALL_PATH = PKG_DIR / "_torch_call.so"
 def torch_call_command(out: Path, lib: Path) -> list[str]:
     import sysconfig
 
+    import torch
     from torch.utils import cpp_extension
 
     libs = cpp_extension.library_paths()[0]
-    return [cxx(), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D_GLIBCXX_USE_CXX11_ABI=1",
+    return [cxx(), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            f'-DFD_BUILT_FOR_TORCH="{torch.__version__}"',
             *(f"-isystem{p}" for p in cpp_extension.include_paths()),
             f"-isystem{sysconfig.get_paths()['include']}", str(TORCH_CALL_SRC), "-o", str(out),
             str(lib), f"-L{libs}", "-Wl,-rpath,$ORIGIN", f"-Wl,-rpath,{libs}",

@@ -26,6 +26,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <algorithm>
+#include <cstring>
 
 #include "../../../include/fdattn.h"
 
@@ -396,10 +397,20 @@ PyObject* cache_write_tiers(PyObject*, PyObject* const* a, Py_ssize_t na) {
   });
 }
 
-// init(WORKSPACE.get, pinned.device_ptr, raw current-stream query)
+// init(WORKSPACE.get, pinned.device_ptr, raw current-stream query,
+//      torch.__version__): an ImportError where the module was built against
+// another torch, whose tensors it would read by the wrong layout, or beside a
+// library of another ABI.
 PyObject* init(PyObject*, PyObject* args) {
   PyObject *ws, *dp, *rs;
-  if (!PyArg_ParseTuple(args, "OOO", &ws, &dp, &rs)) return nullptr;
+  const char* torch_version;
+  if (!PyArg_ParseTuple(args, "OOOs", &ws, &dp, &rs, &torch_version)) return nullptr;
+  if (strcmp(torch_version, FD_BUILT_FOR_TORCH) != 0)
+    return PyErr_Format(PyExc_ImportError, "_torch_call was built for torch %s, not %s",
+                        FD_BUILT_FOR_TORCH, torch_version);
+  if (fd_abi_version() != FD_ABI_VERSION)
+    return PyErr_Format(PyExc_ImportError, "_torch_call was built for ABI %d of the library, not %d",
+                        FD_ABI_VERSION, fd_abi_version());
   Py_INCREF(ws);
   Py_INCREF(dp);
   Py_INCREF(rs);

@@ -205,15 +205,16 @@ _NATIVE = None  # the native call module; False once it could not be loaded
 def _native():
     """The native call path (csrc/torch/torch_call.cpp): ordinary calls go
     from the tensors straight to the C ABI. False where the module cannot be
-    loaded (built for another torch): every call then takes the checks below
-    and ctypes, with the same kernels and results."""
+    loaded or says it was built for another torch or library: every call then
+    takes the checks below and ctypes, with the same kernels and results."""
     global _NATIVE
     if _NATIVE is None:
         _lib.load_lib()  # a missing or stale library fails here
         try:
             from . import _torch_call
 
-            _torch_call.init(WORKSPACE.get, device_ptr, torch._C._cuda_getCurrentRawStream)
+            _torch_call.init(WORKSPACE.get, device_ptr, torch._C._cuda_getCurrentRawStream,
+                             torch.__version__)
             _NATIVE = _torch_call
         except (ImportError, AttributeError) as e:
             logging.getLogger("fastdecode").warning(
