@@ -256,6 +256,10 @@ int fd_decode_workspace_need(int32_t n, int32_t num_heads, int32_t num_kv_heads,
  * reference. */
 int fd_in_host_memory(const void* p, int32_t* host);
 
+/* *capturing: 1 while the stream records a graph. No counterpart in the
+ * reference. */
+int fd_stream_capturing(void* stream, int32_t* capturing);
+
 /* Which kernel a decode launch of these sizes takes, and how it is cut into
  * tasks (the planner of fd_paged_decode_partial / fd_split_decode, on the
  * current device). No counterpart in the reference; for tests and for

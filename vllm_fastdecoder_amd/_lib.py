@@ -157,6 +157,7 @@ SIGNATURES: dict[str, tuple] = {
          c_int32, c_int32, c_int64,                             # kv_dtype, host_tier, total_tokens
          POINTER(c_size_t)],
     ),
+    "fd_stream_capturing": (c_int, [c_void_p, POINTER(c_int32)]),
     "fd_in_host_memory": (c_int, [c_void_p, POINTER(c_int32)]),
     "fd_decode_plan_info": (
         c_int,

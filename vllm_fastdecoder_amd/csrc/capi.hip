@@ -341,6 +341,15 @@ int fd_in_host_memory(const void* p, int32_t* host) {
   return FD_OK;
 }
 
+int fd_stream_capturing(void* stream, int32_t* capturing) {
+  if (capturing == nullptr) return set_error(FD_ERR_INVALID, "stream_capturing: NULL result");
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  const hipError_t e = hipStreamIsCapturing(static_cast<hipStream_t>(stream), &st);
+  if (e != hipSuccess) return hip_error(e, "hipStreamIsCapturing");
+  *capturing = st == hipStreamCaptureStatusNone ? 0 : 1;
+  return FD_OK;
+}
+
 int fd_decode_plan_info(int32_t n, int32_t num_heads, int32_t num_kv_heads, int32_t head_size,
                         int32_t block_size, int32_t bt_width, int32_t kv_dtype, int32_t aligned,
                         int32_t host_tier, int64_t total_tokens, FdDecodePlan* plan) {

@@ -115,7 +115,10 @@ bool workspace(const at::Tensor& q, size_t need, void* stream, PyRef& hold, void
   if (dev.p == nullptr) return false;
   PyRef n(PyLong_FromSize_t(need)), s(PyLong_FromVoidPtr(stream));
   if (n.p == nullptr || s.p == nullptr) return false;
-  hold.p = PyObject_CallFunctionObjArgs(g_workspace_get, dev.p, n.p, s.p, nullptr);
+  int32_t capturing = 1;  // (an error: the slower answer is right in either case)
+  (void)fd_stream_capturing(stream, &capturing);
+  hold.p = PyObject_CallFunctionObjArgs(g_workspace_get, dev.p, n.p, s.p, Py_False,
+                                        capturing != 0 ? Py_True : Py_False, nullptr);
   if (hold.p == nullptr) return false;
   const at::Tensor& buf = THPVariable_Unpack(hold.p);
   *ws = buf.data_ptr();

@@ -115,14 +115,21 @@ class _Workspace:
         return idx, _current_stream(idx) if stream is None else int(stream)
 
     def get(self, device: torch.device, nbytes: int, stream: int | None = None,
-            pin: bool = False) -> torch.Tensor | None:
+            pin: bool = False, capturing: bool | None = None) -> torch.Tensor | None:
         """The workspace of `stream` (a raw handle; the current stream on
         `device`, the one the caller's launch goes on, unless only room is
-        made for it), at least nbytes long. pin: keep this stream's buffers alive (see above)."""
+        made for it), at least nbytes long. pin: keep this stream's buffers
+        alive (see above). capturing: whether the stream records a graph,
+        where the caller has asked."""
         if nbytes == 0 and not pin:
             return None
-        key = self._key(device, stream)
-        if not pin and key not in self._pinned and _capturing():
+        idx = device.index
+        if stream is None or idx is None:
+            key = self._key(device, stream)
+        else:
+            key = (idx, stream)
+        if (not pin and key not in self._pinned
+                and (_capturing() if capturing is None else capturing)):
             # (freed when the caller drops it, to the pool that torch keeps for
             # this graph: only its later captured work uses that)
             return self._allocate(key, nbytes)
