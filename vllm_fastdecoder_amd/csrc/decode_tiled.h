@@ -875,6 +875,15 @@ __device__ __forceinline__ bool count_arrival(const TiledParams& p, const Task& 
   return done;
 }
 
+// This wave's partial stores are done (vmcnt(0)). The fences emit nothing:
+// they keep the compiler from moving the stores, or the arrival, across the
+// wait.
+__device__ __forceinline__ void partial_written() {
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  __builtin_amdgcn_s_waitcnt(0x0F70);
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+}
+
 // Whether the tasks of this row still to come leave the merge to this one: a
 // balanced launch has no combine pass; the last of a row's parts to arrive
 // merges them. Called by the whole workgroup once its partial is written;
@@ -883,11 +892,13 @@ __device__ __forceinline__ bool count_arrival(const TiledParams& p, const Task& 
 // parts with sc1 loads, so no cache is written back or invalidated (an
 // agent-scope release / acquire pair does both, and held launches up to 2x).
 __device__ __forceinline__ bool last_to_arrive(const TiledParams& p, const Task& t, int* last) {
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's partial stores are done
+  partial_written();
   __syncthreads();
   if (threadIdx.x == 0) *last = count_arrival(p, t) ? 1 : 0;
   __syncthreads();
-  return __builtin_amdgcn_readfirstlane(*last) != 0;
+  const bool merge = __builtin_amdgcn_readfirstlane(*last) != 0;
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");  // no part is read before
+  return merge;
 }
 
 // Merges the row's parts and writes its result (thread `tid` of `threads`: the
@@ -968,10 +979,12 @@ __device__ __forceinline__ void end_task(const TiledParams& p, const Task& t, Wa
 template <typename T, int D>
 __device__ __forceinline__ void end_solo_part(const TiledParams& p, const Task& t, int lane) {
   if (t.nsplit == 1) return;
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), as in last_to_arrive
+  partial_written();
   int last = 0;
   if (lane == 0) last = count_arrival(p, t) ? 1 : 0;
-  if (__builtin_amdgcn_readfirstlane(last) != 0) merge_parts<T, D>(p, t, lane, kWave);
+  const bool merge = __builtin_amdgcn_readfirstlane(last) != 0;
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");  // no part is read before
+  if (merge) merge_parts<T, D>(p, t, lane, kWave);
 }
 
 // Query head of the task's head slot g: slots past the task's heads repeat
