@@ -81,10 +81,12 @@ def _check(got, dtype, rows=None):
     assert torch.all(out[~nz] == 0) and torch.all(torch.isneginf(lse[:, ~nz]))
 
 
+@pytest.mark.parametrize("divided", ["1", "0"])
 @pytest.mark.parametrize("split", ["256", "32"])
 @pytest.mark.parametrize("H,KVH,D,dtype", [(2, 2, 128, torch.float16), (4, 1, 128, torch.bfloat16),
                                            (2, 1, 256, torch.float16), (2, 2, 64, torch.float32)])
-def test_tier_shares(gpu, H, KVH, D, dtype, split, monkeypatch):
+def test_tier_shares(gpu, H, KVH, D, dtype, split, divided, monkeypatch):
+    monkeypatch.setenv("FD_TIER_WAVES", divided)
     monkeypatch.setenv("FD_SPLIT_BLOCKS", split)
     _check(_run(gpu, H, KVH, D, dtype, ROWS), dtype)
 

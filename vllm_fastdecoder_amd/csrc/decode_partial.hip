@@ -194,7 +194,8 @@ __global__ __launch_bounds__(kWave) void decode_generic_kernel(GenericParams p) 
 //   FD_WG_CAP=<k>        at most k workgroups per CU (0: no cap);
 //   FD_BALANCE=<w>       balanced cuts aiming at w workgroups wherever they can be made
 //                        (0: none);
-//   FD_HOST_WGS=<w>      w workgroups for a host tier in pinned memory (0: none).
+//   FD_HOST_WGS=<w>      w workgroups for a host tier in pinned memory (0: none);
+//   FD_TIER_WAVES=<0|1>  tasks over both tiers never / always divide their waves.
 // Like getenv, the first definition of a name counts.
 struct Tuning {
   const char* split_blocks = nullptr;
@@ -204,6 +205,7 @@ struct Tuning {
   const char* wg_cap = nullptr;
   const char* balance = nullptr;
   const char* host_wgs = nullptr;
+  const char* tier_waves = nullptr;
 
   bool kernel_forced(const char* name) const {
     return kernel != nullptr && strcmp(kernel, name) == 0;
@@ -229,6 +231,7 @@ Tuning read_tuning() {
     else if (!t.wg_cap && (v = value(s, "WG_CAP"))) t.wg_cap = v;
     else if (!t.balance && (v = value(s, "BALANCE"))) t.balance = v;
     else if (!t.host_wgs && (v = value(s, "HOST_WGS"))) t.host_wgs = v;
+    else if (!t.tier_waves && (v = value(s, "TIER_WAVES"))) t.tier_waves = v;
   }
   return t;
 }
@@ -915,6 +918,12 @@ int launch_decode(const DecodeArgs& a, const SplitPlan& sp, hipStream_t s) {
   tp.split_blocks = sp.split_blocks;
   tp.wave_blocks = sp.wave_blocks;
   tp.xcd_group = a.D % 64 != 0;
+  if (two) {  // see wave_blocks()
+    const Tuning tune = read_tuning();
+    tp.tier_waves = tune.tier_waves != nullptr
+                        ? atoi(tune.tier_waves) > 0
+                        : (int64_t)a.n * a.KVH * sp.passes >= 3LL * device_cus();
+  }
   tp.timeline = a.timeline;
   const bool balanced = sp.bal_parts > 0;
   const size_t parts = (size_t)a.n * a.H * sp.max_splits;

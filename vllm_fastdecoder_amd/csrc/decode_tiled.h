@@ -92,6 +92,7 @@ struct TiledParams {
   uint64_t* counters; // balanced cuts: arrivals per (sequence, kv-head pass) (count_arrival())
   uint64_t launch;    // balanced cuts: this launch's number, kArrivalBits up
   int32_t counter_stride;  // balanced cuts: counters are this many words apart
+  bool tier_waves;  // two tiers: a task's waves are divided between them (wave_blocks())
   bool xcd_group;   // adjacent kv heads of a row on one XCD (xcd_task)
   uint64_t* timeline;  // measurement only: kTimelineSlots stamps per workgroup (NULL: none)
 };
@@ -637,19 +638,25 @@ __device__ __forceinline__ WaveBlocks wave_blocks(const TiledParams& p, const Ta
   w.nw = wave < ws && w.first < t.b_end ? (t.b_end - w.first + ws - 1) / ws : 0;
   w.k1 = TWO ? (t.nba > w.first ? (t.nba - w.first + ws - 1) / ws : 0) : w.nw;
   if constexpr (TWO) {
-    // A range with blocks of both tiers: the last `h` waves take tier 1's
-    // (one to three waves, by its share of the blocks), the others tier 0's:
-    // a wave that waits for the link holds up no HBM blocks, and the link is
-    // busy from the start. Measured with the shorter host reads of block_src
-    // (HIP graph replay, us; HBM and link time of the bytes in brackets):
-    // 33 rows of U[40, 1800], 32/8, one host block each [15 + 21] 53 -> 45;
-    // 24 x 32 heads of U[256, 1024], 7.5 % host [35 + 303] 362 -> 316; 8 x 32,
-    // 10 % [10 + 119] 146 -> 132; 60 % host [15 + 2787] 2783 -> 2761.
+    // A range with blocks of both tiers, in a launch of many tasks
+    // (p.tier_waves): the last `h` waves take tier 1's (one to three waves, by
+    // its share of the blocks), the others tier 0's: a wave that waits for the
+    // link holds up no HBM blocks, and the link is busy from the start.
+    // Measured without -> with (HIP graph replay, us; the newest block of each
+    // row in the host tier, 7.5 %, 30 %): 100 x U[300, 900], 32/8, bf16 89 -> 85,
+    // 303 -> 301, 1312 -> 1285; 100 x U[200, 900], 32/8, fp32 178 -> 163, 565 ->
+    // 570, 2698 -> 2504; 120 x U[200, 900], 16/8, D = 256 189 -> 172, 656 -> 662,
+    // 2915 -> 2902; 90 x U[100, 600], 32/32 249 -> 241, 562 -> 557, 2628 -> 2608.
+    // Where the tasks are fewer, the few waves on the link are what the launch
+    // waits for: 8 x U[128, 1024], 32/32, fp32 54 -> 69, 177 -> 195, 799 -> 783;
+    // 40 x U[200, 1500], 16/8, D = 256 87 -> 108, 354 -> 392, 1488 -> 1507; 20 x
+    // U[200, 900], 64/32 79 -> 85. 24 x U[256, 1024], 32/32, three tasks per CU:
+    // 83 -> 78 us. The line lies there.
     const int na = min(t.nba, t.b_end) - t.b_begin;
     const int nh = t.b_end - t.b_begin - na;
     const int h = min(kWavesPerTask - 1, max(1, (4 * nh + (na + nh) / 2) / max(na + nh, 1)));
     const int wa = kWavesPerTask - h;
-    if (na > 0 && nh > 0 && ws == kWavesPerTask && na <= wa * kMaxWaveBlocks &&
+    if (p.tier_waves && na > 0 && nh > 0 && ws == kWavesPerTask && na <= wa * kMaxWaveBlocks &&
         nh <= h * kMaxWaveBlocks) {
       const bool host = wave >= wa;
       w.stride = host ? h : wa;
