@@ -127,7 +127,7 @@ SplitPlan choose_plan(const CallSizes& c, bool counted, size_t ws_bytes, bool ti
   // host memory take the VALU kernel. A two-tier launch on decode_mm_kernel
   // reads its host blocks in whole rows and stays there for its HBM blocks,
   // most of which the VALU kernel's per-head work holds up (33 rows of
-  // U[40, 1800], 32/8, one host block each: 44 -> 39 us; 64 of U[500, 1500]: 96 -> 85).
+  // U[40, 1800], 32/8, one host block each: 42 -> 34 us; 64 of U[500, 1500]: 79 -> 72).
   bool host = false;
   const int read_in_rows = c.ntiers > 1 && sp.mm ? 1 : 0;  // of the tiers, the last
   for (int t = 0; (sp.mfma || sp.mm) && t < c.ntiers - read_in_rows; ++t) host = host || pinned(t);

@@ -751,22 +751,27 @@ size_t decode_workspace_bytes(const SplitPlan& sp, int32_t n, int32_t H, int32_t
 // are. Measured without -> with (HIP graph replay, us; rows of the given
 // lengths, the share of their blocks in the host tier, "1": the newest):
 //                                       1       5 %        20 %        60 %
-//   64 x U[500, 1500], 32/8          85 -> 67  234 -> 208  893 -> 891  2757 -> 2732
-//   20 x U[200, 900], 64/32          84 -> 72  174 -> 155  653 -> 651  2035 -> 1998
-//   33 x U[40, 1800], 32/8           39 -> 37   95 -> 94   365 -> 383  1109 -> 1128
-//   12 x U[300, 1500], 16/8          23 -> 17   44 -> 40   160 -> 166   488 -> 476
-//   16 x U[300, 2000], 32/8          26 -> 23   69 -> 71   257 -> 265   799 -> 783
-//   40 x U[500, 3000], 8/1           20 -> 15   44 -> 54   148 -> 164   451 -> 460
-//   8 x U[128, 1024], 32/8           16 -> 14   23 -> 23    70 -> 73    221 -> 212
-//   1 x 900, 32/8                    11 -> 10   12 -> 13    21 -> 24     47 -> 49
-//   64 x U[100, 500], 32/32         175 -> 180 192 -> 196  983 -> 1003 3225 -> 3165
-// So: not past 4 (row, kv head) pairs per CU; with a host table of at most a
-// 50th of the HBM table's width, or of half of it and more (rows mostly in the
-// host tier, or tables that hold the whole context for either tier, as a step
-// planned on the device has them: most often the newest blocks spilled);
-// between those from 3/8 of a pair per CU on, down to a 12th. Widths given as
-// -1: whether any widths of bt_width together take it (workspace sizes).
-// FD_HOST_WGS=<w> forces the workers wherever they can be made.
+//   64 x U[500, 1500], 32/8          72 -> 68  219 -> 208  916 -> 894  2740 -> 2735
+//   20 x U[200, 900], 64/32          79 -> 71  161 -> 158  657 -> 647  2017 -> 2002
+//   12 x U[300, 1500], 16/8          21 -> 18   43 -> 40   157 -> 166   487 -> 476
+//   16 x U[300, 2000], 32/8          25 -> 23   71 -> 70   257 -> 266   793 -> 783
+//   40 x U[500, 3000], 8/1           18 -> 15   45 -> 55   148 -> 164   453 -> 460
+//   8 x U[128, 1024], 32/8           15 -> 14   24 -> 23    70 -> 73    224 -> 212
+//   2 x U[500, 1500], 32/8           12 -> 12   16 -> 18    42 -> 43    115 -> 108
+//   33 x U[40, 1800], 32/8           34 -> 39   94 -> 94   366 -> 383  1111 -> 1129
+//   the same, full-width tables      31 -> 38   92 -> 94   364 -> 382  1117 -> 1130
+//   48 x U[200, 2000], 28/4          33 -> 37   99 -> 98   375 -> 388  1153 -> 1135
+//   8 x U[128, 1024], 32/32          31 -> 36   68 -> 67   254 -> 258   818 -> 795
+//   64 x U[100, 500], 32/32         174 -> 180 193 -> 196  981 -> 1003 3223 -> 3160
+// So: not past 4 (row, kv head) pairs per CU, nor at about one, where each CU
+// has a whole row and nothing needs cutting; else with a host table of at most
+// a 50th of the HBM table's width, or of half of it and more (rows mostly in
+// the host tier, or tables that hold the whole context for either tier, as a
+// step planned on the device has them: most often the newest blocks spilled;
+// below 32 pairs only if the host table is the wider), and between those from
+// 3/8 of a pair per CU on, down to a 12th. Widths given as -1: whether any
+// widths of bt_width together take it (workspace sizes). FD_HOST_WGS=<w>
+// forces the workers wherever they can be made.
 bool plan_host_workers(SplitPlan& sp, int32_t n, int32_t H, int32_t KVH, int32_t D, int32_t BS,
                        int32_t bt_width, int32_t hbm_width, int32_t host_width,
                        int32_t kv_dtype) {
@@ -788,8 +793,10 @@ bool plan_host_workers(SplitPlan& sp, int32_t n, int32_t H, int32_t KVH, int32_t
   if (wgs <= 0 || wt > kMaxBalBlocks || pairs > kMaxBalPairs) return false;
   if (tune.host_wgs == nullptr) {
     const int64_t w0 = hbm_width, w1 = host_width;
-    const bool widths = w0 < 0 || w0 >= 50 * w1 || 2 * w1 >= w0 ||
+    const bool widths = w0 < 0 || w0 >= 50 * w1 || (2 * w1 >= w0 && (pairs >= 32 || w1 > w0)) ||
                         (8 * pairs >= 3LL * cus && w0 >= 12 * w1);
+    const bool row_per_cu = 4 * pairs >= 3LL * cus && 4 * pairs <= 5LL * cus;
+    if (row_per_cu) return false;
     if (pairs > 4LL * cus || !widths) return false;
   }
   const double units = 2.0 * kTileTokens * D * 2 / kBalTileBytes;
