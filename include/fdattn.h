@@ -202,8 +202,9 @@ int fd_paged_decode_counted(
     void* stream, int64_t total_tokens, uint32_t* counters);
 
 /* Measurement helper: fd_paged_decode_partial (same arguments; the same bits
- * where fd_decode_balanced_parts gives 0, within rounding otherwise) that also records when each workgroup of the decode launch reaches a few
- * points, for launches that take the 16-bit VALU kernel (otherwise
+ * where fd_decode_balanced_parts gives 0, within rounding otherwise) that also
+ * records when each workgroup of the decode launch reaches a few points, for
+ * launches that take the 16-bit VALU kernel (otherwise
  * FD_ERR_UNSUPPORTED, nothing launched). timeline: a device buffer of
  * timeline_workgroups * 8 uint64 (16-byte aligned, zeroed by the caller);
  * a launch of more workgroups is FD_ERR_INVALID. Words of workgroup w, at
@@ -365,9 +366,10 @@ int fd_paged_decode_partial_noalloc(
  *   lse[h, i]    = logsumexp over both tiers (natural log),
  * which equals merge(partial_hbm, partial_host) of the separate calls. The
  * kernel takes each row's HBM-tier and host-tier blocks as one list and merges
- * in-kernel: no partial round trip and no merge launch. Up to 64 rows over a
- * host tier in pinned memory, some workgroups take the host tier's blocks and
- * the others the HBM tier's, so that the link and HBM are read at once.
+ * in-kernel: no partial round trip and no merge launch. In some launches of up
+ * to 64 rows over a host tier in pinned memory (fd_split_decode_plan_info)
+ * some workgroups take the host tier's blocks and the others the HBM tier's,
+ * so that the link and HBM are read at once.
  *
  * Each tier is described by an fd_kv_tier: the same cache/stride/table/length
  * conventions as fd_paged_decode_partial, per tier (tier-relative block ids,
