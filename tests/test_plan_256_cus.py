@@ -143,17 +143,17 @@ def workers(n, H, KVH, a, b, D=128):
 done([
     workers(64, 32, 8, 112, 1), workers(64, 32, 8, 100, 2), workers(64, 32, 8, 112, 112),
     workers(40, 8, 1, 178, 10), workers(12, 16, 8, 88, 5), workers(12, 16, 8, 59, 5),
-    workers(2, 32, 8, 46, 11), workers(2, 32, 8, 22, 11), workers(2, 32, 8, 11, 22),
-    workers(4, 32, 8, 22, 22), workers(24, 32, 8, 112, 1), workers(23, 32, 8, 112, 1),
-    workers(40, 32, 8, 112, 112), workers(41, 32, 8, 112, 112),
-    workers(64, 16, 16, 60, 1), workers(64, 32, 32, 60, 1), workers(65, 32, 8, 112, 1)])
+    workers(2, 32, 8, 46, 11), workers(2, 32, 8, 22, 11), workers(2, 32, 8, 22, 44),
+    workers(24, 32, 8, 31, 31), workers(24, 32, 8, 32, 32), workers(24, 32, 8, 16, 32),
+    workers(64, 16, 16, 32, 32), workers(33, 32, 32, 63, 63), workers(33, 32, 32, 64, 64),
+    workers(65, 32, 8, 112, 1)])
 """)
     assert got == [True, True, True,
                    False, True, False,
                    False, False, True,
+                   False, True, True,
                    True, False, True,
-                   False, True,
-                   True, False, False]
+                   False]
 
 
 def test_uncounted_launches_are_cut_by_length_where_that_pays_for_the_clearing(planner):

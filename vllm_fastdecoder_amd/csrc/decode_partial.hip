@@ -748,8 +748,20 @@ size_t decode_workspace_bytes(const SplitPlan& sp, int32_t n, int32_t H, int32_t
 //
 // What it gains is the shorter of the two times, and what it costs is that few
 // waves work on the link; the lengths are not known here, the tables' widths
-// are. Measured without -> with (HIP graph replay, us; rows of the given
-// lengths, the share of their blocks in the host tier, "1": the newest):
+// are. Measured without -> with (HIP graph replay, us; the rows' lengths, the
+// share of their blocks in the host tier, "1": the newest block of each).
+// Tables as wide as the whole context for either tier, as a step planned on
+// the device has them; rows of U[L, 2L], 32 query heads, widths of 2L:
+//   rows x kv heads      1, L = 60      120        250        450        800     10 %, 250   450
+//   1 x 8                 8 -> 10    8 -> 10   12 -> 10   10 -> 10   11 -> 10   13 -> 12   14 -> 16
+//   24 x 8               23 -> 28   22 -> 28   26 -> 27   34 -> 28   42 -> 37   63 -> 66  126 -> 122
+//   40 x 8               37 -> 43   37 -> 42   41 -> 42   50 -> 42   62 -> 59  105 -> 106 217 -> 209
+//   64 x 8               47 -> 53   49 -> 53   58 -> 58   62 -> 55   76 -> 77  170 -> 168 293 -> 288
+//   8 x 32               26 -> 28   24 -> 26   37 -> 34   36 -> 30   42 -> 34   92 -> 91  179 -> 170
+//   24 x 32              70 -> 76   67 -> 71   71 -> 73   90 -> 78  111 -> 101 228 -> 227 463 -> 457
+//   56 x 32             138 -> 149 150 -> 158 148 -> 157 150 -> 155 223 -> 195 536 -> 544 933 -> 942
+// (rows of very uneven lengths lose there: 33 x U[40, 1800], 32/8 31 -> 38; the
+// widths do not tell). Tables as wide as the rows need:
 //                                       1       5 %        20 %        60 %
 //   64 x U[500, 1500], 32/8          72 -> 68  219 -> 208  916 -> 894  2740 -> 2735
 //   20 x U[200, 900], 64/32          79 -> 71  161 -> 158  657 -> 647  2017 -> 2002
@@ -757,21 +769,13 @@ size_t decode_workspace_bytes(const SplitPlan& sp, int32_t n, int32_t H, int32_t
 //   16 x U[300, 2000], 32/8          25 -> 23   71 -> 70   257 -> 266   793 -> 783
 //   40 x U[500, 3000], 8/1           18 -> 15   45 -> 55   148 -> 164   453 -> 460
 //   8 x U[128, 1024], 32/8           15 -> 14   24 -> 23    70 -> 73    224 -> 212
-//   2 x U[500, 1500], 32/8           12 -> 12   16 -> 18    42 -> 43    115 -> 108
 //   33 x U[40, 1800], 32/8           34 -> 39   94 -> 94   366 -> 383  1111 -> 1129
-//   the same, full-width tables      31 -> 38   92 -> 94   364 -> 382  1117 -> 1130
-//   48 x U[200, 2000], 28/4          33 -> 37   99 -> 98   375 -> 388  1153 -> 1135
 //   8 x U[128, 1024], 32/32          31 -> 36   68 -> 67   254 -> 258   818 -> 795
-//   64 x U[100, 500], 32/32         174 -> 180 193 -> 196  981 -> 1003 3223 -> 3160
-// So: not past 4 (row, kv head) pairs per CU, nor at about one, where each CU
-// has a whole row and nothing needs cutting; else with a host table of at most
-// a 50th of the HBM table's width, or of half of it and more (rows mostly in
-// the host tier, or tables that hold the whole context for either tier, as a
-// step planned on the device has them: most often the newest blocks spilled;
-// below 32 pairs only if the host table is the wider), and between those from
-// 3/8 of a pair per CU on, down to a 12th. Widths given as -1: whether any
-// widths of bt_width together take it (workspace sizes). FD_HOST_WGS=<w>
-// forces the workers wherever they can be made.
+// So: where the wider table holds 32 tiles (64 past 4 (row, kv head) pairs per
+// CU), and the host table is at most a 50th as wide as HBM's, or half as wide
+// and more, or, from 3/8 of a pair per CU on, at most a 12th. Widths given as
+// -1: whether any widths of bt_width together take it (workspace sizes).
+// FD_HOST_WGS=<w> forces the workers wherever they can be made.
 bool plan_host_workers(SplitPlan& sp, int32_t n, int32_t H, int32_t KVH, int32_t D, int32_t BS,
                        int32_t bt_width, int32_t hbm_width, int32_t host_width,
                        int32_t kv_dtype) {
@@ -793,11 +797,10 @@ bool plan_host_workers(SplitPlan& sp, int32_t n, int32_t H, int32_t KVH, int32_t
   if (wgs <= 0 || wt > kMaxBalBlocks || pairs > kMaxBalPairs) return false;
   if (tune.host_wgs == nullptr) {
     const int64_t w0 = hbm_width, w1 = host_width;
-    const bool widths = w0 < 0 || w0 >= 50 * w1 || (2 * w1 >= w0 && (pairs >= 32 || w1 > w0)) ||
+    const int64_t tiles = w0 < 0 ? wt : std::max(w0, w1) * (BS / kTileTokens);
+    const bool widths = w0 < 0 || w0 >= 50 * w1 || 2 * w1 >= w0 ||
                         (8 * pairs >= 3LL * cus && w0 >= 12 * w1);
-    const bool row_per_cu = 4 * pairs >= 3LL * cus && 4 * pairs <= 5LL * cus;
-    if (row_per_cu) return false;
-    if (pairs > 4LL * cus || !widths) return false;
+    if (!widths || tiles < (pairs > 4LL * cus ? 64 : 32)) return false;
   }
   const double units = 2.0 * kTileTokens * D * 2 / kBalTileBytes;
   int64_t want = (5 * pairs <= 2LL * cus ? cus : 2LL * cus) - wgs;
