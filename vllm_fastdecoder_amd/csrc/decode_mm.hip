@@ -392,6 +392,11 @@ __device__ __forceinline__ void mm_task(const TiledParams& p, const Task& t, MmL
   const int w0 = SOLO ? wave : 0;
   auto& mg = lds.merge;
   const bool write_final = t.nsplit == 1;
+  if constexpr (SOLO) {
+    if (!write_final && lane == 0) start_count(p, t);
+  } else if constexpr (CG == 1) {
+    if (p.bal_parts > 0 && !write_final && threadIdx.x == 0) start_count(p, t);
+  }
 #pragma unroll
   for (int g = 0; g < CG; ++g) {
     const float lt = xor_sum<16>(l[g]);

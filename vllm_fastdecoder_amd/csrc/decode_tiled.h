@@ -853,28 +853,36 @@ __device__ __forceinline__ void finish_task(const TiledParams& p, const Task& t,
 }
 
 
-// Counts one part of a row as written; true for the row's last. One thread.
-// Rows are counted by their place in the launch's list: an order with entries
-// outside [0, n) may list a row twice, and each listing is cut, counted and
-// merged by itself.
+// Arrivals of a row's parts: one thread of a task calls start_count() before
+// the part's stores and, once they are waited for, count_arrival(), which is
+// true for the row's last. Rows are counted by their place in the launch's
+// list: an order with entries outside [0, n) may list a row twice, and each
+// listing is cut, counted and merged by itself.
 //
 // A counter holds the number of a launch above its arrivals (kArrivalBits).
-// Numbers rise from launch to launch, so the first atomic starts the count
-// anew whatever an earlier launch left (one that overlapped another on the
-// same counters leaves a count behind), and changes nothing otherwise; the
+// Numbers rise from launch to launch, so start_count()'s maximum starts the
+// count anew whatever an earlier launch left (one that overlapped another on
+// the same counters leaves a count behind), and changes nothing otherwise; the
 // last arrival takes its count back out, for replays of a graph, which keep
-// the number they were captured with. The two atomics go out together: one
-// thread's on one address stay in order. Counters of a launch with few of
-// them lie in lines of their own: the tasks finish together, and atomics on
-// one line go one by one. A row of 900 tokens, 32/8, eight counters of 32
-// parts each (HIP graph replay): 7.65 us with one atomic and the counters side
-// by side, 8.29 with both, 7.58 with both and the counters 256 bytes apart.
+// the number they were captured with. The tasks of a row finish together, and
+// atomics on one line go one by one, so the maximum goes out beside the
+// part's stores, and counters of a launch with few of them lie in lines of
+// their own. A row of 900 tokens, 32/8, eight counters of 32 parts each (HIP
+// graph replay): 7.65 us with one atomic and the counters side by side, 8.29
+// with both atomics at the end, 7.58 with the counters 256 bytes apart.
 constexpr int kArrivalBits = 24;  // parts of a row: below 2^22 (cut_balanced)
+
+__device__ __forceinline__ uint64_t* arrivals(const TiledParams& p, const Task& t) {
+  return p.counters + (t.pos * p.KVH * p.passes + t.kp) * p.counter_stride;
+}
+
+__device__ __forceinline__ void start_count(const TiledParams& p, const Task& t) {
+  __hip_atomic_fetch_max(arrivals(p, t), p.launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 
 __device__ __forceinline__ bool count_arrival(const TiledParams& p, const Task& t) {
   constexpr uint64_t kCount = (1ull << kArrivalBits) - 1;
-  uint64_t* c = p.counters + (t.pos * p.KVH * p.passes + t.kp) * p.counter_stride;
-  __hip_atomic_fetch_max(c, p.launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  uint64_t* c = arrivals(p, t);
   const uint64_t before =
       __hip_atomic_fetch_add(c, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   const bool done = (uint32_t)(before & kCount) == (uint32_t)t.nsplit - 1;
@@ -974,9 +982,11 @@ __device__ __forceinline__ void merge_parts(const TiledParams& p, const Task& t,
 template <typename T, int D, int G>
 __device__ __forceinline__ void end_task(const TiledParams& p, const Task& t, WaveStates<D, G>& ws,
                                          int wave, int lane) {
+  const bool part = p.bal_parts > 0 && t.nsplit > 1;
+  if (part && threadIdx.x == 0) start_count(p, t);
   __syncthreads();
   if (wave == 0) finish_task<T, D, G>(p, t, ws, lane);
-  if (p.bal_parts == 0 || t.nsplit == 1) return;
+  if (!part) return;
   if (last_to_arrive(p, t, &ws.last))
     merge_parts<T, D>(p, t, threadIdx.x, kWave * kWavesPerTask);
 }
