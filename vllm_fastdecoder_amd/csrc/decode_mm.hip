@@ -33,7 +33,10 @@
 //           Distance from 64 bits of an fp32 out, two parts, so, VALU: 33 x
 //           U[40, 1800], 32/8, bf16 20, 1.5 and 1.8e-7; 24 x U[256, 1024],
 //           32/32, bf16 24, 1.7 and 1.8e-7, fp16 2.8, 1.7 and 1.9e-7. It
-//           costs 0-3 % (64 x U[500, 1500], 32/8: 66.5 -> 68.5 us).
+//           costs 0-4 % (64 x U[500, 1500], 32/8: 66.5 -> 68.5 us), more in
+//           some launches of wide tasks, whose registers leave one wave per
+//           SIMD (40 x U[200, 2000], 71/1, D = 64: 24 -> 32; held to two waves
+//           such kernels spill: 32/1, D = 128 18.5 -> 30.4).
 //           The B operand needs 4 consecutive tokens of one dim per lane:
 //           each wave writes its V block row-major to LDS (lane l of load j
 //           carries 16-byte chunk 64 j + l of the block, so the loads stay

@@ -456,7 +456,7 @@ int32_t quarter_row_blocks(int32_t n, int32_t kv_tasks, int32_t D, bool f32, boo
 // the longest rows finished last, and split rows paid a combine launch
 // (4-5 us). Measured on MI355X against that plan (HIP graph replay, us, the
 // same inputs in turn; 6.8 TB/s floor in brackets):
-//   1 x 900 tokens, 32/8 heads, bf16 [0.5]                14.0 -> 7.2
+//   1 x 900 tokens, 32/8 heads, bf16 [0.5]                14.0 -> 7.0
 //   64 x U[1024, 4096], 8/1, bf16 [12.1]                  22.7 -> 19.0
 //   40 x U[50, 3100], 28/4, bf16 [21.4]                   33.8 -> 29.7
 //   24 x U[200, 4000], 16/8, D = 256, bf16 [56.0]         95.2 -> 66.8

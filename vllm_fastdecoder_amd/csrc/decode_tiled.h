@@ -852,7 +852,6 @@ __device__ __forceinline__ void finish_task(const TiledParams& p, const Task& t,
   }
 }
 
-
 // Arrivals of a row's parts: one thread of a task calls start_count() before
 // the part's stores and, once they are waited for, count_arrival(), which is
 // true for the row's last. Rows are counted by their place in the launch's
@@ -868,8 +867,10 @@ __device__ __forceinline__ void finish_task(const TiledParams& p, const Task& t,
 // atomics on one line go one by one, so the maximum goes out beside the
 // part's stores, and counters of a launch with few of them lie in lines of
 // their own. A row of 900 tokens, 32/8, eight counters of 32 parts each (HIP
-// graph replay): 7.65 us with one atomic and the counters side by side, 8.29
-// with both atomics at the end, 7.58 with the counters 256 bytes apart.
+// graph replay): both atomics at the end 8.29 us with the counters side by
+// side and 7.58 with them 256 bytes apart; the maximum beside the stores takes
+// another 0.2 off, and 14.7 -> 13.5 off 3 rows of 2,678 to 10,717 tokens, 8/1
+// (85 parts each).
 constexpr int kArrivalBits = 24;  // parts of a row: below 2^22 (cut_balanced)
 
 __device__ __forceinline__ uint64_t* arrivals(const TiledParams& p, const Task& t) {
