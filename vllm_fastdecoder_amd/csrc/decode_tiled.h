@@ -865,7 +865,7 @@ __device__ __forceinline__ void finish_task(const TiledParams& p, const Task& t,
 // last arrival takes its count back out, for replays of a graph, which keep
 // the number they were captured with. The tasks of a row finish together, and
 // atomics on one line go one by one, so the maximum goes out beside the
-// part's stores, and counters of a launch with few of them lie in lines of
+// part's stores (a host worker wave's before its blocks are read), and counters of a launch with few of them lie in lines of
 // their own. A row of 900 tokens, 32/8, eight counters of 32 parts each (HIP
 // graph replay): both atomics at the end 8.29 us with the counters side by
 // side and 7.58 with them 256 bytes apart; the maximum beside the stores takes
